@@ -54,10 +54,11 @@ struct Dev {
                            // that broke up this step; [256 + 32 x] and [512 + 32 x], x < 8: the
                            // counters that deal P2G's and G2P's blocks (reset by k_begin)
   unsigned long long* rwords;  // RED_WORDS: tagged chunk sums of the solve's reductions
-  unsigned long long* hz;      // 3 x capc: tagged halo words of each water cell (the register
-                               // forms and the memory form's streaming passes: z in the first
-                               // third, the streaming passes' directions alternating between the
-                               // other two; the pipelined form alternates between the first two)
+  unsigned long long* hz;      // 3 x capc: tagged halo words. By cell, for the memory form's
+                               // streaming passes (z in the first third, the directions
+                               // alternating between the other two) and the pipelined form
+                               // (alternating between the first two); by face, for the solve's
+                               // on-chip forms (z in the first half, p in the second)
   float* pcg;                  // 4 x capc: z, q and two m buffers of the pipelined solve's memory
                                // form (NATRAY_CG_PIPELINED only; else null)
   float* vmax_part;        // fastest particle of each g2p workgroup (<= cap workgroups)

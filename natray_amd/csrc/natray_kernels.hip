@@ -1039,8 +1039,14 @@ constexpr uint32_t SOLVE_ITER_CAP = 1u << 24;
 
 constexpr uint32_t SOLVE_THREADS = 1024;
 constexpr uint32_t SOLVE_WAVES = SOLVE_THREADS / 64;
-// Blocks a wave of the solve keeps in registers.
+// Blocks a wave of the pipelined solve keeps in registers.
 constexpr uint32_t SOLVE_RMAX = 2;
+// Sets of four blocks a wave of the solve keeps on the chip: one with every field in registers
+// (workgroups of at most 64 blocks), or QUAD_WIDE (at most 256 blocks).
+constexpr uint32_t QUAD_WIDE = 4;
+constexpr uint32_t SOLVE_BLOCKS = SOLVE_WAVES * 4u * QUAD_WIDE;
+// Dev::nbm's bits from here on: the cell's neighbours that are not solid (0..6).
+constexpr uint32_t NBM_COUNT = 8;
 // The memory form's streaming passes: at most this many blocks per wave, the loads of this
 // many blocks issued together.
 constexpr uint32_t SOLVE_JMAX = 32;
@@ -1051,6 +1057,7 @@ constexpr uint32_t SOLVE_GROUP = 2;
 constexpr uint32_t RED_SLOTS = 8;
 constexpr uint32_t RED_PAIRS = RED_SLOTS / 2;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // Cache policy of the chunk records' 16-byte loads and stores: sc1, the bits of the agent-scope
 // atomics the other tagged words use.
 constexpr int kRedPolicy = 16;
@@ -1160,10 +1167,13 @@ __device__ __forceinline__ bool converged(R rr, R tol, R b_norm) {
 // The blocks and chunks of one solve workgroup.
 struct SolveSpan {
   uint32_t n, K, m, G;
+  uint32_t W, logw;  // the chunk fold's width (chunk_width) and its logarithm
   uint32_t wg;      // this workgroup among the G of its scene
   uint32_t c0, c1;  // chunks of this workgroup
   uint32_t b0, b1;  // their blocks
-  bool in_regs;     // every workgroup's blocks fit in registers (the same for all)
+  bool in_regs;     // every workgroup's blocks fit on the chip (the same for all)
+  bool narrow;      // at most 64 blocks per workgroup (the same for all)
+  bool lead;        // the workgroup that writes the solve's results
   bool stream;      // the memory form's streaming passes (the same for all)
   bool coherent;    // a reduction also publishes the plain stores before it to the other
                     // workgroups (agent-scope release and acquire)
@@ -1180,8 +1190,43 @@ struct NoWait {
 // start) r.z, r.r, b.b and its water cells (a count, exact in either precision).
 template <class R>
 struct LPart {
-  R v[4][SOLVE_WAVES * SOLVE_RMAX];
+  R v[4][SOLVE_BLOCKS];
 };
+// The solve's LDS, shared by the forms a workgroup may take (one per launch). Quads: the
+// direction of the workgroup's cells, the diagonal's values and their reciprocals by the number
+// of neighbours that are not solid; with QUAD_WIDE sets per wave also each block's six face
+// neighbours and, for the faces towards other workgroups, the halo's directions (16 values a
+// face). A workgroup's blocks follow each other in slot order, z fastest, so a block's z
+// neighbours are the blocks next to it in the list: of the z faces only the first block's lower
+// and the last one's upper can lead to another workgroup. Streaming passes: each wave's blocks'
+// face neighbours and neighbour masks, and its first block.
+constexpr uint32_t QUAD_FACES = 4u * SOLVE_BLOCKS + 2u;
+struct QuadLds {
+  float4 d[SOLVE_BLOCKS][16];
+  float4 hd[QUAD_FACES][4];
+  float2 diag[8];
+  uint32_t nb[SOLVE_BLOCKS][6];
+  uint16_t slot[SOLVE_BLOCKS][6];
+  uint32_t faces;
+};
+struct StreamLds {
+  uint32_t nbl[SOLVE_WAVES][6][SOLVE_JMAX];
+  uint8_t mk[SOLVE_WAVES][SOLVE_JMAX][64];
+  uint32_t wave_b0[SOLVE_WAVES];
+};
+union SolveLds {
+  QuadLds q;
+  StreamLds s;
+};
+__device__ __forceinline__ SolveLds& solve_lds() {
+  __shared__ SolveLds lds;
+  return lds;
+}
+template <class R>
+__device__ __forceinline__ LPart<R>& part_lds() {
+  __shared__ LPart<R> lp;
+  return lp;
+}
 
 // The chunk fold's tree width: the next power of two >= K (at most MAX_CHUNKS).
 __host__ __device__ __forceinline__ uint32_t chunk_width(uint32_t K) {
@@ -1236,6 +1281,7 @@ __device__ __forceinline__ double first_lane(double x) {
 template <class R>
 struct RedLds {
   R red[4][256];
+  R total[2];
   uint32_t fail[2];
 };
 
@@ -1360,10 +1406,15 @@ __device__ bool reduce_wait(const Dev& d, const SolveSpan& sp, uint32_t tag, int
   return ok;
 }
 
+template <class R>
+__device__ __forceinline__ RedLds<R>& red_lds() {
+  __shared__ RedLds<R> lds;
+  return lds;
+}
 template <class R, class Wait = NoWait>
 __device__ bool reduce(const Dev& d, const SolveSpan& sp, uint32_t tag, int nc, const LPart<R>* lp, R* out,
                        Wait wait = Wait()) {
-  __shared__ RedLds<R> L;
+  RedLds<R>& L = red_lds<R>();
   reduce_publish<R>(d, sp, tag, nc, lp, L);
   return reduce_wait<R, Wait>(d, sp, tag, nc, out, L, wait);
 }
@@ -1421,6 +1472,7 @@ __device__ __forceinline__ Row cell_row(const Dev& d, uint32_t cell, int lx, int
       const float nt = tn[k];
       if (nt == SOLID) continue;
       w.diag += 1.0f;
+      w.mask += 1u << NBM_COUNT;
       if (nt == WATER) {
         off -= qn[k];
         w.mask |= 1u << k;
@@ -1437,30 +1489,33 @@ __device__ __forceinline__ Row cell_row(const Dev& d, uint32_t cell, int lx, int
   return w;
 }
 
-// solve_init (fluid.wgsl:450-491) for one cell from p0: the operator row, b, r = b - A p0 and
-// z. Writes diag, r, b, the neighbour mask and z; in register form also z as a tagged word
-// (tag `ztag`) into zw. Stores the block partials (r.z, r.r, b.b, water cells) through `prow`
-// from lane 0.
-template <class R>
-__device__ __forceinline__ void init_cell(const Dev& d, uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk,
-                                          unsigned long long* zw, uint32_t ztag, R* prow, const float* p0) {
-  const uint32_t capc = d.capc;
+// solve_init's rows (fluid.wgsl:450-489) for one cell from p0: diag, r = b - A p0, b and the
+// neighbour mask to memory.
+__device__ __forceinline__ Row row_cell(const Dev& d, uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk,
+                                        const float* p0) {
   const uint32_t cell = b * 64u + lane;
   const Row w = cell_row(d, cell, lx, ly, lz, lk, p0);
   if (w.water) {
-    d.cf[(size_t)NATRAY_F_DIAG * capc + cell] = w.diag;
-    d.cf[(size_t)NATRAY_F_R * capc + cell] = w.r;
+    d.cf[(size_t)NATRAY_F_DIAG * d.capc + cell] = w.diag;
+    d.cf[(size_t)NATRAY_F_R * d.capc + cell] = w.r;
     d.bvec[cell] = w.bv;
   }
   d.nbm[cell] = w.water ? w.mask : 0u;
-  const float r = w.water ? w.r : 0.0f, bv = w.water ? w.bv : 0.0f;
-  const float z = precondition(r, w.diag, w.water, lx, ly, lz, d.sc->precond);
-  if (w.water) {
-    d.cf[(size_t)NATRAY_F_Z * capc + cell] = z;
+  return w;
+}
+// The rest of solve_init (fluid.wgsl:490-491): z, also as a tagged word (tag `ztag`) into zw
+// where that is given, and the block partials (r.z, r.r, b.b, water cells) through `prow` from
+// lane 0.
+template <class R>
+__device__ __forceinline__ void start_cell(const Dev& d, uint32_t cell, uint32_t lane, int lx, int ly, int lz, bool water,
+                                           float diag, float r, float bv, unsigned long long* zw, uint32_t ztag, R* prow) {
+  const float z = precondition(r, diag, water, lx, ly, lz, d.sc->precond);
+  if (water) {
+    d.cf[(size_t)NATRAY_F_Z * d.capc + cell] = z;
     if (zw) store_word(&zw[cell], tag_word(ztag, __float_as_uint(z)));
   }
   const R v0 = wave_tree<R>(prod<R>(r, z)), v1 = wave_tree<R>(prod<R>(r, r)), v2 = wave_tree<R>(prod<R>(bv, bv));
-  const uint32_t nw = (uint32_t)__popcll(__ballot(w.water));
+  const uint32_t nw = (uint32_t)__popcll(__ballot(water));
   if (lane == 0) {
     prow[0] = v0;
     prow[1] = v1;
@@ -1468,11 +1523,31 @@ __device__ __forceinline__ void init_cell(const Dev& d, uint32_t b, uint32_t lan
     prow[3] = (R)nw;
   }
 }
+template <class R>
+__device__ __forceinline__ void init_cell(const Dev& d, uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk,
+                                          unsigned long long* zw, uint32_t ztag, R* prow, const float* p0) {
+  const Row w = row_cell(d, b, lane, lx, ly, lz, lk, p0);
+  start_cell<R>(d, b * 64u + lane, lane, lx, ly, lz, w.water, w.diag, w.water ? w.r : 0.0f, w.water ? w.bv : 0.0f, zw, ztag,
+                prow);
+}
 
 // The starting pressure of this solve: the warm start's guess when it was accepted this step
 // (Dev::bar[11]), else the particle-carried pressure.
 __device__ __forceinline__ const float* start_pressure(const Dev& d) {
   return d.bar[11] ? d.guess : d.cf + (size_t)NATRAY_F_P * d.capc;
+}
+
+// The rows of every cell, before the solve. On its own the pass has eight waves a SIMD to hide
+// its chain of loads (block links, types, pressures and velocities) behind; inside the solve it
+// had four, in lock step: 190 us of the 15.2M impact's solve, 25 us here.
+template <class L>
+__global__ __launch_bounds__(256) void k_solve_rows(L l) {
+  const View v = view(l);
+  const Dev& d = v.d;
+  if (d.st->dt_ns == 0u) return;
+  const float* const p0 = start_pressure(d);
+  for_blocks(d, v.wg * 4u, n_blocks(d), v.wgs * 4u,
+             [&](uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk) { row_cell(d, b, lane, lx, ly, lz, lk, p0); });
 }
 
 // The solver scalars of a solve, kept by every workgroup alike.
@@ -1515,11 +1590,11 @@ __device__ __forceinline__ bool solve_beta(const Dev& d, const R* tt, SolveScala
   return true;
 }
 
-// End of a solve: the scene's workgroup 0 writes State, the solver scalars, the counters and
+// End of a solve: one workgroup of the scene writes State, the solver scalars, the counters and
 // the last tag.
 template <class R>
 __device__ __forceinline__ void solve_finish(const Dev& d, const SolveSpan& sp, uint32_t tag, const SolveScalars<R>& s) {
-  if (sp.wg != 0 || threadIdx.x != 0) return;
+  if (!sp.lead || threadIdx.x != 0) return;
   const uint32_t n = sp.n;
   __hip_atomic_store(d.bar + 4, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   natray_state* st = d.st;
@@ -1589,9 +1664,12 @@ __device__ __noinline__ void solve_memory(const Dev* dp, SolveSpan sp, uint32_t 
   float* const cDiag = d.cf + (size_t)NATRAY_F_DIAG * capc;
   unsigned long long* const zw = d.hz;
   const float* const p0 = start_pressure(d);
-  for_blocks<SOLVE_WAVES>(d, b0, b1, SOLVE_WAVES, [&](uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk) {
+  for_blocks<SOLVE_WAVES>(d, b0, b1, SOLVE_WAVES, [&](uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t*) {
     R v[4];
-    init_cell<R>(d, b, lane, lx, ly, lz, lk, stream ? zw : nullptr, tag + 1u, v, p0);
+    const uint32_t cell = b * 64u + lane;
+    const bool water = (d.nbm[cell] & 64u) != 0u;
+    start_cell<R>(d, cell, lane, lx, ly, lz, water, water ? cDiag[cell] : 1.0f, water ? cR[cell] : 0.0f,
+                  water ? d.bvec[cell] : 0.0f, stream ? zw : nullptr, tag + 1u, v);
     if (lane == 0)
       for (uint32_t k = 0; k < 4u; ++k) d.part[b * 4u + k] = (double)v[k];
   });
@@ -1599,7 +1677,7 @@ __device__ __noinline__ void solve_memory(const Dev* dp, SolveSpan sp, uint32_t 
   SolveScalars<R> s;
   bool go = solve_start<R>(d, tt, reduce<R>(d, sp, ++tag, 4, nullptr, tt), s);
   if (p0 != cP) {
-    // The iterate starts at the guess; every workgroup has read the carried pressure by now.
+    // The iterate starts at the guess (every row was formed before this kernel).
     for (uint32_t c = b0 * 64u + threadIdx.x; c < b1 * 64u; c += blockDim.x)
       if (d.nbm[c] & 64u) cP[c] = p0[c];
     __syncthreads();
@@ -1614,11 +1692,11 @@ __device__ __noinline__ void solve_memory(const Dev* dp, SolveSpan sp, uint32_t 
   // that block the face touches (the coordinate on the axis 0 <-> 3).
   const uint32_t nb_dir[3] = {lx == 3 ? 1u : 0u, ly == 3 ? 3u : 2u, lz == 3 ? 5u : 4u};
   const uint32_t nb_cell[3] = {ln ^ 48u, ln ^ 12u, ln ^ 3u};
-  __shared__ uint32_t nbl[SOLVE_WAVES][6][SOLVE_JMAX];
-  __shared__ uint8_t mk[SOLVE_WAVES][SOLVE_JMAX][64];
+  auto& nbl = solve_lds().s.nbl;
+  auto& mk = solve_lds().s.mk;
   // Each pass reads its wave's first block from LDS, so that the blocks' addresses are formed
   // inside the iteration rather than held in registers across it.
-  __shared__ uint32_t wave_b0[SOLVE_WAVES];
+  auto& wave_b0 = solve_lds().s.wave_b0;
   if (stream) {
     for (uint32_t j = 0; j < SOLVE_JMAX; ++j) {
       const uint32_t b = b0 + wv + SOLVE_WAVES * j;
@@ -1940,12 +2018,14 @@ __device__ __noinline__ void solve_memory(const Dev* dp, SolveSpan sp, uint32_t 
 }
 
 // This workgroup's chunks and blocks in its scene's solve, and whether every workgroup keeps
-// its blocks in registers.
-__device__ __forceinline__ SolveSpan solve_span(const View& v, bool streams) {
+// its blocks on the chip (at most `regs` of them).
+__device__ __forceinline__ SolveSpan solve_span(const View& v, uint32_t regs, bool streams) {
   SolveSpan sp;
   sp.n = n_blocks(v.d);
   sp.K = sp.n ? (sp.n + MAX_CHUNKS - 1u) / MAX_CHUNKS : 1u;
   sp.m = sp.n ? (sp.n + sp.K - 1u) / sp.K : 0u;
+  sp.W = chunk_width(sp.K);
+  sp.logw = (uint32_t)__builtin_ctz(sp.W);
   sp.G = v.wgs;
   sp.wg = v.wg;
   sp.c0 = (uint32_t)((uint64_t)v.wg * sp.m / sp.G);
@@ -1954,10 +2034,895 @@ __device__ __forceinline__ SolveSpan solve_span(const View& v, bool streams) {
   sp.b1 = min(sp.n, sp.c1 * sp.K);
   // The most blocks a workgroup holds: its chunks are at most ceil(m / G).
   const uint32_t most = (sp.m + sp.G - 1u) / sp.G * sp.K;
-  sp.in_regs = most <= SOLVE_WAVES * SOLVE_RMAX;
+  sp.in_regs = most <= regs;
+  sp.narrow = most <= SOLVE_WAVES * 4u;
+  sp.lead = v.wg == 0u;
   sp.stream = streams && !sp.in_regs && most <= SOLVE_WAVES * SOLVE_JMAX;
   sp.coherent = !sp.in_regs && !sp.stream;
   return sp;
+}
+
+// ---- quads: four blocks per wave ----------------------------------------------------------------------
+//
+// The solve's on-chip forms give a wave sets of four consecutive blocks, and a lane a column of
+// four cells: lane 16 q + 4 x + y holds the cells (x, y, 0..3) of the set's block q. A field of a
+// set is then one 16-byte access per lane; x and y neighbours are DPP moves inside a row of 16
+// lanes, folded into the additions that use them; z neighbours lie in the same lane. With one
+// cell per lane, each neighbour cost two to four instructions for one block instead of one for
+// four, and each half sweep of the preconditioner left half of the lanes idle.
+//
+// A lane keeps its column in colour order (quad_swap): slots 0, 1 are its red cells ((x + y + z)
+// even) from the bottom up, slots 2, 3 its black ones. A cell's x and y neighbours are then the
+// other colour's slot of the same height in the next lane, and the half sweeps need no selects.
+struct QuadLane {
+  uint32_t ln, q, col;      // lane, block of the set, column 4 x + y
+  bool x0, x3, y0, y3, odd; // odd: the column's red cells are z = 1 and 3
+};
+__device__ __forceinline__ QuadLane quad_lane() {
+  const uint32_t ln = lane_id(), col = ln & 15u, x = col >> 2, y = col & 3u;
+  return {ln, ln >> 4, col, x == 0u, x == 3u, y == 0u, y == 3u, ((x + y) & 1u) != 0u};
+}
+// Between z order and colour order (its own inverse).
+template <class T>
+__device__ __forceinline__ void quad_swap(const T* v, T* o, bool odd) {
+  const T a0 = odd ? v[1] : v[0], b0 = odd ? v[0] : v[1], a1 = odd ? v[3] : v[2], b1 = odd ? v[2] : v[3];
+  o[0] = a0, o[1] = a1, o[2] = b0, o[3] = b1;
+}
+template <class T>
+__device__ __forceinline__ void quad_unswap(const T* v, T* o, bool odd) {
+  const T z0 = odd ? v[2] : v[0], z1 = odd ? v[0] : v[2], z2 = odd ? v[3] : v[1], z3 = odd ? v[1] : v[3];
+  o[0] = z0, o[1] = z1, o[2] = z2, o[3] = z3;
+}
+__device__ __forceinline__ void quad_load(const float* f, uint32_t cell0, bool odd, float* o) {
+  const float4 v = *reinterpret_cast<const float4*>(f + cell0);
+  const float z[4] = {v.x, v.y, v.z, v.w};
+  quad_swap(z, o, odd);
+}
+// Stores the column's water cells (bits 0..3 of m, in colour order).
+__device__ __forceinline__ void quad_store(float* f, uint32_t cell0, bool odd, const float* v, uint32_t m) {
+  float z[4];
+  quad_unswap(v, z, odd);
+  if ((m & 15u) == 15u) {
+    *reinterpret_cast<float4*>(f + cell0) = make_float4(z[0], z[1], z[2], z[3]);
+  } else if (m & 15u) {
+    const uint32_t c[4] = {m & 1u, m >> 1 & 1u, m >> 2 & 1u, m >> 3 & 1u};
+    uint32_t w[4];
+    quad_unswap(c, w, odd);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (w[k]) f[cell0 + k] = z[k];
+  }
+}
+
+// block_sum's tree (fluid.wgsl:414-422) of a set's four blocks at once, from the lanes' values in
+// colour order; lane 16 q ends with block q's sum. Steps by one in x or y change the colour, so
+// they add the other colour's slot of the next lane.
+template <class R>
+__device__ __forceinline__ R quad_tree(const R* v) {
+  R a[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a[k] = v[k] + row_down<8>(v[k]);
+  R b[4] = {a[0] + row_down<4>(a[2]), a[1] + row_down<4>(a[3]), a[2] + row_down<4>(a[0]), a[3] + row_down<4>(a[1])};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a[k] = b[k] + row_down<2>(b[k]);
+  R c[4] = {a[0] + row_down<1>(a[2]), a[1] + row_down<1>(a[3]), a[2] + row_down<1>(a[0]), a[3] + row_down<1>(a[1])};
+  return (c[0] + c[1]) + (c[2] + c[3]);
+}
+
+// What a lane's column sees across its block's faces: hx, hy in colour order, for the lanes at x
+// (y) = 3 the neighbour below's column and for those at 0 the one above's, the columns a rotation
+// of the row by one brings to the lanes that need them; zm, zp for every lane.
+struct QuadHalo {
+  float x[4], y[4], zm, zp;
+};
+
+// Correctly rounded s / d by a divisor known in advance, from y = RN(1 / d): one multiplication
+// and two fused multiply-adds (Brisebarre, Muller and Raina, "Accelerating correctly rounded
+// floating-point division when the divisor is known in advance", IEEE Trans. Computers 53,
+// 2004), against the eleven dependent instructions of a general IEEE division. The residual is
+// formed as q0 d - s, so that a zero keeps the sign s / d has. The result is RN(s / d) while
+// nothing under- or overflows: DivGuard tells when that may have happened, and the caller then
+// divides in full. (Compared with the division over all 2^23 significands of s for 24,000
+// divisors, the extreme ones among them.)
+__device__ __forceinline__ float div_by(float s, float d, float y) {
+  const float q0 = s * y;
+  const float e = __builtin_fmaf(q0, d, -s);
+  return __builtin_fmaf(-e, y, q0);
+}
+
+// What div_by needs: every nonzero dividend of at least 2^-70, a divisor within 2^+-30, and
+// results below 2^100 (an overflow or a NaN in any sweep reaches a later result). The exponents
+// are compared with the sign shifted out; a zero dividend, which is exact, wraps to the top.
+struct DivGuard {
+  uint32_t lo = 0xffffffffu, hi = 0u;
+  __device__ __forceinline__ void dividend(float s) { lo = min(lo, (__float_as_uint(s) << 1) - 1u); }
+  __device__ __forceinline__ void result(float z) { hi = max(hi, __float_as_uint(z) << 1); }
+  static __device__ __forceinline__ bool divisor(float d) { return d >= 0x1p-30f && d <= 0x1p30f; }
+  __device__ __forceinline__ bool bad() const { return lo < (57u << 24) - 1u || hi >= 227u << 24; }
+};
+
+// The preconditioner (see precondition) of a set of quads: z = M^-1 r, 0 off water. m: bits 0..3
+// the slots that are water, bits 4, 5 the red slots with a water neighbour inside the block.
+// A cell that is not water holds -0 during the sweeps, which an addition leaves out bit for bit,
+// as it does the -0 the rotations bring across the block's faces.
+template <bool FAST>
+__device__ __forceinline__ void precondition_quad_as(const float* r, const float* dg, const float* y, uint32_t m,
+                                                     const QuadLane& l, uint32_t mode, float* z, DivGuard& g) {
+  auto div = [&](float s, int k) -> float {
+    if (!FAST) return s / dg[k];
+    g.dividend(s);
+    return div_by(s, dg[k], y[k]);
+  };
+  const bool w[4] = {(m & 1u) != 0u, (m & 2u) != 0u, (m & 4u) != 0u, (m & 8u) != 0u};
+  if (mode == NATRAY_PRECOND_JACOBI) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      z[k] = w[k] ? div(r[k], k) : 0.0f;
+      g.result(z[k]);
+    }
+    return;
+  }
+  // The first half sweep starts from z = +0: each water neighbour adds +0, which changes only
+  // r = -0.
+  float v[4];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) v[k] = w[k] ? div(r[k] + ((m >> (4 + k) & 1u) ? 0.0f : -0.0f), k) : -0.0f;
+#pragma unroll
+  for (int sweep = 1; sweep < 5; ++sweep) {
+    const int c = (sweep & 1) ? 2 : 0;         // the colour's slots c, c + 1
+    const float n0 = v[2 - c], n1 = v[3 - c];  // the other colour's values
+    const bool up = (sweep & 1) ? !l.odd : l.odd;  // the colour's cells are z = 1 and 3
+    const float mid = up ? n1 : n0;            // the neighbour between the two
+    float s0 = r[c] + row_rot<4>(l.x3 ? -0.0f : n0);
+    float s1 = r[c + 1] + row_rot<4>(l.x3 ? -0.0f : n1);
+    s0 += row_rot<12>(l.x0 ? -0.0f : n0);
+    s1 += row_rot<12>(l.x0 ? -0.0f : n1);
+    s0 += quad_rot<1>(l.y3 ? -0.0f : n0);
+    s1 += quad_rot<1>(l.y3 ? -0.0f : n1);
+    s0 += quad_rot<3>(l.y0 ? -0.0f : n0);
+    s1 += quad_rot<3>(l.y0 ? -0.0f : n1);
+    s0 += up ? n0 : -0.0f;
+    s1 += mid;
+    s0 += mid;
+    s1 += up ? -0.0f : n1;
+    const float q0 = div(s0, c), q1 = div(s1, c + 1);
+    v[c] = w[c] ? q0 : -0.0f;
+    v[c + 1] = w[c + 1] ? q1 : -0.0f;
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    z[k] = w[k] ? v[k] : 0.0f;
+    g.result(z[k]);
+  }
+}
+__device__ __forceinline__ void precondition_quad(const float* r, const float* dg, const float* y, bool fast, uint32_t m,
+                                                  const QuadLane& l, uint32_t mode, float* z) {
+  if (fast) {
+    DivGuard g;
+    precondition_quad_as<true>(r, dg, y, m, l, mode, z, g);
+    if (__builtin_expect(__ballot(g.bad()) == 0ull, 1)) return;
+  }
+  DivGuard g;
+  precondition_quad_as<false>(r, dg, y, m, l, mode, z, g);
+}
+
+// (A v) of a column: diag v minus the neighbours in the order -x, +x, -y, +y, -z, +z. v and the
+// halo are 0 where a cell is not water, which the subtraction leaves out bit for bit. T: the
+// precision it is computed in.
+template <class T>
+__device__ __forceinline__ void quad_row(const float* v, const float* dg, const QuadHalo& h, const QuadLane& l, T* o) {
+  T q[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int n = k ^ 2;  // the other colour's slot of the same height
+    q[k] = (T)dg[k] * (T)v[k];
+    q[k] -= (T)row_rot<4>(l.x3 ? h.x[n] : v[n]);
+    q[k] -= (T)row_rot<12>(l.x0 ? h.x[n] : v[n]);
+    q[k] -= (T)quad_rot<1>(l.y3 ? h.y[n] : v[n]);
+    q[k] -= (T)quad_rot<3>(l.y0 ? h.y[n] : v[n]);
+  }
+#pragma unroll
+  for (int c = 0; c < 4; c += 2) {
+    const float n0 = v[2 - c], n1 = v[3 - c];
+    const bool up = c == 0 ? l.odd : !l.odd;
+    const float mid = up ? n1 : n0;
+    q[c] -= (T)(up ? n0 : h.zm);
+    q[c] -= (T)mid;
+    q[c + 1] -= (T)mid;
+    q[c + 1] -= (T)(up ? h.zp : n1);
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = q[k];
+}
+
+// Faces between workgroups. Words that cross them lie face by face: block b's face f (0, 1: -x,
+// +x; 2, 3: -y, +y; 4, 5: -z, +z) at 16 (6 b + f), its cells in the order of their other two
+// coordinates, so that a face is one 128-byte line. Faces inside a workgroup go through LDS. (With
+// every neighbour's z read from words by cell, whose z faces are spread over all of a block's
+// lines, the 15.2M impact took 31.9 us per iteration, 9.8 without the halo.)
+constexpr uint32_t FACE_BYTES = 128, FACES_BYTES = 6u * FACE_BYTES;
+// One buffer of face words: z in the first half of Dev::hz, p before a residual refresh in the
+// second.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t face_rsrc(const Dev& d, uint32_t half, uint32_t n) {
+  return __builtin_amdgcn_make_buffer_rsrc(d.hz + (size_t)half * (d.capc / 64u) * 96u, 0, (int)(n * FACES_BYTES), 0x00020000);
+}
+// A lane's four halo links: across its x and y faces (lanes at 3 the neighbour below, at 0 the
+// one above, as QuadHalo has them), below and above. Each is a block's place in this workgroup,
+// or QUAD_FAR | a block of another workgroup, or NONE.
+constexpr uint32_t QUAD_FAR = 0x80000000u;
+struct QuadLinks {
+  uint32_t x, y, m, p;
+};
+__device__ __forceinline__ bool quad_far(uint32_t k) { return k != NONE && (k & QUAD_FAR); }
+// A set's face flags, per lane: bits 0..3 and 4..7 the water cells (z order) of the x and y halo
+// columns, 8 and 9 the cells below and above; 10..13 whether x, y, below and above lie in another
+// workgroup; 14..17 whether this lane's own faces (its x face, y face, bottom, top) do, and
+// 18..21 whether they face a block at all.
+__device__ __forceinline__ uint32_t quad_flags(const Dev& d, const uint32_t* nb, const QuadLinks& k, const QuadLane& l,
+                                               uint32_t b0, uint32_t b1) {
+  uint32_t w = 0;
+  auto cells = [](uint4 v) -> uint32_t { return (v.x >> 6 & 1u) | (v.y >> 5 & 2u) | (v.z >> 4 & 4u) | (v.w >> 3 & 8u); };
+  auto id = [&](uint32_t link) -> uint32_t { return (link & QUAD_FAR) ? link & ~QUAD_FAR : b0 + link; };
+  if (k.x != NONE) w |= cells(*reinterpret_cast<const uint4*>(d.nbm + (size_t)id(k.x) * 64u + l.col * 4u));
+  if (k.y != NONE) w |= cells(*reinterpret_cast<const uint4*>(d.nbm + (size_t)id(k.y) * 64u + l.col * 4u)) << 4;
+  if (k.m != NONE) w |= (d.nbm[(size_t)id(k.m) * 64u + l.col * 4u + 3u] >> 6 & 1u) << 8;
+  if (k.p != NONE) w |= (d.nbm[(size_t)id(k.p) * 64u + l.col * 4u] >> 6 & 1u) << 9;
+  w |= (quad_far(k.x) ? 1u << 10 : 0u) | (quad_far(k.y) ? 1u << 11 : 0u) | (quad_far(k.m) ? 1u << 12 : 0u) |
+       (quad_far(k.p) ? 1u << 13 : 0u);
+  const uint32_t own[4] = {l.x0 ? nb[0] : (l.x3 ? nb[1] : NONE), l.y0 ? nb[2] : (l.y3 ? nb[3] : NONE), nb[4], nb[5]};
+#pragma unroll
+  for (uint32_t f = 0; f < 4u; ++f) {
+    if (own[f] != NONE) w |= 1u << (18u + f);
+    if (quad_far(own[f])) w |= 1u << (14u + f);
+  }
+  return w;
+}
+// The halo words to wait for: all, or (far) those of other workgroups.
+__device__ __forceinline__ uint32_t quad_want(uint32_t w, bool far) {
+  if (!far) return w & 0x3ffu;
+  return w & (((w >> 10 & 1u) ? 15u : 0u) | ((w >> 11 & 1u) ? 240u : 0u) | ((w >> 12 & 3u) << 8));
+}
+
+// Tagged halo words of a column as loaded, two per 16-byte record.
+struct QuadWords {
+  u32x4 x0, x1, y0, y1;
+  u32x2 m, p;
+};
+// Loads the words still missing (have: bit 0 x, bit 1 y, bit 2 z) and marks those that carry
+// `tag`; true once every word wanted is there. A word counts by its own tag. k: the links as
+// block numbers.
+__device__ __forceinline__ bool quad_words(__amdgpu_buffer_rsrc_t rs, const QuadLinks& k, uint32_t want, const QuadLane& l,
+                                           uint32_t tag, QuadWords& q, uint32_t& have) {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  if (!(have & 1u)) {
+    const uint32_t at = k.x * FACES_BYTES + (l.x3 ? FACE_BYTES : 0u) + (l.col & 3u) * 32u;
+    q.x0 = __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, kRedPolicy);
+    q.x1 = __builtin_amdgcn_raw_buffer_load_b128(rs, at + 16u, 0, kRedPolicy);
+  }
+  if (!(have & 2u)) {
+    const uint32_t at = k.y * FACES_BYTES + (l.y3 ? 3u : 2u) * FACE_BYTES + (l.col >> 2) * 32u;
+    q.y0 = __builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, kRedPolicy);
+    q.y1 = __builtin_amdgcn_raw_buffer_load_b128(rs, at + 16u, 0, kRedPolicy);
+  }
+  if (!(have & 4u)) {
+    if (want & 256u) q.m = __builtin_amdgcn_raw_buffer_load_b64(rs, k.m * FACES_BYTES + 5u * FACE_BYTES + l.col * 8u, 0, kRedPolicy);
+    if (want & 512u) q.p = __builtin_amdgcn_raw_buffer_load_b64(rs, k.p * FACES_BYTES + 4u * FACE_BYTES + l.col * 8u, 0, kRedPolicy);
+  }
+  auto lacks = [&](uint32_t bit, uint32_t t) -> bool { return (want >> bit & 1u) && t != tag; };
+  const bool fx = !(lacks(0, q.x0.y) || lacks(1, q.x0.w) || lacks(2, q.x1.y) || lacks(3, q.x1.w));
+  const bool fy = !(lacks(4, q.y0.y) || lacks(5, q.y0.w) || lacks(6, q.y1.y) || lacks(7, q.y1.w));
+  const bool fz = !(lacks(8, q.m.y) || lacks(9, q.p.y));
+  have |= (fx ? 1u : 0u) | (fy ? 2u : 0u) | (fz ? 4u : 0u);
+  return have == 7u;
+}
+__device__ __forceinline__ uint32_t quad_had(uint32_t want) {
+  return ((want & 15u) ? 0u : 1u) | ((want & 240u) ? 0u : 2u) | ((want & 768u) ? 0u : 4u);
+}
+// Waits until every halo word wanted carries `tag`; false once the solve aborts.
+__device__ __forceinline__ bool quad_wait(const Dev& d, __amdgpu_buffer_rsrc_t rs, const QuadLinks& k, uint32_t want,
+                                          const QuadLane& l, uint32_t tag, QuadWords& q, uint32_t have) {
+  uint32_t spins = 0;
+  while (!quad_words(rs, k, want, l, tag, q, have)) {
+    __builtin_amdgcn_s_sleep(1);
+    if ((++spins & 255u) == 0u &&
+        (__hip_atomic_load(d.bar + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u || spins > kSpinLimit)) {
+      __hip_atomic_store(d.bar + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return false;
+    }
+  }
+  return true;
+}
+// The wanted words' payloads, 0 elsewhere.
+__device__ __forceinline__ void quad_payload(const QuadWords& q, uint32_t want, bool odd, QuadHalo& h) {
+  auto val = [&](uint32_t bit, uint32_t v) -> float { return (want >> bit & 1u) ? __uint_as_float(v) : 0.0f; };
+  const float x[4] = {val(0, q.x0.x), val(1, q.x0.z), val(2, q.x1.x), val(3, q.x1.z)};
+  const float y[4] = {val(4, q.y0.x), val(5, q.y0.z), val(6, q.y1.x), val(7, q.y1.z)};
+  quad_swap(x, h.x, odd);
+  quad_swap(y, h.y, odd);
+  h.zm = val(8, q.m.x);
+  h.zp = val(9, q.p.x);
+}
+// Publishes the faces of block b marked in `faces` (this lane's x, y, bottom and top face) with
+// tag `tag`. The words of cells that are not water are never read.
+__device__ __forceinline__ void quad_publish(__amdgpu_buffer_rsrc_t rs, uint32_t b, const float* v, uint32_t faces,
+                                             const QuadLane& l, uint32_t tag) {
+  if (!faces) return;
+  float z[4];
+  quad_unswap(v, z, l.odd);
+  const u32x4 lo = {__float_as_uint(z[0]), tag, __float_as_uint(z[1]), tag};
+  const u32x4 hi = {__float_as_uint(z[2]), tag, __float_as_uint(z[3]), tag};
+  const uint32_t base = b * FACES_BYTES;
+  if (faces & 1u) {
+    const uint32_t at = base + (l.x3 ? FACE_BYTES : 0u) + (l.col & 3u) * 32u;
+    __builtin_amdgcn_raw_buffer_store_b128(lo, rs, at, 0, kRedPolicy);
+    __builtin_amdgcn_raw_buffer_store_b128(hi, rs, at + 16u, 0, kRedPolicy);
+  }
+  if (faces & 2u) {
+    const uint32_t at = base + (l.y3 ? 3u : 2u) * FACE_BYTES + (l.col >> 2) * 32u;
+    __builtin_amdgcn_raw_buffer_store_b128(lo, rs, at, 0, kRedPolicy);
+    __builtin_amdgcn_raw_buffer_store_b128(hi, rs, at + 16u, 0, kRedPolicy);
+  }
+  if (faces & 4u) {
+    const u32x2 w = {__float_as_uint(z[0]), tag};
+    __builtin_amdgcn_raw_buffer_store_b64(w, rs, base + 4u * FACE_BYTES + l.col * 8u, 0, kRedPolicy);
+  }
+  if (faces & 8u) {
+    const u32x2 w = {__float_as_uint(z[3]), tag};
+    __builtin_amdgcn_raw_buffer_store_b64(w, rs, base + 5u * FACE_BYTES + l.col * 8u, 0, kRedPolicy);
+  }
+}
+
+// The cells of a set this lane holds: bits 0..3 of m water, 4..5 as precondition_quad takes them,
+// 8 + 3 k the number of neighbours of slot k that are not solid.
+__device__ __forceinline__ uint32_t quad_mask(const Dev& d, uint32_t cell0, bool valid, const QuadLane& l) {
+  if (!valid) return 0u;
+  const uint4 v = *reinterpret_cast<const uint4*>(d.nbm + cell0);
+  const uint32_t z[4] = {v.x, v.y, v.z, v.w};
+  uint32_t c[4];
+  quad_swap(z, c, l.odd);
+  const uint32_t side = (l.x0 ? 0u : 1u) | (l.x3 ? 0u : 2u) | (l.y0 ? 0u : 4u) | (l.y3 ? 0u : 8u);
+  uint32_t m = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    m |= (c[k] >> 6 & 1u) << k;
+    m |= (c[k] >> NBM_COUNT & 7u) << (8u + 3u * k);
+  }
+  // In the block: -z unless z = 0, +z unless z = 3; red slot 0 is z = odd, slot 1 z = odd + 2.
+  const uint32_t in0 = side | (l.odd ? 48u : 32u), in1 = side | (l.odd ? 16u : 48u);
+  m |= (c[0] & in0) ? 16u : 0u;
+  m |= (c[1] & in1) ? 32u : 0u;
+  return m;
+}
+
+// The waves of a workgroup on quads once the iteration runs: those that hold sets, and one that
+// makes the reductions, which holds none unless every wave does. Any others have ended.
+struct QuadWaves {
+  uint32_t wv;      // this wave
+  uint32_t reducer;
+  bool sets;        // this wave holds sets
+};
+
+// Reduction `tag` over NC components of the block partials in lp, with reduce's words and order.
+// A reduction's time is the length of this chain as much as the round trip inside it (at 22
+// blocks a workgroup an iteration was 18,000 cycles, 7,000 of them round trips), so one wave does
+// it alone: it folds the chunks, as many at once as its lanes hold, publishes them, waits for
+// everyone's, four to a lane, and forms the totals. The other waves meanwhile run `after`, which
+// nothing in this reduction needs, then `wait` until it returns true.
+template <class R, int NC, class After, class Wait>
+__device__ __forceinline__ bool quad_reduce(const Dev& d, const SolveSpan& sp, uint32_t tag, const QuadWaves& q,
+                                            const LPart<R>& lp, R* out, After after, Wait wait) {
+  constexpr int H = Halves<R>::N, P = (NC * H + 1) / 2;
+  static_assert(NC == 1 || NC == 2, "the totals' slots");
+  RedLds<R>& L = red_lds<R>();
+  const uint32_t ln = threadIdx.x & 63u, buf = tag & 1u;
+  const bool reducer = q.wv == q.reducer;
+  if (reducer && ln == 0u) L.fail[buf] = 0u;
+  wg_sync(false);
+  const __amdgpu_buffer_rsrc_t rs = red_rsrc(d);
+  if (reducer) {
+    const uint32_t W = sp.W, chunks = sp.c1 - sp.c0;
+    auto publish = [&](uint32_t c, const R* a) {
+#pragma unroll
+      for (int j = 0; j < P; ++j) {
+        const int k0 = 2 * j / H, k1 = (2 * j + 1) / H;
+        const u32x4 rec = {Halves<R>::part(a[k0], 2 * j % H), tag, k1 < NC ? Halves<R>::part(a[k1], (2 * j + 1) % H) : 0u, tag};
+        __builtin_amdgcn_raw_buffer_store_b128(rec, rs, red_pair(c, buf, (uint32_t)j), 0, kRedPolicy);
+      }
+    };
+    R a[NC];
+    if (W <= 64u) {
+      // 64 / W chunks at once, W lanes each.
+      const uint32_t slot = ln & (W - 1u), group = ln >> sp.logw;
+      for (uint32_t g0 = 0; g0 < chunks; g0 += 64u >> sp.logw) {
+        const uint32_t i = (g0 + group) * sp.K + slot;  // the block among the workgroup's
+        const bool in = slot < sp.K && g0 + group < chunks && sp.b0 + i < sp.b1;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+          R x = lp.v[k][in ? i : 0u];
+          x = in ? x : (R)0;
+          if (W >= 64u) x += lane_xor32(x);
+          if (W >= 32u) x += lane_xor16(x);
+          if (W >= 16u) x += row_down<8>(x);
+          if (W >= 8u) x += row_down<4>(x);
+          if (W >= 4u) x += row_down<2>(x);
+          if (W >= 2u) x += row_down<1>(x);
+          a[k] = x;
+        }
+        if (slot == 0u && g0 + group < chunks) publish(sp.c0 + g0 + group, a);
+      }
+    } else {
+      for (uint32_t c = sp.c0; c < sp.c1; ++c) {
+        const uint32_t lo = c * sp.K, hi = min(sp.n, lo + sp.K);
+#pragma unroll
+        for (int k = 0; k < NC; ++k) a[k] = chunk_tree<R>(d, sp, &lp, lo, hi, W, k, ln);
+        if (ln == 0u) publish(c, a);
+      }
+    }
+  }
+  if (q.sets) after();
+  bool lost = false;
+  uint32_t spins = 0;
+  // After a poll in vain: true once the solve has aborted, or this wait has lasted too long.
+  auto stuck = [&]() -> bool {
+    __builtin_amdgcn_s_sleep(1);
+    if ((++spins & 255u) != 0u ||
+        (__hip_atomic_load(d.bar + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u && spins <= kSpinLimit))
+      return false;
+    __hip_atomic_store(d.bar + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return lost = true;
+  };
+  if (reducer) {
+    uint32_t have = 0, pay[4][2 * P];
+#pragma unroll
+    for (uint32_t c = 0; c < 4u; ++c) {
+      if (ln + 64u * c >= sp.m) have |= 1u << c;
+#pragma unroll
+      for (int w = 0; w < 2 * P; ++w) pay[c][w] = 0u;
+    }
+    while (true) {
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      u32x4 rec[4][P];
+#pragma unroll
+      for (uint32_t c = 0; c < 4u; ++c)
+        if (!(have >> c & 1u)) {
+#pragma unroll
+          for (int j = 0; j < P; ++j)
+            rec[c][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, red_pair(ln + 64u * c, buf, (uint32_t)j), 0, kRedPolicy);
+        }
+#pragma unroll
+      for (uint32_t c = 0; c < 4u; ++c) {
+        if (have >> c & 1u) continue;
+        bool all = true;
+#pragma unroll
+        for (int j = 0; j < P; ++j) all = all && rec[c][j].y == tag && rec[c][j].w == tag;
+        if (!all) continue;
+        have |= 1u << c;
+#pragma unroll
+        for (int j = 0; j < P; ++j) pay[c][2 * j] = rec[c][j].x, pay[c][2 * j + 1] = rec[c][j].z;
+      }
+      if (have == 15u || stuck()) break;
+    }
+    // total()'s tree: (c_l + c_l+128) + (c_l+64 + c_l+192), then the 64 lanes.
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      R v[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[c] = (R)0 + Halves<R>::join(pay[c][k * H], pay[c][k * H + H - 1]);
+      const R x = lane_sum0((v[0] + v[2]) + (v[1] + v[3]));
+      if (ln == 0u) L.total[k] = x;
+    }
+  }
+  if (q.sets)
+    while (!wait())
+      if (stuck()) break;
+  if (lost) L.fail[buf] = 1u;
+  wg_sync(false);
+#pragma unroll
+  for (int k = 0; k < NC; ++k) out[k] = first_lane(L.total[k]);
+  return L.fail[buf] == 0u;
+}
+
+// x, for the compiler a new value: the bit tests on a set's masks are made again in each pass
+// (one or two instructions) rather than kept as lane masks across the iterations, which took
+// more scalar registers than there are.
+__device__ __forceinline__ uint32_t fresh(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// The solve on quads. RM sets per wave: one (workgroups of at most 64 blocks), or QUAD_WIDE (at
+// most 256). p, r and z stay in registers for the whole solve (z's place holds q between q's
+// making and its use), the direction in LDS. The faces between workgroups keep the direction
+// across them too, rebuilt each iteration as its owner does, z + beta d_old, from z's words: in
+// registers with one set, else in LDS.
+template <class R, uint32_t RM>
+__device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, uint32_t tag) {
+  constexpr bool WIDE = RM > 1u;
+  QuadLds& lds = solve_lds().q;
+  LPart<R>& lp = part_lds<R>();
+  const uint32_t mode = d.sc->precond, b0 = sp.b0, b1 = sp.b1, capc = d.capc;
+  const uint32_t wv = threadIdx.x >> 6;
+  QuadLane l = quad_lane();
+  float* const cP = d.cf + (size_t)NATRAY_F_P * capc;
+  float* const cR = d.cf + (size_t)NATRAY_F_R * capc;
+  float* const cZ = d.cf + (size_t)NATRAY_F_Z * capc;
+  float* const cQ = d.cf + (size_t)NATRAY_F_Q * capc;
+  float* const cD = d.cf + (size_t)NATRAY_F_D * capc;
+  const float* const p0 = start_pressure(d);
+  const __amdgpu_buffer_rsrc_t wz = face_rsrc(d, 0u, sp.n), wp = face_rsrc(d, 1u, sp.n);
+  // The diagonal is kc plus one per neighbour that is not solid, added one at a time.
+  float kc;
+  {
+    const float h = d.U->origin[3], cs = d.U->gravity[3] * dt_of(d);
+    kc = h * h / (cs * cs);
+  }
+  const bool fast = DivGuard::divisor(kc) && DivGuard::divisor(kc + 6.0f);
+  if (threadIdx.x < 8u) {
+    float dg = kc;
+    for (uint32_t k = 0; k < threadIdx.x; ++k) dg += 1.0f;
+    lds.diag[threadIdx.x] = make_float2(dg, 1.0f / dg);
+  }
+  if (threadIdx.x == 0u) lds.faces = 0u;
+  __syncthreads();
+
+  float rP[RM][4], rR[RM][4], rZ[RM][4], rG[4], rY[4];
+  uint32_t rM[RM], hw[RM];
+  QuadHalo hD{};                            // one set: the far halo's directions
+  QuadLinks lk = {NONE, NONE, NONE, NONE};  // one set: the links
+  auto first_block = [&](uint32_t r) -> uint32_t { return b0 + 4u * (wv + SOLVE_WAVES * r); };
+  // The block of this lane in set r, among the workgroup's.
+  uint32_t at = 4u * wv + l.q;
+  auto place = [&](uint32_t r) -> uint32_t { return at + 4u * SOLVE_WAVES * r; };
+  // The addresses a pass forms from these are formed in the pass, not held across the iterations.
+  auto new_pass = [&]() {
+    at = fresh(at);
+    l.col = fresh(l.col);
+  };
+  auto diag_of = [&](uint32_t m, float* g, float* y) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (WIDE) {
+        const float2 t = lds.diag[m >> (8 + 3 * k) & 7u];
+        g[k] = t.x, y[k] = t.y;
+      } else {
+        g[k] = rG[k], y[k] = rY[k];
+      }
+    }
+  };
+  auto links_of = [&](uint32_t r) -> QuadLinks {
+    if (!WIDE) return lk;
+    const uint32_t* nb = lds.nb[place(r)];
+    return {(l.x0 || l.x3) ? nb[l.x3 ? 0 : 1] : NONE, (l.y0 || l.y3) ? nb[l.y3 ? 2 : 3] : NONE, nb[4], nb[5]};
+  };
+  // The links as block numbers.
+  auto ids_of = [&](const QuadLinks& k) -> QuadLinks {
+    auto id = [&](uint32_t link) -> uint32_t { return (link & QUAD_FAR) ? link & ~QUAD_FAR : b0 + link; };
+    return {id(k.x), id(k.y), id(k.m), id(k.p)};
+  };
+  // WIDE: the far halo's directions of set r, face by face.
+  auto face_at = [&](uint32_t pl, uint32_t f) -> float* { return reinterpret_cast<float*>(lds.hd[lds.slot[pl][f]]); };
+  auto far_d = [&](uint32_t r, uint32_t w, const QuadHalo& z, float fb, QuadHalo& h) {
+    // h = z + fb h_old at the far faces, kept for the next iteration.
+    auto go4 = [&](float* at, const float* zv, float* hv) {
+      float4 o = *reinterpret_cast<float4*>(at);
+      o = make_float4(zv[0] + fb * o.x, zv[1] + fb * o.y, zv[2] + fb * o.z, zv[3] + fb * o.w);
+      *reinterpret_cast<float4*>(at) = o;
+      hv[0] = o.x, hv[1] = o.y, hv[2] = o.z, hv[3] = o.w;
+    };
+    if (!WIDE) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        hD.x[k] = z.x[k] + fb * hD.x[k];
+        hD.y[k] = z.y[k] + fb * hD.y[k];
+      }
+      hD.zm = z.zm + fb * hD.zm;
+      hD.zp = z.zp + fb * hD.zp;
+      h = hD;
+      return;
+    }
+    const uint32_t pl = place(r);
+    h = QuadHalo{};
+    if (w >> 10 & 1u) go4(face_at(pl, l.x3 ? 0u : 1u) + 4u * (l.col & 3u), z.x, h.x);
+    if (w >> 11 & 1u) go4(face_at(pl, l.y3 ? 2u : 3u) + 4u * (l.col >> 2), z.y, h.y);
+    if (w >> 12 & 1u) {
+      float* at = face_at(pl, 4u) + l.col;
+      *at = h.zm = z.zm + fb * *at;
+    }
+    if (w >> 13 & 1u) {
+      float* at = face_at(pl, 5u) + l.col;
+      *at = h.zp = z.zp + fb * *at;
+    }
+  };
+  // Where no z is added: the directions as far_d last left them.
+  auto far_d_kept = [&](uint32_t r, uint32_t w, QuadHalo& h) {
+    if (!WIDE) {
+      h = hD;
+      return;
+    }
+    const uint32_t pl = place(r);
+    h = QuadHalo{};
+    auto get4 = [&](const float* at, float* hv) {
+      const float4 o = *reinterpret_cast<const float4*>(at);
+      hv[0] = o.x, hv[1] = o.y, hv[2] = o.z, hv[3] = o.w;
+    };
+    if (w >> 10 & 1u) get4(face_at(pl, l.x3 ? 0u : 1u) + 4u * (l.col & 3u), h.x);
+    if (w >> 11 & 1u) get4(face_at(pl, l.y3 ? 2u : 3u) + 4u * (l.col >> 2), h.y);
+    if (w >> 12 & 1u) h.zm = face_at(pl, 4u)[l.col];
+    if (w >> 13 & 1u) h.zp = face_at(pl, 5u)[l.col];
+  };
+  // The halo's directions inside the workgroup, from LDS (behind a barrier): a neighbour's
+  // column has this lane's colours, and its top and bottom cells their slots.
+  auto near_d = [&](const QuadLinks& k, uint32_t w, QuadHalo& h) {
+    auto get4 = [&](uint32_t pl, float* hv) {
+      const float4 o = lds.d[pl][l.col];
+      hv[0] = o.x, hv[1] = o.y, hv[2] = o.z, hv[3] = o.w;
+    };
+    if ((w & 15u) && !(w >> 10 & 1u)) get4(k.x, h.x);
+    if ((w & 240u) && !(w >> 11 & 1u)) get4(k.y, h.y);
+    if ((w & 256u) && !(w >> 12 & 1u)) h.zm = reinterpret_cast<const float*>(&lds.d[k.m][l.col])[l.odd ? 1 : 3];
+    if ((w & 512u) && !(w >> 13 & 1u)) h.zp = reinterpret_cast<const float*>(&lds.d[k.p][l.col])[l.odd ? 2 : 0];
+  };
+  auto part = [&](int k, uint32_t r, R v) {
+    if (l.col == 0u && b0 + place(r) < b1) lp.v[k][place(r)] = v;
+  };
+
+  // The rows are in memory (k_solve_rows): the start's z, its words and the block partials.
+#pragma unroll
+  for (uint32_t r = 0; r < RM; ++r) {
+    const uint32_t pl = place(r), b = b0 + pl, cell0 = b * 64u + l.col * 4u;
+    const bool valid = b < b1;
+    rM[r] = hw[r] = 0u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      rP[r][k] = rR[r][k] = rZ[r][k] = 0.0f;
+      if (!WIDE) rG[k] = rY[k] = 1.0f;
+    }
+    if (first_block(r) >= b1) continue;
+    uint32_t nb[6] = {NONE, NONE, NONE, NONE, NONE, NONE};
+    if (valid) {
+#pragma unroll
+      for (uint32_t f = 0; f < 6u; ++f) {
+        const uint32_t step = f < 2u ? 9u : (f < 4u ? 3u : 1u);
+        const uint32_t n = d.block_nb[(size_t)b * 27u + ((f & 1u) ? 13u + step : 13u - step)];
+        nb[f] = n == NONE ? NONE : (n >= b0 && n < b1 ? n - b0 : n | QUAD_FAR);
+      }
+    }
+    const QuadLinks q = {l.x3 ? nb[0] : (l.x0 ? nb[1] : NONE), l.y3 ? nb[2] : (l.y0 ? nb[3] : NONE), nb[4], nb[5]};
+    rM[r] = quad_mask(d, cell0, valid, l);
+    hw[r] = quad_flags(d, nb, q, l, b0, b1);
+    float bv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, d0[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (valid) {
+      quad_load(cR, cell0, l.odd, rR[r]);
+      quad_load(d.bvec, cell0, l.odd, bv);
+      quad_load(cD, cell0, l.odd, d0);
+      quad_load(p0, cell0, l.odd, rP[r]);
+    }
+    lds.d[pl][l.col] = make_float4(d0[0], d0[1], d0[2], d0[3]);
+    // The far halo's directions as the solve found them, 0 where they are not water.
+    auto far4 = [&](uint32_t link, uint32_t water, float* o) {
+      if (!quad_far(link)) return;
+      const float4 v = *reinterpret_cast<const float4*>(cD + (size_t)(link & ~QUAD_FAR) * 64u + l.col * 4u);
+      const float z[4] = {(water & 1u) ? v.x : 0.0f, (water & 2u) ? v.y : 0.0f, (water & 4u) ? v.z : 0.0f,
+                          (water & 8u) ? v.w : 0.0f};
+      quad_swap(z, o, l.odd);
+    };
+    auto far1 = [&](uint32_t link, uint32_t z, uint32_t water) -> float {
+      return quad_far(link) && water ? cD[(size_t)(link & ~QUAD_FAR) * 64u + l.col * 4u + z] : 0.0f;
+    };
+    if (WIDE) {
+      if (l.col < 6u) {
+        const uint32_t n = l.col == 0 ? nb[0] : l.col == 1 ? nb[1] : l.col == 2 ? nb[2] : l.col == 3 ? nb[3] : l.col == 4 ? nb[4] : nb[5];
+        lds.nb[pl][l.col] = n;
+        lds.slot[pl][l.col] = (uint16_t)(quad_far(n) ? atomicAdd(&lds.faces, 1u) : 0u);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+      float o[4];
+      if (quad_far(q.x)) {
+        far4(q.x, hw[r], o);
+        *reinterpret_cast<float4*>(face_at(pl, l.x3 ? 0u : 1u) + 4u * (l.col & 3u)) = make_float4(o[0], o[1], o[2], o[3]);
+      }
+      if (quad_far(q.y)) {
+        far4(q.y, hw[r] >> 4, o);
+        *reinterpret_cast<float4*>(face_at(pl, l.y3 ? 2u : 3u) + 4u * (l.col >> 2)) = make_float4(o[0], o[1], o[2], o[3]);
+      }
+      if (quad_far(q.m)) face_at(pl, 4u)[l.col] = far1(q.m, 3u, hw[r] & 256u);
+      if (quad_far(q.p)) face_at(pl, 5u)[l.col] = far1(q.p, 0u, hw[r] & 512u);
+    } else {
+      lk = q;
+      far4(q.x, hw[r], hD.x);
+      far4(q.y, hw[r] >> 4, hD.y);
+      hD.zm = far1(q.m, 3u, hw[r] & 256u);
+      hD.zp = far1(q.p, 0u, hw[r] & 512u);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float2 t = lds.diag[rM[r] >> (8 + 3 * k) & 7u];
+        rG[k] = t.x, rY[k] = t.y;
+      }
+    }
+    float g[4], y[4];
+    diag_of(rM[r], g, y);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (!(rM[r] >> k & 1u)) rR[r][k] = bv[k] = 0.0f;
+    precondition_quad(rR[r], g, y, fast, rM[r], l, mode, rZ[r]);
+    quad_publish(wz, b, rZ[r], hw[r] >> 14 & 15u, l, tag + 1u);
+    R v0[4], v1[4], v2[4];
+    uint32_t nw = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v0[k] = prod<R>(rR[r][k], rZ[r][k]);
+      v1[k] = prod<R>(rR[r][k], rR[r][k]);
+      v2[k] = prod<R>(bv[k], bv[k]);
+      nw += (uint32_t)__popcll(__ballot((rM[r] >> k & 1u) != 0u) >> (16u * l.q) & 0xffffull);
+    }
+    part(0, r, quad_tree<R>(v0));
+    part(1, r, quad_tree<R>(v1));
+    part(2, r, quad_tree<R>(v2));
+    part(3, r, (R)nw);
+  }
+  R tt[4];
+  SolveScalars<R> s;
+  bool go = solve_start<R>(d, tt, reduce<R>(d, sp, ++tag, 4, &lp, tt), s);
+  // From here on the waves without sets, but for the one that makes the reductions, would only
+  // take issue slots: they end.
+  const uint32_t holders = min((b1 - b0 + 3u) / 4u, SOLVE_WAVES);
+  const QuadWaves qw = {wv, min(holders, SOLVE_WAVES - 1u), wv < holders};
+  if (wv > qw.reducer) return;
+  const bool refresh_on = std::is_same<R, double>::value && d.sc->precision == NATRAY_CG_MIXED && d.sc->refresh_every > 0u;
+
+  // With one set the halo's z is awaited while the reduction before its use completes.
+  const QuadLinks far = {lk.x & ~QUAD_FAR, lk.y & ~QUAD_FAR, lk.m & ~QUAD_FAR, lk.p & ~QUAD_FAR};
+  QuadHalo hz{};
+  bool ok = true;
+  if (!WIDE && go) {
+    QuadWords q{};
+    const uint32_t want = quad_want(hw[0], true);
+    ok = quad_wait(d, wz, far, want, l, tag, q, quad_had(want));
+    quad_payload(q, want, l.odd, hz);
+  }
+  while (go) {
+    // solve_q (fluid.wgsl:508-534): the new direction, then q = A d.
+    float* const cDn = cD + (size_t)(1u - s.iters % 2u) * capc;
+    const float fb = (float)s.beta;
+    new_pass();
+#pragma unroll
+    for (uint32_t r = 0; r < RM; ++r) {
+      if (first_block(r) >= b1) continue;
+      const uint32_t pl = place(r), m = fresh(rM[r]);
+      const float4 o = lds.d[pl][l.col];
+      const float dn[4] = {(m & 1u) ? rZ[r][0] + fb * o.x : 0.0f, (m & 2u) ? rZ[r][1] + fb * o.y : 0.0f,
+                           (m & 4u) ? rZ[r][2] + fb * o.z : 0.0f, (m & 8u) ? rZ[r][3] + fb * o.w : 0.0f};
+      lds.d[pl][l.col] = make_float4(dn[0], dn[1], dn[2], dn[3]);
+      quad_store(cDn, (b0 + pl) * 64u + l.col * 4u, l.odd, dn, m);
+    }
+    wg_sync(false);
+    new_pass();
+#pragma unroll
+    for (uint32_t r = 0; r < RM; ++r) {
+      if (first_block(r) >= b1) continue;
+      const uint32_t pl = place(r), m = fresh(rM[r]), w = fresh(hw[r]), want = quad_want(w, true);
+      const QuadLinks k = links_of(r);
+      QuadHalo h;
+      if (WIDE) {
+        QuadWords q{};
+        QuadHalo z;
+        const QuadLinks far = {k.x & ~QUAD_FAR, k.y & ~QUAD_FAR, k.m & ~QUAD_FAR, k.p & ~QUAD_FAR};
+        ok = quad_wait(d, wz, far, want, l, tag, q, quad_had(want)) && ok;
+        quad_payload(q, want, l.odd, z);
+        far_d(r, w, z, fb, h);
+      } else {
+        far_d(r, w, hz, fb, h);
+      }
+      near_d(k, w, h);
+      float g[4], y[4], q[4];
+      diag_of(m, g, y);
+      const float4 o = lds.d[pl][l.col];
+      const float dn[4] = {o.x, o.y, o.z, o.w};
+      quad_row<float>(dn, g, h, l, q);
+      R v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        rZ[r][k] = (m >> k & 1u) ? q[k] : 0.0f;
+        v[k] = prod<R>(dn[k], rZ[r][k]);
+      }
+      part(0, r, quad_tree<R>(v));
+    }
+    if (!quad_reduce<R, 1>(d, sp, ++tag, qw, lp, tt, [] {}, [] { return true; }) || !ok) break;
+    // solve_alpha (fluid.wgsl:536-541)
+    s.alpha = tt[0] > (R)0 ? s.rz / tt[0] : (R)0;
+    const float fa = (float)s.alpha;
+    const bool refresh = refresh_on && (s.iters + 1u) % d.sc->refresh_every == 0u;
+    // solve_update (fluid.wgsl:543-559): p += alpha d, r -= alpha q, z = M^-1 r; with the
+    // refresh, r = b - A p in double instead, every neighbour's p from its words.
+    new_pass();
+#pragma unroll
+    for (uint32_t r = 0; r < RM; ++r) {
+      if (first_block(r) >= b1) continue;
+      const uint32_t pl = place(r), m = fresh(rM[r]);
+      const float4 o = lds.d[pl][l.col];
+      const float dn[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (m >> k & 1u) rP[r][k] += fa * dn[k];
+        rR[r][k] = (m >> k & 1u) ? rR[r][k] - fa * rZ[r][k] : 0.0f;
+      }
+      if (refresh) quad_publish(wp, b0 + pl, rP[r], hw[r] >> 18 & 15u, l, tag + 1u);
+    }
+    new_pass();
+#pragma unroll
+    for (uint32_t r = 0; r < RM; ++r) {
+      if (first_block(r) >= b1) continue;
+      const uint32_t pl = place(r), m = fresh(rM[r]), w = fresh(hw[r]);
+      float g[4], y[4];
+      diag_of(m, g, y);
+      if (refresh) {
+        QuadWords q{};
+        const uint32_t want = quad_want(w, false);
+        ok = quad_wait(d, wp, ids_of(links_of(r)), want, l, tag + 1u, q, quad_had(want)) && ok;
+        QuadHalo h;
+        quad_payload(q, want, l.odd, h);
+        float p[4], bv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (m & 15u) quad_load(d.bvec, (b0 + pl) * 64u + l.col * 4u, l.odd, bv);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) p[k] = (m >> k & 1u) ? rP[r][k] : 0.0f;
+        double ap[4];
+        quad_row<double>(p, g, h, l, ap);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) rR[r][k] = (m >> k & 1u) ? (float)((double)bv[k] - ap[k]) : 0.0f;
+      }
+      precondition_quad(rR[r], g, y, fast, m, l, mode, rZ[r]);
+      R v0[4], v1[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v0[k] = prod<R>(rR[r][k], rZ[r][k]);
+        v1[k] = prod<R>(rR[r][k], rR[r][k]);
+      }
+      part(0, r, quad_tree<R>(v0));
+      part(1, r, quad_tree<R>(v1));
+    }
+    ++tag;
+    QuadWords q{};
+    uint32_t have = quad_had(quad_want(hw[0], true));
+    auto publish_z = [&]() {
+      new_pass();
+#pragma unroll
+      for (uint32_t r = 0; r < RM; ++r)
+        if (first_block(r) < b1) quad_publish(wz, b0 + place(r), rZ[r], fresh(hw[r]) >> 14 & 15u, l, tag);
+    };
+    auto halo_z = [&]() -> bool {
+      if (WIDE) return true;
+      const uint32_t want = quad_want(hw[0], true);
+      if (!quad_words(wz, far, want, l, tag, q, have)) return false;
+      quad_payload(q, want, l.odd, hz);
+      return true;
+    };
+    if (!quad_reduce<R, 2>(d, sp, tag, qw, lp, tt, publish_z, halo_z)) break;
+    go = solve_beta<R>(d, tt, s);
+  }
+  // The fields the other kernels and the host read: p, r, z and q of the water cells (solve_q
+  // stored the directions). q is formed again from the last direction: the same bits.
+  new_pass();
+#pragma unroll
+  for (uint32_t r = 0; r < RM; ++r) {
+    if (first_block(r) >= b1) continue;
+    const uint32_t pl = place(r), cell0 = (b0 + pl) * 64u + l.col * 4u, m = rM[r], w = hw[r];
+    quad_store(cP, cell0, l.odd, rP[r], m);
+    quad_store(cR, cell0, l.odd, rR[r], m);
+    quad_store(cZ, cell0, l.odd, rZ[r], m);
+    if (s.iters == 0u) continue;
+    QuadHalo h;
+    far_d_kept(r, w, h);
+    near_d(links_of(r), w, h);
+    float g[4], y[4], q[4];
+    diag_of(m, g, y);
+    const float4 o = lds.d[pl][l.col];
+    const float dn[4] = {o.x, o.y, o.z, o.w};
+    quad_row<float>(dn, g, h, l, q);
+    quad_store(cQ, cell0, l.odd, q, m);
+  }
+  solve_finish<R>(d, sp, tag, s);
 }
 
 template <bool MIXED, class L>
@@ -1965,7 +2930,6 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_solve(L l) {
   const View v = view(l);
   const Dev& d = v.d;
   using R = typename std::conditional<MIXED, double, float>::type;
-  constexpr uint32_t RM = SOLVE_RMAX;
   if (d.st->dt_ns == 0u) return;
   // A test of the plain launch's failure path: the last workgroup stays out, as one that is not
   // resident would, and the others' bounded waits abort the solve.
@@ -1974,218 +2938,19 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_solve(L l) {
   }
   // An earlier solve of this batch lost its barrier: the host reports it, nothing more runs.
   if (__hip_atomic_load(d.bar + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
-  const SolveSpan sp = solve_span(v, true);
-  uint32_t tag = __hip_atomic_load(d.bar + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (!sp.in_regs) {
-    // Called with the device copy of Dev, which the callee reads with scalar loads.
+  SolveSpan sp = solve_span(v, SOLVE_BLOCKS, true);
+  if (sp.in_regs) {
+    // A workgroup without a chunk has nothing to do; the one with the first chunk leads.
+    if (sp.c0 == sp.c1 && (sp.m != 0u || v.wg != 0u)) return;
+    sp.lead = sp.c0 == 0u;
+  }
+  const uint32_t tag = __hip_atomic_load(d.bar + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (sp.narrow)
+    solve_quads<R, 1>(d, sp, tag);
+  else if (sp.in_regs)
+    solve_quads<R, QUAD_WIDE>(d, sp, tag);
+  else  // called with the device copy of Dev, which the callee reads with scalar loads
     solve_memory<MIXED>(d.self, sp, tag);
-    return;
-  }
-
-  // Register form. Wave wv holds blocks b0 + wv + SOLVE_WAVES r (r < RM), the blocks
-  // for_blocks gives it. Per block and lane: p, r, z, the direction d, q, diag, the neighbour
-  // mask, and for each axis the halo cell across the block face (when it is water) with its
-  // direction and p as this wave rebuilds them, and its tagged z as last loaded.
-  const uint32_t mode = d.sc->precond;
-  const uint32_t b0 = sp.b0, b1 = sp.b1;
-  const uint32_t capc = d.capc;
-  float* const cP = d.cf + (size_t)NATRAY_F_P * capc;
-  const float* const p0 = start_pressure(d);
-  unsigned long long* const hz = d.hz;
-  __shared__ LPart<R> lp;
-  for_blocks<SOLVE_WAVES>(d, b0, b1, SOLVE_WAVES, [&](uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk) {
-    R v[4];
-    init_cell<R>(d, b, lane, lx, ly, lz, lk, d.hz, tag + 1u, v, p0);
-    if (lane == 0)
-      for (uint32_t k = 0; k < 4u; ++k) lp.v[k][b - b0] = v[k];
-  });
-  R tt[4];
-  SolveScalars<R> s;
-  bool go = solve_start<R>(d, tt, reduce<R>(d, sp, ++tag, 4, &lp, tt), s);
-  const bool refresh_on = MIXED && d.sc->precision == NATRAY_CG_MIXED && d.sc->refresh_every > 0u;
-
-  __shared__ uint32_t lkr[SOLVE_WAVES][SOLVE_RMAX][27];
-  const uint32_t wv = threadIdx.x >> 6, ln = lane_id();
-  const int lx = (int)(ln >> 4), ly = (int)((ln >> 2) & 3u), lz = (int)(ln & 3u);
-  // Mask bit of the neighbour across the block face on each axis, if this lane is on one.
-  const uint32_t face_bit[3] = {lx == 0 ? 1u : (lx == 3 ? 2u : 0u), ly == 0 ? 4u : (ly == 3 ? 8u : 0u),
-                                lz == 0 ? 16u : (lz == 3 ? 32u : 0u)};
-  float rP[RM], rR[RM], rZ[RM], rD[RM], rQ[RM], rDg[RM];
-  uint32_t rM[RM];
-  float hD[RM][3], hPr[RM][3];
-  unsigned long long hW[RM][3];
-  auto halo_cell = [&](uint32_t r, int a) -> uint32_t {
-    const int sg = (face_bit[a] & 0x2Au) ? 1 : -1;
-    return nbr(lkr[wv][r], lx, ly, lz, a == 0 ? sg : 0, a == 1 ? sg : 0, a == 2 ? sg : 0);
-  };
-  auto has_halo = [&](uint32_t r, int a) -> bool { return (rM[r] & face_bit[a]) != 0u; };
-#pragma unroll
-  for (uint32_t r = 0; r < RM; ++r) {
-    const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-    if (b < b1 && ln < 27) lkr[wv][r][ln] = d.block_nb[b * 27u + ln];
-  }
-  __syncthreads();
-#pragma unroll
-  for (uint32_t r = 0; r < RM; ++r) {
-    rP[r] = rR[r] = rZ[r] = rD[r] = rQ[r] = 0.0f;
-    rDg[r] = 1.0f;
-    rM[r] = 0;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      hD[r][a] = hPr[r][a] = 0.0f;
-      hW[r][a] = 0ull;
-    }
-    const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-    if (b < b1) {
-      const uint32_t cell = b * 64u + ln;
-      rM[r] = d.nbm[cell];
-      rP[r] = p0[cell];
-      rR[r] = d.cf[(size_t)NATRAY_F_R * capc + cell];
-      rZ[r] = d.cf[(size_t)NATRAY_F_Z * capc + cell];
-      rDg[r] = d.cf[(size_t)NATRAY_F_DIAG * capc + cell];
-      rD[r] = d.cf[(size_t)NATRAY_F_D * capc + cell];
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        if (!has_halo(r, a)) continue;
-        const uint32_t o = halo_cell(r, a);
-        hD[r][a] = d.cf[(size_t)NATRAY_F_D * capc + o];
-        if (refresh_on) hPr[r][a] = p0[o];
-        hW[r][a] = load_word(&hz[o]);
-      }
-    }
-  }
-
-  bool ok = true;
-  while (go) {
-    // solve_q (fluid.wgsl:508-534): the new direction and q = A d.
-    float* cDn = d.cf + (size_t)(NATRAY_F_D + 1u - s.iters % 2u) * capc;
-    const float fb = (float)s.beta;
-#pragma unroll
-    for (uint32_t r = 0; r < RM; ++r) {
-      const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-      if (b >= b1) continue;
-      const uint32_t cell = b * 64u + ln, mask = rM[r];
-      // Halo directions: z across the face (tagged with the last reduction's tag), rebuilt
-      // as the owner does, z + beta d_old.
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        if (!has_halo(r, a)) continue;
-        uint32_t spins = 0;
-        while ((uint32_t)(hW[r][a] >> 32) != tag) {
-          __builtin_amdgcn_s_sleep(1);
-          hW[r][a] = load_word(&hz[halo_cell(r, a)]);
-          if ((++spins & 255u) == 0u &&
-              (__hip_atomic_load(d.bar + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u || spins > kSpinLimit)) {
-            __hip_atomic_store(d.bar + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            ok = false;
-            break;
-          }
-        }
-        hD[r][a] = __uint_as_float((uint32_t)hW[r][a]) + fb * hD[r][a];
-      }
-      const float dn = rZ[r] + fb * rD[r];
-      const Faces f = block_faces(dn);
-      R v = (R)0;
-      if (mask & 64u) {
-        float q = rDg[r] * dn;
-        if (mask & 1u) q -= lx > 0 ? f.xm : hD[r][0];
-        if (mask & 2u) q -= lx < 3 ? f.xp : hD[r][0];
-        if (mask & 4u) q -= ly > 0 ? f.ym : hD[r][1];
-        if (mask & 8u) q -= ly < 3 ? f.yp : hD[r][1];
-        if (mask & 16u) q -= lz > 0 ? f.zm : hD[r][2];
-        if (mask & 32u) q -= lz < 3 ? f.zp : hD[r][2];
-        cDn[cell] = dn;
-        rD[r] = dn;
-        rQ[r] = q;
-        v = prod<R>(dn, q);
-      }
-      v = wave_tree<R>(v);
-      if (ln == 0) lp.v[0][b - b0] = v;
-    }
-    if (!reduce<R>(d, sp, ++tag, 1, &lp, tt) || !ok) break;
-    // solve_alpha (fluid.wgsl:536-541)
-    s.alpha = tt[0] > (R)0 ? s.rz / tt[0] : (R)0;
-    const float fa = (float)s.alpha;
-    const bool refresh = refresh_on && (s.iters + 1u) % d.sc->refresh_every == 0u;
-    // solve_update (fluid.wgsl:543-559): p += alpha d, r -= alpha q, z = M^-1 r; with the
-    // refresh, r = b - A p in double instead, p of the halo rebuilt as its owner updates it.
-#pragma unroll
-    for (uint32_t r = 0; r < RM; ++r) {
-      const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-      if (b >= b1) continue;
-      const uint32_t cell = b * 64u + ln, mask = rM[r];
-      const bool water = (mask & 64u) != 0u;
-      float rr = 0.0f, diag = 1.0f;
-      if (water) {
-        rP[r] += fa * rD[r];
-        rR[r] = rR[r] - fa * rQ[r];
-        rr = rR[r];
-        diag = rDg[r];
-      }
-      if (refresh_on) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-          if (has_halo(r, a)) hPr[r][a] += fa * hD[r][a];
-      }
-      if (refresh) {
-        const float p = rP[r];
-        const Faces f = block_faces(p);
-        if (water) {
-          double ap = (double)diag * (double)p;
-          if (mask & 1u) ap -= (double)(lx > 0 ? f.xm : hPr[r][0]);
-          if (mask & 2u) ap -= (double)(lx < 3 ? f.xp : hPr[r][0]);
-          if (mask & 4u) ap -= (double)(ly > 0 ? f.ym : hPr[r][1]);
-          if (mask & 8u) ap -= (double)(ly < 3 ? f.yp : hPr[r][1]);
-          if (mask & 16u) ap -= (double)(lz > 0 ? f.zm : hPr[r][2]);
-          if (mask & 32u) ap -= (double)(lz < 3 ? f.zp : hPr[r][2]);
-          rr = (float)((double)d.bvec[cell] - ap);
-          rR[r] = rr;
-        }
-      }
-      const float z = precondition(rr, diag, water, lx, ly, lz, mode);
-      if (water) {
-        rZ[r] = z;
-        store_word(&hz[cell], tag_word(tag + 1u, __float_as_uint(z)));
-      }
-      const R v0 = wave_tree<R>(prod<R>(rr, z)), v1 = wave_tree<R>(prod<R>(rr, rr));
-      if (ln == 0) {
-        lp.v[0][b - b0] = v0;
-        lp.v[1][b - b0] = v1;
-      }
-    }
-    // Halo z for the next solve_q: neighbours publish it before their part of the reduction
-    // below, so every wave reloads its stale halo words while the reduction completes.
-    auto halo_poll = [&](uint32_t want) -> bool {
-      bool fresh = true;
-#pragma unroll
-      for (uint32_t r = 0; r < RM; ++r) {
-        if (b0 + wv + SOLVE_WAVES * r >= b1) continue;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          if (!has_halo(r, a) || (uint32_t)(hW[r][a] >> 32) == want) continue;
-          hW[r][a] = load_word(&hz[halo_cell(r, a)]);
-          fresh = fresh && (uint32_t)(hW[r][a] >> 32) == want;
-        }
-      }
-      return fresh;
-    };
-    if (!reduce<R>(d, sp, ++tag, 2, &lp, tt, halo_poll)) break;
-    go = solve_beta<R>(d, tt, s);
-  }
-  // The fields the other kernels and the host read: p, r, z and q of this wave's water cells
-  // (solve_q stored the directions).
-#pragma unroll
-  for (uint32_t r = 0; r < RM; ++r) {
-    const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-    if (b < b1 && (rM[r] & 64u)) {
-      const uint32_t cell = b * 64u + ln;
-      cP[cell] = rP[r];
-      d.cf[(size_t)NATRAY_F_R * capc + cell] = rR[r];
-      d.cf[(size_t)NATRAY_F_Z * capc + cell] = rZ[r];
-      if (s.iters > 0u) d.cf[(size_t)NATRAY_F_Q * capc + cell] = rQ[r];
-    }
-  }
-  solve_finish<R>(d, sp, tag, s);
 }
 
 // ---- pipelined CG (NATRAY_CG_PIPELINED; not in the reference) ---------------------------------------
@@ -2452,7 +3217,7 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_solve_pipe(L l) {
     if (d.solve_plain == 2u && v.wg + 1u == v.wgs) return;
   }
   if (__hip_atomic_load(d.bar + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
-  const SolveSpan sp = solve_span(v, false);
+  const SolveSpan sp = solve_span(v, SOLVE_WAVES * SOLVE_RMAX, false);
   uint32_t tag = __hip_atomic_load(d.bar + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (!sp.in_regs) {
     solve_pipe_memory(d.self, sp, tag);
@@ -4644,6 +5409,7 @@ int launch_solve(const Target& t, void* stream, int kind) {
   void* args_one[] = {&one};
   void* args_many[] = {&many};
   const void* fn;
+  if (kind != (int)NATRAY_CG_PIPELINED) NATRAY_LAUNCH(k_solve_rows, LK_WAVES, 256, t, S(stream));
   if (kind == (int)NATRAY_CG_PIPELINED)
     fn = t.d ? (const void*)k_solve_pipe<One> : (const void*)k_solve_pipe<Many>;
   else if (kind == (int)NATRAY_CG_MIXED)

@@ -70,6 +70,50 @@ __device__ __forceinline__ R lane_tree(R v) {
   return v;
 }
 
+// DPP moves whose result the compiler can fold into the operation that uses it. Value of lane
+// l + N of the row (0 where that lies past the row's end)
+template <int N>
+__device__ __forceinline__ float row_down(float v) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x100 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ __forceinline__ double row_down(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, 0x100 + N, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), 0x100 + N, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// lane_tree's sum in lane 0 alone: each step takes the half it needs of a lane swap as it comes.
+__device__ __forceinline__ float lane_sum0(float v) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v += __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v += __uint_as_float(b[1]);
+  v += row_down<8>(v);
+  v += row_down<4>(v);
+  v += row_down<2>(v);
+  return v + row_down<1>(v);
+}
+__device__ __forceinline__ double lane_sum0(double v) {
+  v += lane_xor32(v);
+  v += lane_xor16(v);
+  v += row_down<8>(v);
+  v += row_down<4>(v);
+  v += row_down<2>(v);
+  return v + row_down<1>(v);
+}
+// ... of lane (l - N) mod 16 of the row ...
+template <int N>
+__device__ __forceinline__ float row_rot(float v) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x120 + N, 0xf, 0xf, true));
+}
+// ... and of lane (l - N) mod 4 of the quad.
+template <int N>
+__device__ __forceinline__ float quad_rot(float v) {
+  constexpr int sel = ((4 - N) & 3) | ((5 - N) & 3) << 2 | ((6 - N) & 3) << 4 | ((7 - N) & 3) << 6;
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), sel, 0xf, 0xf, true));
+}
+
 // The six face neighbours of each lane's cell inside its 4x4x4 block. A neighbour outside the
 // block gives a meaningless value; callers mask those.
 struct Faces {
