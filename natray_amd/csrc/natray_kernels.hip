@@ -4370,99 +4370,129 @@ __global__ __launch_bounds__(256) void k_mark_rubber(L l) {
 
 // mem_splat (membrane.wgsl:182-216): every vertex with area adds its area (mm^2) and area
 // times velocity to its own cell (A_MW, A_MV); a vertex on the water also spreads its push
-// (A_MF) and area (A_MA) over the 27 cells around it with the particles' B-spline weights.
+// (A_MF) and area (A_MA) over the 27 cells around it with the particles' B-spline weights. A
+// vertex takes 32 lanes, 27 for the cells and 4 for the own cell's sums: with one thread per
+// vertex, the 27 look-ups of a cell's block were a chain of dependent loads, and 41k vertices
+// were two waves a compute unit to hide it: 131 us at 41k vertices, now 51, of which the 2.2M
+// atomics take most. The sums are integers, so their order is free.
 template <class L>
 __global__ __launch_bounds__(256) void k_mem_splat(L l) {
   const View v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
-  const uint32_t i = v.wg * blockDim.x + threadIdx.x;
-  if (i >= mem_count(d) || d.mem_mass[i] == 0.0f) return;
-  const float2 pa = d.mem_push[i];
-  if (pa.y <= 0.0f) return;
-  const float4 p = d.mem_x[i];
-  int cx, cy, cz;
-  point_cell(d, p, cx, cy, cz);
-  const uint32_t own = cell_at(d, cx, cy, cz);
-  if (own != NONE) {
-    const float a = pa.y * 1e6f;
-    const float4 mv = d.mem_v[i];
-    atomicAdd(&accr(d, NATRAY_A_MW, own), to_fp(a, NATRAY_FP_A));
-    atomicAdd(&accr(d, NATRAY_A_MV + 0u, own), to_fp(a * mv.x, NATRAY_FP_A));
-    atomicAdd(&accr(d, NATRAY_A_MV + 1u, own), to_fp(a * mv.y, NATRAY_FP_A));
-    atomicAdd(&accr(d, NATRAY_A_MV + 2u, own), to_fp(a * mv.z, NATRAY_FP_A));
-  }
-  if (!on_water(d, i)) return;
   const natray_params* U = d.U;
   const float h = U->origin[3];
-  const float x[3] = {(p.x - U->origin[0]) / h - 0.5f, (p.y - U->origin[1]) / h - 0.5f, (p.z - U->origin[2]) / h - 0.5f};
-  int base[3];
-  float w[3][3];
+  const uint32_t n = mem_count(d), lane = threadIdx.x & 31u;
+  for (uint32_t i = (v.wg * blockDim.x + threadIdx.x) >> 5; i < n; i += v.wgs * blockDim.x >> 5) {
+    const float2 pa = d.mem_push[i];
+    if (d.mem_mass[i] == 0.0f || pa.y <= 0.0f || lane > 30u) continue;
+    const float4 p = d.mem_x[i];
+    if (lane >= 27u) {
+      int cx, cy, cz;
+      point_cell(d, p, cx, cy, cz);
+      const uint32_t own = cell_at(d, cx, cy, cz);
+      if (own == NONE) continue;
+      const float a = pa.y * 1e6f;
+      const float4 mv = d.mem_v[i];
+      const float val = lane == 27u ? a : a * (lane == 28u ? mv.x : (lane == 29u ? mv.y : mv.z));
+      const uint32_t f = lane == 27u ? NATRAY_A_MW : NATRAY_A_MV + (lane - 28u);
+      atomicAdd(&accr(d, f, own), to_fp(val, NATRAY_FP_A));
+      continue;
+    }
+    if (!on_water(d, i)) continue;
+    const int a = (int)(lane / 9u), b = (int)(lane / 3u % 3u), c = (int)(lane % 3u);
+    const float x[3] = {(p.x - U->origin[0]) / h - 0.5f, (p.y - U->origin[1]) / h - 0.5f, (p.z - U->origin[2]) / h - 0.5f};
+    int base[3];
+    float w[3][3];
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const float bf = floorf(x[k] - 0.5f);
-    base[k] = (int)bf;
-    axis_weights(x[k] - bf, w[k]);
+    for (int k = 0; k < 3; ++k) {
+      const float bf = floorf(x[k] - 0.5f);
+      base[k] = (int)bf;
+      axis_weights(x[k] - bf, w[k]);
+    }
+    const uint32_t cell = cell_at(d, base[0] + a, base[1] + b, base[2] + c);
+    if (cell == NONE) continue;
+    auto pick = [](const float* q, int k) -> float { return k == 0 ? q[0] : (k == 1 ? q[1] : q[2]); };
+    const float wt = pick(w[0], a) * pick(w[1], b) * pick(w[2], c);
+    atomicAdd(&accr(d, NATRAY_A_MF, cell), to_fp(wt * pa.x, NATRAY_FP_F));
+    atomicAdd(&accr(d, NATRAY_A_MA, cell), to_fp(wt * pa.y * 1e6f, NATRAY_FP_A));
   }
-  for (int a = 0; a < 3; ++a)
-    for (int b = 0; b < 3; ++b)
-      for (int c = 0; c < 3; ++c) {
-        const uint32_t cell = cell_at(d, base[0] + a, base[1] + b, base[2] + c);
-        if (cell == NONE) continue;
-        const float wt = w[0][a] * w[1][b] * w[2][c];
-        atomicAdd(&accr(d, NATRAY_A_MF, cell), to_fp(wt * pa.x, NATRAY_FP_F));
-        atomicAdd(&accr(d, NATRAY_A_MA, cell), to_fp(wt * pa.y * 1e6f, NATRAY_FP_A));
-      }
 }
 
-// sample_grid (membrane.wgsl:218-237): the B-spline sums around x (in cells, on the lattice)
-// of cell field fu weighted by transfer field fw, and of the weights.
-__device__ __forceinline__ float2 sample_grid(const Dev& d, const float x[3], uint32_t fu, uint32_t fw) {
-  int base[3];
-  float w[3][3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const float bf = floorf(x[k] - 0.5f);
-    base[k] = (int)bf;
-    axis_weights(x[k] - bf, w[k]);
-  }
-  float sx = 0.0f, sy = 0.0f;
-  for (int a = 0; a < 3; ++a)
-    for (int b = 0; b < 3; ++b)
-      for (int c = 0; c < 3; ++c) {
-        const uint32_t cell = cell_at(d, base[0] + a, base[1] + b, base[2] + c);
-        if (cell == NONE) continue;
-        const float wt = w[0][a] * w[1][b] * w[2][c] * from_fp(accr(d, fw, cell), NATRAY_FP_W);
-        sx = sx + wt * cfr(d, fu, cell);
-        sy = sy + wt;
-      }
-  return make_float2(sx, sy);
-}
-
-// mem_sample (membrane.wgsl:239-254): the velocity of the faces around each vertex, weighted
-// by the water they carry, and how full of water the cells around it are (a bulk cell holds 8
-// particles whose weights sum to 1 each).
+// mem_sample (membrane.wgsl:239-254) with sample_grid (:218-237): the velocity of the faces
+// around each vertex, weighted by the water they carry, and how full of water the cells around
+// it are (a bulk cell holds 8 particles whose weights sum to 1 each): B-spline sums over 27 cells
+// on each of four lattices, in the reference's order. A vertex takes 32 lanes, one per cell, so
+// that the cells of an x plane of a block are one line of a load, and all four lattices' loads
+// are in flight together; the terms then go through LDS to one lane per lattice, which adds them
+// in order. A cell that is in no block adds zero to sums that are never -0. (58 us at 41k
+// vertices with one thread per vertex, 38 with one per lattice and its loads issued at once; now
+// 20.)
+constexpr uint32_t MEM_VERTS = 8;  // vertices per workgroup
 template <class L>
 __global__ __launch_bounds__(256) void k_mem_sample(L l) {
   const View v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
-  const uint32_t i = v.wg * blockDim.x + threadIdx.x;
-  if (i >= mem_count(d) || d.mem_mass[i] == 0.0f) return;
+  __shared__ float2 term[MEM_VERTS][4][28];
   const natray_params* U = d.U;
   const float h = U->origin[3];
-  const float4 p = d.mem_x[i];
-  const float x[3] = {(p.x - U->origin[0]) / h, (p.y - U->origin[1]) / h, (p.z - U->origin[2]) / h};
-  float vel[3];
+  const uint32_t n = mem_count(d), lane = threadIdx.x & 31u, row = threadIdx.x >> 5;
+  const int a = (int)(lane / 9u), b = (int)(lane / 3u % 3u), c = (int)(lane % 3u);
+  auto pick = [](const float* q, int k) -> float { return k == 0 ? q[0] : (k == 1 ? q[1] : q[2]); };
+  for (uint32_t i0 = v.wg * MEM_VERTS; i0 < n; i0 += v.wgs * MEM_VERTS) {
+    const uint32_t i = i0 + row;
+    if (i < n && lane < 27u) {
+      const float4 p = d.mem_x[i];
+      const float x[3] = {(p.x - U->origin[0]) / h, (p.y - U->origin[1]) / h, (p.z - U->origin[2]) / h};
+      uint32_t cell[4];
+      float wt[4];
 #pragma unroll
-  for (uint32_t dim = 0; dim < 3; ++dim) {
-    const float xs[3] = {dim == 0 ? x[0] : x[0] - 0.5f, dim == 1 ? x[1] : x[1] - 0.5f, dim == 2 ? x[2] : x[2] - 0.5f};
-    const float2 s = sample_grid(d, xs, NATRAY_F_U + dim, NATRAY_A_WT(dim));
-    vel[dim] = s.y > 1e-6f ? s.x / s.y : 0.0f;
+      for (int q = 0; q < 4; ++q) {
+        int at[3];
+        float w[3];
+        const int o[3] = {a, b, c};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const float xs = q == k ? x[k] : x[k] - 0.5f;
+          const float bf = floorf(xs - 0.5f);
+          float ws[3];
+          axis_weights(xs - bf, ws);
+          at[k] = (int)bf + o[k];
+          w[k] = pick(ws, o[k]);
+        }
+        cell[q] = cell_at(d, at[0], at[1], at[2]);
+        wt[q] = w[0] * w[1] * w[2];
+      }
+      float cw[4], cu[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t cl = cell[q] == NONE ? 0u : cell[q];
+        cw[q] = from_fp(accr(d, q < 3 ? NATRAY_A_WT(q) : NATRAY_A_WC, cl), NATRAY_FP_W);
+        cu[q] = q < 3 ? cfr(d, NATRAY_F_U + q, cl) : 0.0f;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float w = wt[q] * cw[q];
+        term[row][q][lane] = cell[q] == NONE ? make_float2(0.0f, 0.0f) : make_float2(w * cu[q], w);
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < 4u * MEM_VERTS) {
+      const uint32_t q = threadIdx.x & 3u, r = threadIdx.x >> 2, k = i0 + r;
+      if (k < n && d.mem_mass[k] != 0.0f) {
+        float sx = 0.0f, sy = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 27; ++j) {
+          const float2 e = term[r][q][j];
+          sx = sx + e.x;
+          sy = sy + e.y;
+        }
+        reinterpret_cast<float*>(d.mem_water)[4u * k + q] = q == 3u ? sy / 8.0f : (sy > 1e-6f ? sx / sy : 0.0f);
+      }
+    }
+    __syncthreads();
   }
-  const float xc[3] = {x[0] - 0.5f, x[1] - 0.5f, x[2] - 0.5f};
-  const float fill = sample_grid(d, xc, NATRAY_F_TYPE, NATRAY_A_WC).y / 8.0f;
-  d.mem_water[i] = make_float4(vel[0], vel[1], vel[2], fill);
 }
 
 // ---- bullets: their step and the water's push (bullet.wgsl:100-386) ------------------------------
@@ -5476,11 +5506,19 @@ int launch_g2p(const Target& t, void* stream) {
 }
 
 int launch_mem_splat(const Target& t, void* stream) {
-  NATRAY_LAUNCH(k_mem_splat, LK_VERTS, 256, t, S(stream));
+  // 32 lanes a vertex.
+  if (t.d)
+    hipLaunchKernelGGL(k_mem_splat<One>, dim3(t.grid[LK_VERTS] * 32u), dim3(256), 0, S(stream), One{*t.d});
+  else
+    hipLaunchKernelGGL(k_mem_splat<Many>, dim3(t.grid[LK_VERTS]), dim3(256), 0, S(stream), Many{t.scenes, t.map[LK_VERTS]});
   return (int)hipGetLastError();
 }
 int launch_mem_sample(const Target& t, void* stream) {
-  NATRAY_LAUNCH(k_mem_sample, LK_VERTS, 256, t, S(stream));
+  // 32 lanes a vertex.
+  if (t.d)
+    hipLaunchKernelGGL(k_mem_sample<One>, dim3(t.grid[LK_VERTS] * 32u), dim3(256), 0, S(stream), One{*t.d});
+  else
+    hipLaunchKernelGGL(k_mem_sample<Many>, dim3(t.grid[LK_VERTS]), dim3(256), 0, S(stream), Many{t.scenes, t.map[LK_VERTS]});
   return (int)hipGetLastError();
 }
 
