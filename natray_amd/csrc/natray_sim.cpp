@@ -1234,14 +1234,13 @@ int natray_sim_water_stats(natray_sim* s, natray_water_stats* out) {
   uint32_t slots = 1024;
   while (slots < 2u * n) slots <<= 1;
   const uint32_t groups = std::min<uint32_t>(1024u, (n + 255u) / 256u);
-  // One allocation: the keys, the counts, the workgroups' parts and the full-cell counter.
+  // One allocation: the keys, the counts and the workgroups' parts.
   const size_t off_counts = (size_t)slots * 8, off_parts = off_counts + (size_t)slots * 4,
-               off_full = off_parts + (size_t)groups * sizeof(natray::WaterPart), bytes = off_full + 256;
+               bytes = off_parts + (size_t)groups * sizeof(natray::WaterPart);
   char* buf = nullptr;
   hipError_t e = hipMalloc(&buf, bytes);
   if (e != hipSuccess) return fail(NATRAY_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
   std::vector<natray::WaterPart> parts(groups);
-  uint32_t full = 0;
   int rc = NATRAY_OK;
   auto step = [&](hipError_t x) {
     if (x != hipSuccess && rc == NATRAY_OK) rc = fail(NATRAY_E_HIP, std::string("HIP: ") + hipGetErrorString(x));
@@ -1250,15 +1249,11 @@ int natray_sim_water_stats(natray_sim* s, natray_water_stats* out) {
   auto* keys = reinterpret_cast<unsigned long long*>(buf);
   auto* counts = reinterpret_cast<uint32_t*>(buf + off_counts);
   auto* dparts = reinterpret_cast<natray::WaterPart*>(buf + off_parts);
-  auto* dfull = reinterpret_cast<uint32_t*>(buf + off_full);
   const float origin[3] = {s->U.origin[0], s->U.origin[1], s->U.origin[2]};
-  if (step(hipMemsetAsync(keys, 0xff, (size_t)slots * 8, s->stream)) &&
-      step(hipMemsetAsync(counts, 0, (size_t)slots * 4, s->stream)) && step(hipMemsetAsync(dfull, 0, 4, s->stream)) &&
-      step((hipError_t)natray::launch_water_stats(s->D.P, n, origin, s->U.origin[3], keys, counts, slots, dparts, groups,
-                                                  dfull, s->stream)) &&
+  if (step((hipError_t)natray::launch_water_stats(s->D.P, n, origin, s->U.origin[3], keys, counts, slots, dparts, groups,
+                                                  s->stream)) &&
       step(hipMemcpyAsync(parts.data(), dparts, (size_t)groups * sizeof(natray::WaterPart), hipMemcpyDeviceToHost,
-                          s->stream)) &&
-      step(hipMemcpyAsync(&full, dfull, 4, hipMemcpyDeviceToHost, s->stream)))
+                          s->stream)))
     step(hipStreamSynchronize(s->stream));
   const hipError_t ef = hipFree(buf);
   if (rc != NATRAY_OK) return rc;
@@ -1277,6 +1272,7 @@ int natray_sim_water_stats(natray_sim* s, natray_water_stats* out) {
       fast = p.fastest;
     }
     r.alive += p.alive;
+    r.full_cells += p.full;
   }
   if (r.alive) {
     for (int a = 0; a < 3; ++a) {
@@ -1293,9 +1289,8 @@ int natray_sim_water_stats(natray_sim* s, natray_water_stats* out) {
   } else {
     r.vmax = 0.0f;
   }
-  r.full_cells = full;
   const double dx = s->U.origin[3];
-  r.volume_l = (double)full * dx * dx * dx * 1e3;
+  r.volume_l = (double)r.full_cells * dx * dx * dx * 1e3;
   *out = r;
   return NATRAY_OK;
 }
