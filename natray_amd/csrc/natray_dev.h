@@ -227,7 +227,7 @@ int launch_water_stats(const float* particles, uint32_t n, const float origin[3]
                        uint32_t* counts, uint32_t slots, WaterPart* parts, uint32_t groups, void* stream);
 // Warm start (one scene), before the solve: the network's inputs for at most `cap` tiles (also
 // into the network's BF16 input buffer `net_in`, [cap][4096][8]), then, after the network has
-// run on them (its output `pred`, [cap][4096][16] FP32), the guess and its acceptance. After a
+// run on them (its output `pred`, [cap][4096] FP32), the guess and its acceptance. After a
 // step, launch_ws_samples writes the training samples of its listed tiles.
 int launch_ws_inputs(const Target& t, void* stream, uint32_t cap, void* net_in);
 int launch_ws_guess(const Target& t, void* stream, const float* pred);

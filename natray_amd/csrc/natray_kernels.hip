@@ -3597,8 +3597,8 @@ __global__ __launch_bounds__(256) void k_ws_gather(L l, bf16x8* __restrict__ net
   }
 }
 
-// guess = p_carried + s o on the water cells of the listed tiles (o: channel 0 of `pred`,
-// [slot][voxel][16] FP32).
+// guess = p_carried + s o on the water cells of the listed tiles (o: `pred`, [slot][voxel]
+// FP32).
 template <class L>
 __global__ __launch_bounds__(256) void k_ws_scatter(L l, const float* __restrict__ pred) {
   const View v = view(l);
@@ -3609,7 +3609,7 @@ __global__ __launch_bounds__(256) void k_ws_scatter(L l, const float* __restrict
     const uint32_t slot = (uint32_t)(i >> 12), v = (uint32_t)(i & 4095u);
     const uint32_t cell = tile_voxel_cell(d, d.tile_list[slot], v, nb);
     if (cell == NONE || cfr(d, NATRAY_F_TYPE, cell) != WATER) continue;
-    d.guess[cell] = d.ws_pcar[cell] + d.tile_scale[slot] * pred[i * 16u];
+    d.guess[cell] = d.ws_pcar[cell] + d.tile_scale[slot] * pred[i];
   }
 }
 

@@ -35,17 +35,10 @@ constexpr int TAPS = 27;
 
 __host__ __device__ constexpr int ksteps(int cin) { return (TAPS * cin + 31) / 32; }
 
-// The neighbour of voxel (x, y, z) at tap `tap`, or -1 outside the tile.
-__device__ __forceinline__ int tap_voxel(int x, int y, int z, int tap) {
-  const int dx = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dz = tap % 3 - 1;
-  const int nx = x + dx, ny = y + dy, nz = z + dz;
-  if ((unsigned)nx >= TILE || (unsigned)ny >= TILE || (unsigned)nz >= TILE) return -1;
-  return (nx * TILE + ny) * TILE + nz;
-}
-
 // Y[t][v][n] = act(bias[n] + sum_k X[t][v + off(tap)][c] W[k][n]) for n < 16, with W in the
 // MFMA B layout `wb` (ksteps(CIN) x 4 groups x 16 columns x 8 values, see k_pack). `yf` (FP32,
-// 16 channels) or `yb` (BF16, 16 channels) receives the result.
+// 16 channels), `y1` (FP32, channel 0 alone) or `yb` (BF16, 16 channels) receives the result;
+// with `gate` (BF16, 16 channels), 0 where it is not positive: the ReLU's gradient.
 //
 // A work item is XP = 2 output x-planes of one tile (32 z-rows). Its input slab, planes
 // x0 - 1 .. x0 + 2 with y and z from -1 to 16, is staged in LDS with zeros outside the tile, so
@@ -66,8 +59,9 @@ struct ConvShape {
 
 template <int CIN>
 __global__ __launch_bounds__(256) void k_conv(const __bf16* __restrict__ X, const bf16x8* __restrict__ wb,
-                                              const float* __restrict__ bias, int relu, __bf16* __restrict__ yb,
-                                              float* __restrict__ yf, int tiles, const uint32_t* __restrict__ tiles_dev) {
+                                              const float* __restrict__ bias, int relu, const __bf16* __restrict__ gate,
+                                              __bf16* __restrict__ yb, float* __restrict__ yf, float* __restrict__ y1,
+                                              int tiles, const uint32_t* __restrict__ tiles_dev) {
   using Sh = ConvShape<CIN>;
   constexpr int VS = Sh::VS, KS = Sh::KS, CH = CIN / 8;  // 16-byte chunks of data per staged voxel
   constexpr int PER_THREAD = (SLAB * CH + 255) / 256;
@@ -138,11 +132,23 @@ __global__ __launch_bounds__(256) void k_conv(const __bf16* __restrict__ X, cons
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int rr = r + 4 * h, row = (x0 + rr / TILE) * TILE + rr % TILE;
+        const size_t vox0 = (size_t)t * VOX + (size_t)row * TILE + 4 * g;
+        if (y1) {
+          f32x4 v = acc[h];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            v[i] += bcol;
+            if (relu) v[i] = v[i] > 0.0f ? v[i] : 0.0f;
+          }
+          if (col == 0) *reinterpret_cast<f32x4*>(y1 + vox0) = v;
+          continue;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float v = acc[h][i] + bcol;
           if (relu) v = v > 0.0f ? v : 0.0f;
-          const size_t o = ((size_t)t * VOX + (size_t)row * TILE + 4 * g + i) * 16 + col;
+          const size_t o = (vox0 + i) * 16 + col;
+          if (gate && !((float)gate[o] > 0.0f)) v = 0.0f;
           if (yf) yf[o] = v;
           if (yb) yb[o] = (__bf16)v;
         }
@@ -155,7 +161,21 @@ __global__ __launch_bounds__(256) void k_conv(const __bf16* __restrict__ X, cons
 // input and 16 output channels (zeros where the padding is), BF16. With `flip`, packs the
 // weights of the input-gradient convolution instead: W'[tap][n][c] = W[26 - tap][c][n], whose
 // input channels are the layer's outputs (cin = 16) and outputs its inputs.
-__global__ void k_pack(const float* __restrict__ W, int cin_real, int cout_real, int cin, int flip, bf16x8* __restrict__ wb) {
+struct PackJob {
+  const float* W;
+  int cin_real, cout_real, cin, flip;
+  bf16x8* wb;
+};
+struct PackJobs {
+  PackJob job[7];
+};
+constexpr int PACK_MAX = (ksteps(16) * 64 + 255) / 256;  // workgroups of the largest job
+// One job per gridDim.y.
+__global__ void k_pack(PackJobs jobs) {
+  const PackJob& jb = jobs.job[blockIdx.y];
+  const float* __restrict__ W = jb.W;
+  const int cin_real = jb.cin_real, cout_real = jb.cout_real, cin = jb.cin, flip = jb.flip;
+  bf16x8* __restrict__ wb = jb.wb;
   const int ks = ksteps(cin);
   const int i = blockIdx.x * blockDim.x + threadIdx.x;  // (s, lane)
   if (i >= ks * 64) return;
@@ -187,109 +207,218 @@ __global__ void k_relu_back(const float* __restrict__ dY, const __bf16* __restri
   }
 }
 
-// dW[tap][c][n] += sum over voxels of X[v + off(tap)][c] dZ[v][n] for one tile per workgroup
-// column: rows are 16 consecutive (tap, c) of the layer's K, K of the MFMA runs over voxels.
-// A: lane l holds (tap, c) row l % 16 at voxels 8 (l / 16) + j of the 32-voxel step; B: dZ at
-// the same voxels for column (output channel) l % 16. Partial sums go to dW with atomics.
-__global__ __launch_bounds__(256) void k_conv_wgrad(const __bf16* __restrict__ X, int cin, const __bf16* __restrict__ dZ,
-                                                    float* __restrict__ dW, int cin_real, int cout_real, int tiles) {
-  const int rowblocks = (TAPS * cin + 15) / 16;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int rb = blockIdx.x % rowblocks, t = blockIdx.x / rowblocks;
-  if (t >= tiles) return;
-  const int g = lane >> 4, m = lane & 15;
-  const int k = rb * 16 + m, tap = k / cin, c = k % cin;
-  const __bf16* Xt = X + (size_t)t * VOX * cin;
-  const __bf16* Zt = dZ + (size_t)t * VOX * 16;
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  // The 4096 voxels in 128 steps of 32, split over the 4 waves.
-  for (int s = wave; s < VOX / 32; s += 4) {
-    bf16x8 a, b;
+// Partial sums over voxels of X[v + off(tap)][c] dZ[v][n] (the weights' gradient) and of dZ[v][n]
+// (the bias's), on MFMA with K over voxels: rows are 16 consecutive k = tap CIN + c, columns n.
+// A work item is XP x-planes of a tile, as in k_conv; a workgroup walks items blockIdx.x,
+// + gridDim.x, ... and leaves its sums in part[blockIdx.x][k][n], the bias's behind them, which
+// k_grad_fold adds up in workgroup order.
+//
+// Eight consecutive voxels of a fragment lie along z, so the item's inputs are staged channel by
+// channel with z fastest, once per dz: each fragment is then one aligned 16-byte LDS read. (With
+// every fragment gathered from global memory two bytes at a time and its sums added to the
+// gradient with atomics, a layer took 36 us at 32 tiles, and its bias 16 in a kernel of its own;
+// now 10 together.)
+template <int CIN>
+struct WgradShape {
+  static constexpr int ROWS = (TAPS * CIN + 15) / 16;       // 16-row blocks
+  static constexpr int CS = (XP + 2) * 18 * TILE + 8;       // bf16 per channel and dz (padded: banks)
+  static constexpr int NS = XP * TILE * TILE + 8;           // bf16 per column of dZ
+  static constexpr int PART = TAPS * CIN * 16 + 16;         // floats per workgroup
+  static constexpr int WAVES = 8;
+  static constexpr int PER = (ROWS + 1 + WAVES - 1) / WAVES;  // row blocks per wave, the bias's among them
+};
+template <int CIN>
+__global__ __launch_bounds__(512) void k_conv_wgrad(const __bf16* __restrict__ X, const __bf16* __restrict__ dZ,
+                                                    float* __restrict__ part, int tiles) {
+  using Sh = WgradShape<CIN>;
+  __shared__ __attribute__((aligned(16))) __bf16 xt[3 * CIN * Sh::CS];
+  __shared__ __attribute__((aligned(16))) __bf16 zt[16 * Sh::NS];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+  const int items = tiles * (TILE / XP);
+  f32x4 acc[Sh::PER];
+  int at[Sh::PER];  // the fragment's row in xt at output plane 0, row 0; -1 padding, -2 the bias
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int v = s * 32 + g * 8 + j;
-      const int x = v / 256, y = (v / 16) % 16, z = v % 16;
-      const int nv = tap < TAPS ? tap_voxel(x, y, z, tap) : -1;
-      a[j] = nv >= 0 ? Xt[(size_t)nv * cin + c] : (__bf16)0.0f;
-      b[j] = Zt[(size_t)v * 16 + m];
+  for (int q = 0; q < Sh::PER; ++q) {
+    acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int rb = wave + Sh::WAVES * q, k = rb * 16 + m, tap = k / CIN, c = k % CIN;
+    at[q] = -1;
+    if (rb < Sh::ROWS && tap < TAPS) at[q] = ((tap % 3) * CIN + c) * Sh::CS + ((tap / 9) * 18 + (tap / 3) % 3) * TILE;
+    if (rb == Sh::ROWS) at[q] = -2;
+  }
+  bf16x8 zero, ones;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) zero[j] = (__bf16)0.0f, ones[j] = (__bf16)1.0f;
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    const int t = item / (TILE / XP), x0 = (item % (TILE / XP)) * XP;
+    const __bf16* Xt = X + (size_t)t * VOX * CIN;
+    const __bf16* Zt = dZ + ((size_t)t * VOX + (size_t)x0 * TILE * TILE) * 16;
+    __syncthreads();  // the previous item's reads are done
+    // Planes x0 - 1 .. x0 + XP, rows y = -1 .. 16, voxel z of copy dz = X[z + dz - 1].
+    constexpr int CH = CIN / 8, ROWVOX = (XP + 2) * 18 * TILE;
+    for (int i = threadIdx.x; i < ROWVOX * CH; i += 512) {
+      const int j = i % CH, v = i / CH, z = v % TILE, py = (v / TILE) % 18, px = v / (TILE * 18);
+      const int x = x0 - 1 + px, y = py - 1;
+      bf16x8 val = zero;
+      if ((unsigned)x < TILE && (unsigned)y < TILE)
+        val = *reinterpret_cast<const bf16x8*>(Xt + (size_t)((x * TILE + y) * TILE + z) * CIN + 8 * j);
+      const int row = (px * 18 + py) * TILE;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int c = 8 * j + e;
+        xt[(0 * CIN + c) * Sh::CS + row + (z + 1) % TILE] = z + 1 < TILE ? val[e] : (__bf16)0.0f;
+        xt[(1 * CIN + c) * Sh::CS + row + z] = val[e];
+        xt[(2 * CIN + c) * Sh::CS + row + (z + TILE - 1) % TILE] = z > 0 ? val[e] : (__bf16)0.0f;
+      }
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-  }
-  // acc[i]: row (tap, c) = rb * 16 + 4 g + i, column n = m.
-  const int n = m;
+    for (int i = threadIdx.x; i < XP * TILE * TILE * 2; i += 512) {
+      const int j = i & 1, v = i >> 1;
+      const bf16x8 val = *reinterpret_cast<const bf16x8*>(Zt + (size_t)v * 16 + 8 * j);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int kk = rb * 16 + 4 * g + i, tp = kk / cin, cc = kk % cin;
-    if (tp < TAPS && cc < cin_real && n < cout_real) atomicAdd(&dW[((size_t)tp * cin_real + cc) * cout_real + n], acc[i]);
+      for (int e = 0; e < 8; ++e) zt[(8 * j + e) * Sh::NS + v] = val[e];
+    }
+    __syncthreads();
+    // 32 voxels a step: rows y and y + 1 of output plane xo, group g taking 8 voxels along z.
+    for (int s = 0; s < XP * TILE / 2; ++s) {
+      const int xo = s / (TILE / 2), y = s % (TILE / 2) * 2 + (g >> 1), z0 = (g & 1) * 8;
+      const bf16x8 b = *reinterpret_cast<const bf16x8*>(zt + m * Sh::NS + (xo * TILE + y) * TILE + z0);
+#pragma unroll
+      for (int q = 0; q < Sh::PER; ++q) {
+        if (wave + Sh::WAVES * q > Sh::ROWS) continue;
+        bf16x8 a = at[q] == -2 ? ones : zero;
+        if (at[q] >= 0) a = *reinterpret_cast<const bf16x8*>(xt + at[q] + (xo * 18 + y) * TILE + z0);
+        acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[q], 0, 0, 0);
+      }
+    }
+  }
+  // acc[q][i]: row rb * 16 + 4 g + i, column m.
+  float* out = part + (size_t)blockIdx.x * Sh::PART;
+#pragma unroll
+  for (int q = 0; q < Sh::PER; ++q) {
+    const int rb = wave + Sh::WAVES * q;
+    if (rb < Sh::ROWS) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int k = rb * 16 + 4 * g + i;
+        if (k < TAPS * CIN) out[k * 16 + m] = acc[q][i];
+      }
+    } else if (rb == Sh::ROWS && g == 0) {
+      out[TAPS * CIN * 16 + m] = acc[q][0];
+    }
   }
 }
 
-// db[n] += sum over voxels of dZ[v][n].
-__global__ void k_bgrad(const __bf16* __restrict__ dZ, float* __restrict__ db, int cout_real, size_t voxels) {
-  __shared__ float part[16];
-  if (threadIdx.x < 16) part[threadIdx.x] = 0.0f;
-  __syncthreads();
-  const int n = threadIdx.x & 15;
-  float s = 0.0f;
-  for (size_t v = (size_t)blockIdx.x * (blockDim.x / 16) + threadIdx.x / 16; v < voxels; v += (size_t)gridDim.x * (blockDim.x / 16))
-    s += (float)dZ[v * 16 + n];
-  atomicAdd(&part[n], s);
-  __syncthreads();
-  if (threadIdx.x < cout_real) atomicAdd(&db[threadIdx.x], part[threadIdx.x]);
+// Adds up the workgroups' partial sums of each layer's gradient, and the loss's into loss[0], in
+// a fixed order: a workgroup per 16 outputs, thread t taking partials t / 16, + 16, ...
+struct FoldJob {
+  const float* part;
+  int groups, stride, cin, cin_real, cout_real;
+  float *dW, *db;
+};
+struct FoldJobs {
+  FoldJob job[4];
+  const float* loss_part;
+  int loss_parts;
+  float* loss;
+};
+constexpr int FOLD_BLOCKS = TAPS * 16 + 1;  // rows of outputs of the largest layer
+__global__ __launch_bounds__(256) void k_grad_fold(FoldJobs jobs) {
+  const FoldJob& jb = jobs.job[blockIdx.y];
+  __shared__ float w[4][16];
+  const int lane = threadIdx.x & 63, n = lane & 15;
+  const int k = blockIdx.x, rows = TAPS * jb.cin;  // row `rows` is the bias
+  if (k <= rows) {
+    float s = 0.0f;
+#pragma unroll 4
+    for (int q = threadIdx.x >> 4; q < jb.groups; q += 16) s += jb.part[(size_t)q * jb.stride + k * 16 + n];
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if (lane < 16) w[threadIdx.x >> 6][n] = s;
+    __syncthreads();
+    if (threadIdx.x < 16u && n < jb.cout_real) {
+      s = (w[0][n] + w[1][n]) + (w[2][n] + w[3][n]);
+      const int tap = k / jb.cin, c = k % jb.cin;
+      if (k == rows)
+        jb.db[n] = s;
+      else if (c < jb.cin_real)
+        jb.dW[((size_t)tap * jb.cin_real + c) * jb.cout_real + n] = s;
+    }
+  }
+  if (jobs.loss && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64u) {
+    float s = 0.0f;
+    for (int i = lane; i < jobs.loss_parts; i += 64) s += jobs.loss_part[i];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) jobs.loss[0] = s;
+  }
 }
 
-// Masked mean squared error of channel 0 of `pred` (FP32, 16 channels) against `target`:
-// the loss goes to loss[0] (summed), dPred = 2 (pred - target) mask / count on channel 0.
-__global__ void k_mse(const float* __restrict__ pred, const float* __restrict__ target, const float* __restrict__ mask,
-                      float inv_count, float* __restrict__ dpred, float* __restrict__ loss, size_t voxels) {
+// A workgroup's share of the loss (all 256 threads call it).
+__device__ __forceinline__ void loss_part(float s, float inv_count, float* __restrict__ part) {
+  __shared__ float w[4];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = ((w[0] + w[1]) + (w[2] + w[3])) * inv_count;
+}
+// The gradient g at channel 0 of a voxel's BF16 record, zeros in the others.
+__device__ __forceinline__ void store_dz(__bf16* __restrict__ dz, size_t v, float g) {
+  bf16x8 lo, hi;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) lo[j] = hi[j] = (__bf16)0.0f;
+  lo[0] = (__bf16)g;
+  reinterpret_cast<bf16x8*>(dz)[2 * v] = lo;
+  reinterpret_cast<bf16x8*>(dz)[2 * v + 1] = hi;
+}
+
+// Masked mean squared error of `pred` against `target`: each workgroup's share of the loss to
+// part, and dZ = 2 (pred - target) mask / count on channel 0.
+__global__ __launch_bounds__(256) void k_mse(const float* __restrict__ pred, const float* __restrict__ target,
+                                             const float* __restrict__ mask, float inv_count, __bf16* __restrict__ dz,
+                                             float* __restrict__ part, size_t voxels) {
   float s = 0.0f;
   for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < voxels; v += (size_t)gridDim.x * blockDim.x) {
-    const float e = (pred[v * 16] - target[v]) * mask[v];
+    const float e = (pred[v] - target[v]) * mask[v];
     s += e * e;
-#pragma unroll
-    for (int n = 0; n < 16; ++n) dpred[v * 16 + n] = n == 0 ? 2.0f * e * inv_count : 0.0f;
+    store_dz(dz, v, 2.0f * e * inv_count);
   }
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  if ((threadIdx.x & 63) == 0) atomicAdd(loss, s * inv_count);
+  loss_part(s, inv_count, part);
 }
 
 // The scaled residual of a guess on each tile: e_v = x_v - (A o)_v on water voxels (diag_v > 0),
 // with (A o)_v = diag_v o_v - sum of o_u over the water neighbours u of v inside the tile (bit
 // 2 axis + 1 of nbm for the + side, 2 axis for the - side; axes x, y, z are voxel strides 256,
-// 16, 1); x is input channel 0 (FP32, [voxel][2]) and o channel 0 of `pred`. Writes e and adds
-// the mean of e^2 over the water voxels to loss[0].
-__device__ __forceinline__ float tile_stencil(const float* __restrict__ f, int fstride, size_t v, uint32_t bits) {
+// 16, 1); x is input channel 0 (FP32, [voxel][2]) and o is `pred`. Writes e, and each workgroup's
+// share of the mean of e^2 over the water voxels to part. (Every wave adding its share to one word
+// took 29 us at 32 tiles; now 5.)
+__device__ __forceinline__ float tile_stencil(const float* __restrict__ f, size_t v, uint32_t bits) {
   const int z = (int)(v & 15), y = (int)((v >> 4) & 15), x = (int)((v >> 8) & 15);
   float s = 0.0f;
-  if ((bits & 1u) && x > 0) s += f[(v - 256) * fstride];
-  if ((bits & 2u) && x < 15) s += f[(v + 256) * fstride];
-  if ((bits & 4u) && y > 0) s += f[(v - 16) * fstride];
-  if ((bits & 8u) && y < 15) s += f[(v + 16) * fstride];
-  if ((bits & 16u) && z > 0) s += f[(v - 1) * fstride];
-  if ((bits & 32u) && z < 15) s += f[(v + 1) * fstride];
+  if ((bits & 1u) && x > 0) s += f[v - 256];
+  if ((bits & 2u) && x < 15) s += f[v + 256];
+  if ((bits & 4u) && y > 0) s += f[v - 16];
+  if ((bits & 8u) && y < 15) s += f[v + 16];
+  if ((bits & 16u) && z > 0) s += f[v - 1];
+  if ((bits & 32u) && z < 15) s += f[v + 1];
   return s;
 }
-__global__ void k_res_e(const float* __restrict__ pred, const float* __restrict__ x, const float* __restrict__ diag,
-                        const uint32_t* __restrict__ nbm, float inv_count, float* __restrict__ e, float* __restrict__ loss,
-                        size_t voxels) {
+__global__ __launch_bounds__(256) void k_res_e(const float* __restrict__ pred, const float* __restrict__ x,
+                                               const float* __restrict__ diag, const uint32_t* __restrict__ nbm,
+                                               float inv_count, float* __restrict__ e, float* __restrict__ part, size_t voxels) {
   float s = 0.0f;
   for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < voxels; v += (size_t)gridDim.x * blockDim.x) {
     float ev = 0.0f;
-    if (diag[v] > 0.0f) ev = x[v * 2] - (diag[v] * pred[v * 16] - tile_stencil(pred, 16, v, nbm[v]));
+    if (diag[v] > 0.0f) ev = x[v * 2] - (diag[v] * pred[v] - tile_stencil(pred, v, nbm[v]));
     e[v] = ev;
     s += ev * ev;
   }
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  if ((threadIdx.x & 63) == 0) atomicAdd(loss, s * inv_count);
+  loss_part(s, inv_count, part);
 }
-// d loss / d o = -2 A e / count on water voxels (A is symmetric), on channel 0 of dpred.
+// d loss / d o = -2 A e / count on water voxels (A is symmetric), as dZ's channel 0.
 __global__ void k_res_grad(const float* __restrict__ e, const float* __restrict__ diag, const uint32_t* __restrict__ nbm,
-                           float inv_count, float* __restrict__ dpred, size_t voxels) {
+                           float inv_count, __bf16* __restrict__ dz, size_t voxels) {
   for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < voxels; v += (size_t)gridDim.x * blockDim.x) {
     float g = 0.0f;
-    if (diag[v] > 0.0f) g = -2.0f * inv_count * (diag[v] * e[v] - tile_stencil(e, 1, v, nbm[v]));
-#pragma unroll
-    for (int n = 0; n < 16; ++n) dpred[v * 16 + n] = n == 0 ? g : 0.0f;
+    if (diag[v] > 0.0f) g = -2.0f * inv_count * (diag[v] * e[v] - tile_stencil(e, v, nbm[v]));
+    store_dz(dz, v, g);
   }
 }
 
@@ -314,6 +443,18 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
 namespace natray {
 namespace net {
 
+// FP32 [voxels][2] -> BF16 [voxels][8], zero padded, 16 bytes a store.
+__global__ __launch_bounds__(256) void k_input(const float2* __restrict__ src, bf16x8* __restrict__ dst, size_t voxels) {
+  for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < voxels; v += (size_t)gridDim.x * blockDim.x) {
+    const float2 s = src[v];
+    bf16x8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = (__bf16)0.0f;
+    o[0] = (__bf16)s.x;
+    o[1] = (__bf16)s.y;
+    dst[v] = o;
+  }
+}
 // FP32 [voxels][cin_real] -> BF16 [voxels][cin] with zero padding.
 __global__ void k_to_bf16(const float* __restrict__ src, int cin_real, int cin, __bf16* __restrict__ dst, size_t voxels) {
   for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < voxels; v += (size_t)gridDim.x * blockDim.x)
@@ -359,9 +500,11 @@ struct natray_net {
   bf16x8* wt[4] = {};     // packed input-gradient weights (layers 2..4)
   __bf16* in = nullptr;   // [T][4096][8]
   __bf16* act[3] = {};    // [T][4096][16] outputs of layers 1..3
-  float* out = nullptr;   // [T][4096][16] output of layer 4
-  float* dy = nullptr;    // [T][4096][16] gradient w.r.t. a layer's output
-  __bf16* dz = nullptr;   // [T][4096][16] the same through the ReLU, BF16
+  float* out = nullptr;   // [T][4096] output of layer 4
+  __bf16* dz[2] = {};     // [T][4096][16] gradient w.r.t. a layer's output through the ReLU, BF16:
+                          // a layer's and the one below's
+  float* part = nullptr;  // the workgroups' partial gradients, layer by layer (part_off)
+  float* lpart = nullptr; // LOSS_PARTS: the workgroups' shares of the loss
   float* target = nullptr;
   float* mask = nullptr;
   float* resid = nullptr;  // [T][4096] residual of the residual loss
@@ -398,20 +541,23 @@ int nalloc(natray_net* n, T** ptr, size_t count) {
   return NATRAY_OK;
 }
 
+// Workgroups of k_conv_wgrad (its LDS leaves one per CU), and of the loss kernels.
+constexpr uint32_t WGRAD_GROUPS = 256, LOSS_PARTS = 512;
+constexpr size_t part_size(int cin) {
+  return (size_t)WGRAD_GROUPS * (cin == 8 ? WgradShape<8>::PART : WgradShape<16>::PART);
+}
+constexpr size_t part_off(int l) { return l == 0 ? 0 : part_size(8) + (size_t)(l - 1) * part_size(16); }
 unsigned grid_for(size_t items) { return (unsigned)std::min<size_t>((items + 255) / 256, 4096); }
 
 int pack(natray_net* n) {
+  PackJobs jobs{};
+  int k = 0;
   for (int l = 0; l < 4; ++l) {
     const Layer& L = LAYERS[l];
-    const int cnt = ksteps(L.cin) * 64;
-    hipLaunchKernelGGL(k_pack, dim3((cnt + 255) / 256), dim3(256), 0, n->stream, n->p + L.w_off, L.cin_real, L.cout_real,
-                       L.cin, 0, n->wb[l]);
-    if (l > 0) {
-      const int cntt = ksteps(16) * 64;
-      hipLaunchKernelGGL(k_pack, dim3((cntt + 255) / 256), dim3(256), 0, n->stream, n->p + L.w_off, L.cin_real, L.cout_real,
-                         16, 1, n->wt[l]);
-    }
+    jobs.job[k++] = PackJob{n->p + L.w_off, L.cin_real, L.cout_real, L.cin, 0, n->wb[l]};
+    if (l > 0) jobs.job[k++] = PackJob{n->p + L.w_off, L.cin_real, L.cout_real, 16, 1, n->wt[l]};
   }
+  hipLaunchKernelGGL(k_pack, dim3(PACK_MAX, k), dim3(256), 0, n->stream, jobs);
   NCHK(hipGetLastError());
   n->packed = true;
   return NATRAY_OK;
@@ -420,12 +566,22 @@ int pack(natray_net* n) {
 // A convolution over `tiles` tiles: one workgroup per work item (2 x-planes), up to 2 per CU
 // (the LDS slab of a 16-channel input takes 62 KB).
 void launch_conv(int cin, uint32_t tiles, hipStream_t stream, const __bf16* X, const bf16x8* wb, const float* bias, int relu,
-                 __bf16* yb, float* yf, const uint32_t* tiles_dev) {
+                 const __bf16* gate, __bf16* yb, float* yf, float* y1, const uint32_t* tiles_dev) {
   const unsigned grid = (unsigned)std::min<uint32_t>(tiles * (TILE / XP), 512u);
   if (cin == 8)
-    hipLaunchKernelGGL(k_conv<8>, dim3(grid), dim3(256), 0, stream, X, wb, bias, relu, yb, yf, (int)tiles, tiles_dev);
+    hipLaunchKernelGGL(k_conv<8>, dim3(grid), dim3(256), 0, stream, X, wb, bias, relu, gate, yb, yf, y1, (int)tiles, tiles_dev);
   else
-    hipLaunchKernelGGL(k_conv<16>, dim3(grid), dim3(256), 0, stream, X, wb, bias, relu, yb, yf, (int)tiles, tiles_dev);
+    hipLaunchKernelGGL(k_conv<16>, dim3(grid), dim3(256), 0, stream, X, wb, bias, relu, gate, yb, yf, y1, (int)tiles, tiles_dev);
+}
+
+// The weights' and bias's partial gradients of a layer; returns the workgroups that left one.
+uint32_t launch_wgrad(int cin, uint32_t tiles, hipStream_t stream, const __bf16* X, const __bf16* dz, float* part) {
+  const uint32_t groups = std::min<uint32_t>(tiles * (TILE / XP), WGRAD_GROUPS);
+  if (cin == 8)
+    hipLaunchKernelGGL(k_conv_wgrad<8>, dim3(groups), dim3(512), 0, stream, X, dz, part, (int)tiles);
+  else
+    hipLaunchKernelGGL(k_conv_wgrad<16>, dim3(groups), dim3(512), 0, stream, X, dz, part, (int)tiles);
+  return groups;
 }
 
 int forward(natray_net* n, uint32_t tiles, const uint32_t* tiles_dev = nullptr) {
@@ -436,7 +592,7 @@ int forward(natray_net* n, uint32_t tiles, const uint32_t* tiles_dev = nullptr) 
   const __bf16* x = n->in;
   for (int l = 0; l < 4; ++l) {
     const Layer& L = LAYERS[l];
-    launch_conv(L.cin, tiles, n->stream, x, n->wb[l], n->p + L.b_off, L.relu, l < 3 ? n->act[l] : nullptr,
+    launch_conv(L.cin, tiles, n->stream, x, n->wb[l], n->p + L.b_off, L.relu, nullptr, l < 3 ? n->act[l] : nullptr, nullptr,
                 l == 3 ? n->out : nullptr, tiles_dev);
     if (l < 3) x = n->act[l];
   }
@@ -449,31 +605,35 @@ int forward(natray_net* n, uint32_t tiles, const uint32_t* tiles_dev = nullptr) 
 // (neighbour bits). The parameters' gradients go to n->g.
 int backward(natray_net* n, uint32_t tiles, float inv_count, bool residual = false) {
   const size_t vox = (size_t)tiles * VOX;
-  NCHK(hipMemsetAsync(n->g, 0, NATRAY_NET_PARAMS * sizeof(float), n->stream));
-  NCHK(hipMemsetAsync(n->loss, 0, sizeof(float), n->stream));
+  const unsigned lgrid = std::min(grid_for(vox), (unsigned)LOSS_PARTS);
+  __bf16* dz = n->dz[0];
   if (!residual) {
-    hipLaunchKernelGGL(k_mse, dim3(grid_for(vox)), dim3(256), 0, n->stream, n->out, n->target, n->mask, inv_count, n->dy,
-                       n->loss, vox);
+    hipLaunchKernelGGL(k_mse, dim3(lgrid), dim3(256), 0, n->stream, n->out, n->target, n->mask, inv_count, dz, n->lpart, vox);
   } else {
     const uint32_t* bits = reinterpret_cast<const uint32_t*>(n->mask);
-    hipLaunchKernelGGL(k_res_e, dim3(grid_for(vox)), dim3(256), 0, n->stream, n->out, n->stage, n->target, bits, inv_count,
-                       n->resid, n->loss, vox);
-    hipLaunchKernelGGL(k_res_grad, dim3(grid_for(vox)), dim3(256), 0, n->stream, n->resid, n->target, bits, inv_count, n->dy,
+    hipLaunchKernelGGL(k_res_e, dim3(lgrid), dim3(256), 0, n->stream, n->out, n->stage, n->target, bits, inv_count,
+                       n->resid, n->lpart, vox);
+    hipLaunchKernelGGL(k_res_grad, dim3(grid_for(vox)), dim3(256), 0, n->stream, n->resid, n->target, bits, inv_count, dz,
                        vox);
   }
+  FoldJobs jobs{};
   for (int l = 3; l >= 0; --l) {
     const Layer& L = LAYERS[l];
-    const __bf16* y = l < 3 ? n->act[l] : nullptr;
-    hipLaunchKernelGGL(k_relu_back, dim3(grid_for(vox * 16)), dim3(256), 0, n->stream, n->dy, y, L.relu, n->dz, vox * 16);
-    const __bf16* xin = l > 0 ? n->act[l - 1] : n->in;
-    const int rowblocks = (TAPS * L.cin + 15) / 16;
-    hipLaunchKernelGGL(k_conv_wgrad, dim3(rowblocks * tiles), dim3(256), 0, n->stream, xin, L.cin, n->dz, n->g + L.w_off,
-                       L.cin_real, L.cout_real, (int)tiles);
-    hipLaunchKernelGGL(k_bgrad, dim3((unsigned)std::min<size_t>((vox + 15) / 16, 1024)), dim3(256), 0, n->stream, n->dz,
-                       n->g + L.b_off, L.cout_real, vox);
-    if (l > 0)
-      launch_conv(16, tiles, n->stream, n->dz, n->wt[l], nullptr, 0, nullptr, n->dy, nullptr);
+    float* part = n->part + part_off(l);
+    const uint32_t groups = launch_wgrad(L.cin, tiles, n->stream, l > 0 ? n->act[l - 1] : n->in, dz, part);
+    jobs.job[l] = FoldJob{part, (int)groups, L.cin == 8 ? WgradShape<8>::PART : WgradShape<16>::PART, L.cin, L.cin_real,
+                          L.cout_real, n->g + L.w_off, n->g + L.b_off};
+    if (l > 0) {
+      // The input's gradient through the ReLU of the layer below.
+      __bf16* below = dz == n->dz[0] ? n->dz[1] : n->dz[0];
+      launch_conv(16, tiles, n->stream, dz, n->wt[l], nullptr, 0, n->act[l - 1], below, nullptr, nullptr, nullptr);
+      dz = below;
+    }
   }
+  jobs.loss_part = n->lpart;
+  jobs.loss_parts = (int)lgrid;
+  jobs.loss = n->loss;
+  hipLaunchKernelGGL(k_grad_fold, dim3(FOLD_BLOCKS, 4), dim3(256), 0, n->stream, jobs);
   NCHK(hipGetLastError());
   return NATRAY_OK;
 }
@@ -481,7 +641,8 @@ int backward(natray_net* n, uint32_t tiles, float inv_count, bool residual = fal
 int upload_input(natray_net* n, const float* input, uint32_t tiles) {
   const size_t vox = (size_t)tiles * VOX;
   NCHK(hipMemcpyAsync(n->stage, input, vox * 2 * 4, hipMemcpyHostToDevice, n->stream));
-  hipLaunchKernelGGL(k_to_bf16, dim3(grid_for(vox)), dim3(256), 0, n->stream, n->stage, 2, 8, n->in, vox);
+  hipLaunchKernelGGL(k_input, dim3(grid_for(vox)), dim3(256), 0, n->stream, reinterpret_cast<const float2*>(n->stage),
+                     reinterpret_cast<bf16x8*>(n->in), vox);
   NCHK(hipGetLastError());
   return NATRAY_OK;
 }
@@ -523,8 +684,8 @@ int natray_net_create(uint32_t max_tiles, uint64_t seed, natray_net** out) {
   if ((e = nalloc(n, &n->p, NATRAY_NET_PARAMS)) || (e = nalloc(n, &n->g, NATRAY_NET_PARAMS)) ||
       (e = nalloc(n, &n->m, NATRAY_NET_PARAMS)) || (e = nalloc(n, &n->v, NATRAY_NET_PARAMS)) ||
       (e = nalloc(n, &n->in, vox * 8)) || (e = nalloc(n, &n->act[0], vox * 16)) || (e = nalloc(n, &n->act[1], vox * 16)) ||
-      (e = nalloc(n, &n->act[2], vox * 16)) || (e = nalloc(n, &n->out, vox * 16)) || (e = nalloc(n, &n->dy, vox * 16)) ||
-      (e = nalloc(n, &n->dz, vox * 16)) || (e = nalloc(n, &n->target, vox)) || (e = nalloc(n, &n->mask, vox)) ||
+      (e = nalloc(n, &n->act[2], vox * 16)) || (e = nalloc(n, &n->out, vox)) || (e = nalloc(n, &n->dz[0], vox * 16)) ||
+      (e = nalloc(n, &n->dz[1], vox * 16)) || (e = nalloc(n, &n->part, part_off(4))) || (e = nalloc(n, &n->lpart, LOSS_PARTS)) || (e = nalloc(n, &n->target, vox)) || (e = nalloc(n, &n->mask, vox)) ||
       (e = nalloc(n, &n->stage, vox * 2)) || (e = nalloc(n, &n->loss, 1)) || (e = nalloc(n, &n->resid, vox)))
     return bail(e);
   for (int l = 0; l < 4; ++l) {
@@ -592,8 +753,7 @@ int natray_net_forward(natray_net* n, const float* input, uint32_t tiles, float*
   if (e) return e;
   if ((e = forward(n, tiles))) return e;
   const size_t vox = (size_t)tiles * VOX;
-  hipLaunchKernelGGL(k_take, dim3(grid_for(vox)), dim3(256), 0, n->stream, n->out, 1, n->stage, vox);
-  NCHK(hipMemcpyAsync(output, n->stage, vox * 4, hipMemcpyDeviceToHost, n->stream));
+  NCHK(hipMemcpyAsync(output, n->out, vox * 4, hipMemcpyDeviceToHost, n->stream));
   NCHK(hipStreamSynchronize(n->stream));
   return NATRAY_OK;
 }
@@ -603,13 +763,14 @@ int natray_net_train_step(natray_net* n, const float* input, const float* target
   if (!n || !input || !target || !mask) return nfail(NATRAY_E_ARG, "null argument");
   if (tiles == 0 || tiles > n->max_tiles) return nfail(NATRAY_E_ARG, "tiles must be 1..max_tiles");
   const size_t vox = (size_t)tiles * VOX;
-  double count = 0.0;
-  for (size_t i = 0; i < vox; ++i) count += mask[i];
   int e = upload_input(n, input, tiles);
   if (e) return e;
   NCHK(hipMemcpyAsync(n->target, target, vox * 4, hipMemcpyHostToDevice, n->stream));
   NCHK(hipMemcpyAsync(n->mask, mask, vox * 4, hipMemcpyHostToDevice, n->stream));
   if ((e = forward(n, tiles))) return e;
+  // The GPU runs the forward pass meanwhile.
+  double count = 0.0;
+  for (size_t i = 0; i < vox; ++i) count += mask[i];
   if ((e = backward(n, tiles, count > 0.0 ? (float)(1.0 / count) : 0.0f))) return e;
   if (lr > 0.0f) {
     n->steps += 1;
@@ -632,14 +793,15 @@ int natray_net_train_step_residual(natray_net* n, const float* input, const floa
   if (!n || !input || !diag || !nbm) return nfail(NATRAY_E_ARG, "null argument");
   if (tiles == 0 || tiles > n->max_tiles) return nfail(NATRAY_E_ARG, "tiles must be 1..max_tiles");
   const size_t vox = (size_t)tiles * VOX;
-  double count = 0.0;
-  for (size_t i = 0; i < vox; ++i) count += diag[i] > 0.0f ? 1.0 : 0.0;
   int e = upload_input(n, input, tiles);
   if (e) return e;
   NCHK(hipMemcpyAsync(n->target, diag, vox * 4, hipMemcpyHostToDevice, n->stream));
   NCHK(hipMemcpyAsync(n->mask, nbm, vox * 4, hipMemcpyHostToDevice, n->stream));
   if ((e = forward(n, tiles))) return e;
-  if ((e = backward(n, tiles, count > 0.0 ? (float)(1.0 / count) : 0.0f, true))) return e;
+  // The GPU runs the forward pass meanwhile.
+  size_t count = 0;
+  for (size_t i = 0; i < vox; ++i) count += diag[i] > 0.0f ? 1u : 0u;
+  if ((e = backward(n, tiles, count ? (float)(1.0 / (double)count) : 0.0f, true))) return e;
   if (lr > 0.0f) {
     n->steps += 1;
     const float b1 = 0.9f, b2 = 0.999f;
@@ -688,7 +850,8 @@ int natray_net_layer_check(uint32_t cin_real, uint32_t cout_real, int relu, cons
   float* dxf = (float*)al(vox * 16 * 4);
   bf16x8* wb = (bf16x8*)al((size_t)ksteps(cin) * 64 * 16);
   bf16x8* wt = (bf16x8*)al((size_t)ksteps(16) * 64 * 16);
-  if (a.size() != 13) return done(nfail(NATRAY_E_NOMEM, "hipMalloc"));
+  float* part = (float*)al(part_size(cin) * 4);
+  if (a.size() != 14) return done(nfail(NATRAY_E_NOMEM, "hipMalloc"));
   const unsigned grid = grid_for(vox);
   std::vector<float> bb(16, 0.0f);
   for (uint32_t i = 0; i < cout_real; ++i) bb[i] = b[i];
@@ -696,22 +859,23 @@ int natray_net_layer_check(uint32_t cin_real, uint32_t cout_real, int relu, cons
       hipMemcpy(stage, X, vox * cin_real * 4, hipMemcpyHostToDevice))
     return done(nfail(NATRAY_E_HIP, "upload"));
   hipLaunchKernelGGL(k_to_bf16, dim3(grid), dim3(256), 0, 0, stage, (int)cin_real, cin, xb, vox);
-  const int cnt = ksteps(cin) * 64, cntt = ksteps(16) * 64;
-  hipLaunchKernelGGL(k_pack, dim3((cnt + 255) / 256), dim3(256), 0, 0, dWd, (int)cin_real, (int)cout_real, cin, 0, wb);
-  hipLaunchKernelGGL(k_pack, dim3((cntt + 255) / 256), dim3(256), 0, 0, dWd, (int)cin_real, (int)cout_real, 16, 1, wt);
-  launch_conv(cin, tiles, 0, xb, wb, bd, relu, yb, yf, nullptr);
+  PackJobs pj{};
+  pj.job[0] = PackJob{dWd, (int)cin_real, (int)cout_real, cin, 0, wb};
+  pj.job[1] = PackJob{dWd, (int)cin_real, (int)cout_real, 16, 1, wt};
+  hipLaunchKernelGGL(k_pack, dim3(PACK_MAX, 2), dim3(256), 0, 0, pj);
+  launch_conv(cin, tiles, 0, xb, wb, bd, relu, nullptr, yb, yf, nullptr, nullptr);
   hipLaunchKernelGGL(k_take, dim3(grid), dim3(256), 0, 0, yf, (int)cout_real, stage, vox);
   if (hipMemcpy(Y, stage, vox * cout_real * 4, hipMemcpyDeviceToHost)) return done(nfail(NATRAY_E_HIP, "download Y"));
   // Backward from dY.
   if (hipMemcpy(stage, dY, vox * cout_real * 4, hipMemcpyHostToDevice)) return done(nfail(NATRAY_E_HIP, "upload dY"));
   hipLaunchKernelGGL(k_pad16, dim3(grid), dim3(256), 0, 0, stage, (int)cout_real, g, vox);
   hipLaunchKernelGGL(k_relu_back, dim3(grid_for(vox * 16)), dim3(256), 0, 0, g, yb, relu, dz, vox * 16);
-  if (hipMemset(dWd, 0, nw * 4) || hipMemset(dbd, 0, 64)) return done(nfail(NATRAY_E_HIP, "memset"));
-  hipLaunchKernelGGL(k_conv_wgrad, dim3(((TAPS * cin + 15) / 16) * tiles), dim3(256), 0, 0, xb, cin, dz, dWd, (int)cin_real,
-                     (int)cout_real, (int)tiles);
-  hipLaunchKernelGGL(k_bgrad, dim3((unsigned)std::min<size_t>((vox + 15) / 16, 1024)), dim3(256), 0, 0, dz, dbd,
-                     (int)cout_real, vox);
-  launch_conv(16, tiles, 0, dz, wt, nullptr, 0, nullptr, dxf, nullptr);
+  const uint32_t groups = launch_wgrad(cin, tiles, 0, xb, dz, part);
+  FoldJobs fj{};
+  fj.job[0] = FoldJob{part, (int)groups, cin == 8 ? WgradShape<8>::PART : WgradShape<16>::PART, cin, (int)cin_real,
+                      (int)cout_real, dWd, dbd};
+  hipLaunchKernelGGL(k_grad_fold, dim3(FOLD_BLOCKS, 1), dim3(256), 0, 0, fj);
+  launch_conv(16, tiles, 0, dz, wt, nullptr, 0, nullptr, nullptr, dxf, nullptr, nullptr);
   hipLaunchKernelGGL(k_take, dim3(grid), dim3(256), 0, 0, dxf, (int)cin_real, dXf, vox);
   if (hipGetLastError() != hipSuccess) return done(nfail(NATRAY_E_HIP, "layer kernels"));
   if (hipMemcpy(dX, dXf, vox * cin_real * 4, hipMemcpyDeviceToHost) || hipMemcpy(dW, dWd, nw * 4, hipMemcpyDeviceToHost) ||
