@@ -109,6 +109,72 @@ __device__ __forceinline__ uint32_t nbr(const uint32_t* lk, int lx, int ly, int 
   return b * 64u + (uint32_t)(qx - nx * 4) * 16u + (uint32_t)(qy - ny * 4) * 4u + (uint32_t)(qz - nz * 4);
 }
 
+// Correctly rounded s / d by a divisor known in advance, from y = RN(1 / d): one multiplication
+// and two fused multiply-adds (Brisebarre, Muller and Raina, "Accelerating correctly rounded
+// floating-point division when the divisor is known in advance", IEEE Trans. Computers 53,
+// 2004), against the eleven dependent instructions of a general IEEE division. The residual is
+// formed as q0 d - s, so that a zero keeps the sign s / d has. The result is RN(s / d) while
+// nothing under- or overflows: DivGuard tells when that may have happened, and the caller then
+// divides in full. (Compared with the division over all 2^23 significands of s for 24,000
+// divisors, the extreme ones among them.)
+__device__ __forceinline__ float div_by(float s, float d, float y) {
+  const float q0 = s * y;
+  const float e = __builtin_fmaf(q0, d, -s);
+  return __builtin_fmaf(-e, y, q0);
+}
+
+// What div_by needs: every nonzero dividend of at least 2^-70, a divisor within 2^+-30, and
+// results below 2^100 (an overflow or a NaN in any sweep reaches a later result). The exponents
+// are compared with the sign shifted out; a zero dividend, which is exact, wraps to the top.
+struct DivGuard {
+  uint32_t lo = 0xffffffffu, hi = 0u;
+  __device__ __forceinline__ void dividend(float s) { lo = min(lo, (__float_as_uint(s) << 1) - 1u); }
+  __device__ __forceinline__ void result(float z) { hi = max(hi, __float_as_uint(z) << 1); }
+  static __device__ __forceinline__ bool divisor(float d) { return d >= 0x1p-30f && d <= 0x1p30f; }
+  __device__ __forceinline__ bool bad() const { return lo < (57u << 24) - 1u || hi >= 227u << 24; }
+};
+
+// Lane 0's value in every lane (all lanes active), in scalar registers.
+__device__ __forceinline__ float first_lane(float x) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(x)));
+}
+__device__ __forceinline__ double first_lane(double x) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The grid's frame for particles, in scalar registers: positions in cells are (p - origin) / h,
+// by div_by where the cell size allows it.
+struct Frame {
+  float o[3], h, y;
+  bool fast;  // h within div_by's divisors
+};
+__device__ __forceinline__ Frame frame_of(const natray_params* U) {
+  Frame f;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) f.o[k] = U->origin[k];
+  f.h = U->origin[3];
+  f.y = first_lane(1.0f / f.h);
+  f.fast = DivGuard::divisor(f.h);
+  return f;
+}
+__device__ __forceinline__ void cells_of(const Frame& f, float px, float py, float pz, float x[3]) {
+  const float s[3] = {px - f.o[0], py - f.o[1], pz - f.o[2]};
+  DivGuard g;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    x[k] = div_by(s[k], f.h, f.y);
+    g.dividend(s[k]);
+    g.result(x[k]);
+  }
+  if (__builtin_expect(!f.fast || g.bad(), 0)) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) x[k] = s[k] / f.h;
+  }
+}
+
 // ---- scene geometry (the reference's ground and knot, plus the synthetic scenes' solids) ------
 
 __device__ __forceinline__ void cell_centre(const Dev& d, int cx, int cy, int cz, float& px, float& py, float& pz) {
@@ -193,12 +259,9 @@ __device__ __forceinline__ float pressure_of(const Dev& d, uint32_t cell) {
   return cfr(d, NATRAY_F_TYPE, cell) == WATER ? fmax_(p, NATRAY_P_FLOOR) : p;
 }
 
-__device__ __forceinline__ uint32_t pack_key(const Dev& d, float px, float py, float pz, bool alive) {
-  if (!alive) return NONE;
-  const natray_params* U = d.U;
-  float h = U->origin[3];
-  int cx = (int)floorf((px - U->origin[0]) / h), cy = (int)floorf((py - U->origin[1]) / h),
-      cz = (int)floorf((pz - U->origin[2]) / h);
+// The key of the cell at x (in cells), or NONE outside the domain.
+__device__ __forceinline__ uint32_t key_of(const natray_params* U, const float x[3]) {
+  const int cx = (int)floorf(x[0]), cy = (int)floorf(x[1]), cz = (int)floorf(x[2]);
   if (cx < 0 || cy < 0 || cz < 0 || cx >= (int)U->dims[0] || cy >= (int)U->dims[1] || cz >= (int)U->dims[2]) return NONE;
   return (uint32_t)cx | ((uint32_t)cy << KEY_BITS) | ((uint32_t)cz << (2 * KEY_BITS));
 }
@@ -376,7 +439,9 @@ __global__ void k_keys(L l) {
   if (i >= d.N) return;
   const float4* p = reinterpret_cast<const float4*>(d.P) + (size_t)i * 5;
   float4 pos = p[0], vel = p[1];
-  d.key[i] = pack_key(d, pos.x, pos.y, pos.z, !(vel.w < 0.5f));
+  float x[3];
+  cells_of(frame_of(d.U), pos.x, pos.y, pos.z, x);
+  d.key[i] = vel.w < 0.5f ? NONE : key_of(d.U, x);
 }
 
 // ---- binning (shaders/fluid.wgsl:91-196) ---------------------------------------------------------
@@ -758,12 +823,13 @@ __device__ __forceinline__ void block_links(const Dev& d, uint32_t b, uint32_t l
 // particle that is not in that cell, which only a position written behind the library's back
 // can cause.
 template <bool PACK>
-__device__ __forceinline__ bool splat_particle(const Dev& d, int* tile, uint32_t i, uint32_t l, int bx, int by, int bz,
-                                               const int corner[3], float h) {
-  const natray_params* U = d.U;
+__device__ __forceinline__ bool splat_particle(const Dev& d, const Frame& f, int* tile, uint32_t i, uint32_t l, int bx, int by,
+                                               int bz, const int corner[3]) {
+  const float h = f.h;
   const float4* p = reinterpret_cast<const float4*>(d.P) + (size_t)i * 5;
   const float4 pos = p[0], vel = p[1], c0 = p[2], c1 = p[3], c2 = p[4];
-  const float x[3] = {(pos.x - U->origin[0]) / h, (pos.y - U->origin[1]) / h, (pos.z - U->origin[2]) / h};
+  float x[3];
+  cells_of(f, pos.x, pos.y, pos.z, x);
   const int ox = (int)floorf(x[0]) - bx * 4, oy = (int)floorf(x[1]) - by * 4, oz = (int)floorf(x[2]) - bz * 4;
   if ((uint32_t)ox * 16u + (uint32_t)oy * 4u + (uint32_t)oz != l || (unsigned)ox > 3u || (unsigned)oy > 3u ||
       (unsigned)oz > 3u)
@@ -810,7 +876,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
   __shared__ uint32_t s_maxc;
   const uint32_t n = n_blocks(d), tid = threadIdx.x;
   const natray_params* U = d.U;
-  const float h = U->origin[3];
+  const Frame f = frame_of(U);
   Dealer deal_s;
   __shared__ uint32_t deal_w[2];
   for (uint32_t b = deal_first(d, DEAL_P2G, n, v.wg, v.wgs, deal_s, deal_w); b < n; b = deal_next(deal_w)) {
@@ -884,12 +950,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
         if (count <= P2G_PACK_MAX) {
           for (uint32_t k = tid; k < placed; k += 256) {
             const uint32_t l = ocell[k];
-            if (!splat_particle<true>(d, tile, order[k], l, bx, by, bz, corner, h)) atomicAdd(&drop[l], 1u);
+            if (!splat_particle<true>(d, f, tile, order[k], l, bx, by, bz, corner)) atomicAdd(&drop[l], 1u);
           }
         } else {
           for (uint32_t k = tid; k < placed; k += 256) {
             const uint32_t l = ocell[k];
-            if (!splat_particle<false>(d, tile, order[k], l, bx, by, bz, corner, h)) atomicAdd(&drop[l], 1u);
+            if (!splat_particle<false>(d, f, tile, order[k], l, bx, by, bz, corner)) atomicAdd(&drop[l], 1u);
           }
         }
       } else {
@@ -897,14 +963,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
         for (uint32_t k = tid; k < count; k += 256) {
           const uint32_t i = d.sorted[first + k];
           const uint32_t l = key_local(d.key[i], bx, by, bz);
-          if (l < 64u && !splat_particle<false>(d, tile, i, l, bx, by, bz, corner, h)) atomicAdd(&drop[l], 1u);
+          if (l < 64u && !splat_particle<false>(d, f, tile, i, l, bx, by, bz, corner)) atomicAdd(&drop[l], 1u);
         }
       }
     } else {
       for (uint32_t k = tid; k < count; k += 256) {
         const uint32_t i = d.sorted[first + k];
         const uint32_t l = key_local(d.key[i], bx, by, bz);
-        if (l < 64u && splat_particle<false>(d, tile, i, l, bx, by, bz, corner, h)) atomicAdd(&cnt[l], 1u);
+        if (l < 64u && splat_particle<false>(d, f, tile, i, l, bx, by, bz, corner)) atomicAdd(&cnt[l], 1u);
       }
     }
     __syncthreads();
@@ -917,9 +983,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
 #pragma unroll
         for (uint32_t j = 0; j < 2u; ++j) {
           // j = 0: the weight (A_WT(lat), or A_WC); j = 1: the momentum (A_MOM(lat)), or A_PC.
-          const uint32_t f = lat < 3u ? 2u * lat + 1u - j : NATRAY_A_WC + j;
+          const uint32_t fl = lat < 3u ? 2u * lat + 1u - j : NATRAY_A_WC + j;
           const int v = tile[2u * (lat * P2G_TILE + pt) + j];
-          if (v != 0) atomicAdd(&accr(d, f, cell), v);
+          if (v != 0) atomicAdd(&accr(d, fl, cell), v);
         }
     }
     if (tid < 64) accr(d, NATRAY_A_N, b * 64u + tid) = (int32_t)(cnt[tid] - drop[tid]);
@@ -1263,17 +1329,6 @@ __device__ __forceinline__ R chunk_tree(const Dev& d, const SolveSpan& sp, const
   if (W == 256u) return lane_tree_from<R>((slot(ln) + slot(ln + 128u)) + (slot(ln + 64u) + slot(ln + 192u)), 32u);
   if (W == 128u) return lane_tree_from<R>(slot(ln) + slot(ln + 64u), 32u);
   return lane_tree_from<R>(slot(ln), W / 2u);
-}
-
-// Lane 0's value in every lane (all lanes active).
-__device__ __forceinline__ float first_lane(float x) {
-  return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(x)));
-}
-__device__ __forceinline__ double first_lane(double x) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(x);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
 // A reduction's LDS: the chunk sums, and the abort flag per tag parity (a wave can leave once it
@@ -2114,31 +2169,6 @@ __device__ __forceinline__ R quad_tree(const R* v) {
 // of the row by one brings to the lanes that need them; zm, zp for every lane.
 struct QuadHalo {
   float x[4], y[4], zm, zp;
-};
-
-// Correctly rounded s / d by a divisor known in advance, from y = RN(1 / d): one multiplication
-// and two fused multiply-adds (Brisebarre, Muller and Raina, "Accelerating correctly rounded
-// floating-point division when the divisor is known in advance", IEEE Trans. Computers 53,
-// 2004), against the eleven dependent instructions of a general IEEE division. The residual is
-// formed as q0 d - s, so that a zero keeps the sign s / d has. The result is RN(s / d) while
-// nothing under- or overflows: DivGuard tells when that may have happened, and the caller then
-// divides in full. (Compared with the division over all 2^23 significands of s for 24,000
-// divisors, the extreme ones among them.)
-__device__ __forceinline__ float div_by(float s, float d, float y) {
-  const float q0 = s * y;
-  const float e = __builtin_fmaf(q0, d, -s);
-  return __builtin_fmaf(-e, y, q0);
-}
-
-// What div_by needs: every nonzero dividend of at least 2^-70, a divisor within 2^+-30, and
-// results below 2^100 (an overflow or a NaN in any sweep reaches a later result). The exponents
-// are compared with the sign shifted out; a zero dividend, which is exact, wraps to the top.
-struct DivGuard {
-  uint32_t lo = 0xffffffffu, hi = 0u;
-  __device__ __forceinline__ void dividend(float s) { lo = min(lo, (__float_as_uint(s) << 1) - 1u); }
-  __device__ __forceinline__ void result(float z) { hi = max(hi, __float_as_uint(z) << 1); }
-  static __device__ __forceinline__ bool divisor(float d) { return d >= 0x1p-30f && d <= 0x1p30f; }
-  __device__ __forceinline__ bool bad() const { return lo < (57u << 24) - 1u || hi >= 227u << 24; }
 };
 
 // The preconditioner (see precondition) of a set of quads: z = M^-1 r, 0 off water. m: bits 0..3
@@ -3867,46 +3897,90 @@ __global__ __launch_bounds__(256) void k_extend2(L l) {
 struct Gathered {
   float s, g0, g1, g2, w;
 };
-
-// gather (fluid.wgsl:780-802)
-template <int OX, int OY, int OZ>
-__device__ __forceinline__ Gathered gather(const float* tg, const float X[3], const int corner[3], uint32_t fa, uint32_t fw,
-                                           float h) {
-  const float o[3] = {0.5f * OX, 0.5f * OY, 0.5f * OZ};
-  int base[3];
-  float fx[3];
+// One axis of a particle's stencil on the lattices with offset 0 or 1/2 there: the first node,
+// the weights, and the nodes' distances k - fx. The four lattices share six of these.
+struct GatherAxis {
+  int base;
+  float w[3], t[3];
+};
+template <int O>
+__device__ __forceinline__ GatherAxis gather_axis(float x) {
+  GatherAxis a;
+  const float o = 0.5f * O;
+  a.base = (int)floorf(x - o - 0.5f);
+  const float fx = x - o - (float)a.base;
+  axis_weights(fx, a.w);
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    base[k] = (int)floorf(X[k] - o[k] - 0.5f);
-    fx[k] = X[k] - o[k] - (float)base[k];
-  }
-  float wx[3], wy[3], wz[3];
-  axis_weights(fx[0], wx);
-  axis_weights(fx[1], wy);
-  axis_weights(fx[2], wz);
-  const int t0 = (base[0] - corner[0]) * 49 + (base[1] - corner[1]) * 7 + (base[2] - corner[2]);
-  const float* ta = tg + fa * TILE + t0;
-  const float* tw = tg + fw * TILE + t0;
+  for (int k = 0; k < 3; ++k) a.t[k] = (float)k - fx;
+  return a;
+}
+
+// gather (fluid.wgsl:780-802) from a lattice's nodes, each its value and its weight side by side
+// (8 bytes a read, two nodes an instruction). Fully unrolled, the weights and distances stay in
+// registers: rolled over the first axis, they were formed again on each turn, a third of the
+// kernel's instructions, which bound it. k_g2p's time for 2M particles in the impact went from 126
+// us to 117, for 15.2M from 868 to 791, for the 64 scenes of a batch from 1109 to 1030; a wave of 64
+// particles now issues 1500 vector instructions, of which the stencils' arithmetic is 1026.
+template <bool GRAD>
+__device__ __forceinline__ Gathered gather(const float2* tg, const GatherAxis& ax, const GatherAxis& ay, const GatherAxis& az,
+                                           const int corner[3], float h) {
+  const float2* tp = tg + (ax.base - corner[0]) * 49 + (ay.base - corner[1]) * 7 + (az.base - corner[2]);
   Gathered r = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 1
+#pragma unroll
   for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int b = 0; b < 3; ++b)
+    for (int b = 0; b < 3; ++b) {
+      const float wxy = ax.w[a] * ay.w[b];
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        const float weight = wx[a] * wy[b] * wz[c];
-        const int t = a * 49 + b * 7 + c;
-        const float u = weight * ta[t];
+        const float2 node = tp[a * 49 + b * 7 + c];
+        const float weight = wxy * az.w[c];
+        const float u = weight * node.x;
         r.s += u;
-        r.g0 += u * ((float)a - fx[0]);
-        r.g1 += u * ((float)b - fx[1]);
-        r.g2 += u * ((float)c - fx[2]);
-        r.w += weight * tw[t];
+        if (GRAD) {
+          r.g0 += u * ax.t[a];
+          r.g1 += u * ay.t[b];
+          r.g2 += u * az.t[c];
+        }
+        r.w += weight * node.y;
       }
-  r.g0 *= h;
-  r.g1 *= h;
-  r.g2 *= h;
+    }
+  if (GRAD) {
+    // Formed here, not where they are stored: sunk behind the tests in between, the gradients
+    // kept every u alive, which spilled.
+    asm volatile("" : "+v"(r.g0), "+v"(r.g1), "+v"(r.g2), "+v"(r.s), "+v"(r.w));
+    r.g0 *= h;
+    r.g1 *= h;
+    r.g2 *= h;
+  } else {
+    asm volatile("" : "+v"(r.s), "+v"(r.w));
+  }
   return r;
+}
+
+// What g2p_one takes from the scene, formed once per workgroup in scalar registers.
+struct G2pScene {
+  Frame f;
+  float step, spacing, t_thin, cs;
+  float lo[3], hi[3];
+  uint32_t flags;
+};
+__device__ __forceinline__ G2pScene g2p_scene(const Dev& d) {
+  const natray_params* U = d.U;
+  G2pScene s;
+  s.f = frame_of(U);
+  s.step = first_lane(dt_of(d));
+  s.spacing = U->fluid[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    s.lo[k] = first_lane(s.f.o[k] + 3.5f * s.f.h);
+    s.hi[k] = first_lane(s.f.o[k] + ((float)U->dims[k] - 4.5f) * s.f.h);
+  }
+  const float r_thin = 0.75f * s.spacing;
+  s.t_thin = first_lane(3.0f * __builtin_sqrtf(U->fluid[0] * r_thin * r_thin * r_thin / NATRAY_SIGMA_W));
+  s.cs = first_lane(4.0f / (s.f.h * s.f.h));
+  s.flags = d.sc->flags;
+  return s;
 }
 
 // carve for the moving capsule (the role of bullet.wgsl:395-424).
@@ -4169,39 +4243,34 @@ __device__ __forceinline__ void carve_cavity(const Dev& d, float x[3], float v[3
 
 // g2p_one (fluid.wgsl:806-861); returns the particle's speed, 0 once it is gone.
 template <bool CAV>
-__device__ __forceinline__ float g2p_one(const Dev& d, const float* tg, const uint32_t* links, uint32_t i, const int corner[3]) {
-  const natray_params* U = d.U;
-  const float hh = U->origin[3];
+__device__ __forceinline__ float g2p_one(const Dev& d, const G2pScene& sc, const float2* tg, const uint32_t* links, uint32_t i,
+                                         const int corner[3]) {
+  const float hh = sc.f.h;
   float4* P = reinterpret_cast<float4*>(d.P) + (size_t)i * 5;
   const float4 pos = P[0];
   const float c1w = P[3].w;
-  const float X[3] = {(pos.x - U->origin[0]) / hh, (pos.y - U->origin[1]) / hh, (pos.z - U->origin[2]) / hh};
+  float X[3];
+  cells_of(sc.f, pos.x, pos.y, pos.z, X);
   const int own[3] = {(int)floorf(X[0]), (int)floorf(X[1]), (int)floorf(X[2])};
   if ((unsigned)(own[0] - corner[0] - 1) > 3u || (unsigned)(own[1] - corner[1] - 1) > 3u ||
       (unsigned)(own[2] - corner[2] - 1) > 3u)
     return 0.0f;  // not in this block: only possible if the particle was moved behind the library's back
-  const Gathered gu = gather<0, 1, 1>(tg, X, corner, NATRAY_A_MOM(0), NATRAY_A_WT(0), hh);
-  const Gathered gv = gather<1, 0, 1>(tg, X, corner, NATRAY_A_MOM(1), NATRAY_A_WT(1), hh);
-  const Gathered gw = gather<1, 1, 0>(tg, X, corner, NATRAY_A_MOM(2), NATRAY_A_WT(2), hh);
-  const Gathered gp = gather<1, 1, 1>(tg, X, corner, NATRAY_A_PC, NATRAY_A_WC, hh);
+  const GatherAxis x0 = gather_axis<0>(X[0]), x1 = gather_axis<1>(X[0]), y0 = gather_axis<0>(X[1]), y1 = gather_axis<1>(X[1]),
+                   z0 = gather_axis<0>(X[2]), z1 = gather_axis<1>(X[2]);
+  const Gathered gu = gather<true>(tg, x0, y1, z1, corner, hh);
+  const Gathered gv = gather<true>(tg + TILE, x1, y0, z1, corner, hh);
+  const Gathered gw = gather<true>(tg + 2u * TILE, x1, y1, z0, corner, hh);
+  const Gathered gp = gather<false>(tg + 3u * TILE, x1, y1, z1, corner, hh);
   float v[3] = {gu.s, gv.s, gw.s};
   const float m_near = gu.w + gv.w + gw.w;
-  const float step = dt_of(d);
+  const float step = sc.step;
   float x[3] = {pos.x + step * v[0], pos.y + step * v[1], pos.z + step * v[2]};
   if (CAV) carve_cavity(d, x, v, i);
-  if (d.sc->flags & NATRAY_SCENE_CAPSULE) carve(d, x, v);
-  const float spacing = U->fluid[3];
-  float lo[3], hi[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    lo[k] = U->origin[k] + 3.5f * hh;
-    hi[k] = U->origin[k] + ((float)U->dims[k] - 4.5f) * hh;
-  }
-  const bool escaped = x[0] < lo[0] || x[2] < lo[2] || x[0] > hi[0] || x[2] > hi[2] || x[1] > hi[1];
+  if (sc.flags & NATRAY_SCENE_CAPSULE) carve(d, x, v);
+  const float spacing = sc.spacing;
+  const bool escaped = x[0] < sc.lo[0] || x[2] < sc.lo[2] || x[0] > sc.hi[0] || x[2] > sc.hi[2] || x[1] > sc.hi[1];
   const float fill = m_near / 24.0f;
   const bool on_ground = x[1] < 1.5f * spacing;
-  const float r_thin = 0.75f * spacing;
-  const float t_thin = 3.0f * __builtin_sqrtf(U->fluid[0] * r_thin * r_thin * r_thin / NATRAY_SIGMA_W);
   // `covered` only matters below fill 0.45 (the thin test and, below 0.2, the removal), so the
   // cell's mark is read only there.
   bool covered = false;
@@ -4209,10 +4278,10 @@ __device__ __forceinline__ float g2p_one(const Dev& d, const float* tg, const ui
     const uint32_t own_cell =
         tile_cell(links, (uint32_t)((own[0] - corner[0]) * 49 + (own[1] - corner[1]) * 7 + (own[2] - corner[2])));
     covered = own_cell != NONE && accr(d, NATRAY_A_MA, own_cell) > 0;
-    if ((d.sc->flags & NATRAY_SCENE_MASK) && in_mask(d, own[0], own[1], own[2])) covered = true;
+    if ((sc.flags & NATRAY_SCENE_MASK) && in_mask(d, own[0], own[1], own[2])) covered = true;
   }
   const float thin_age = (fill < 0.45f && !on_ground && !covered) ? c1w + step : 0.0f;
-  if (escaped || (!covered && fill < 0.2f) || thin_age > t_thin) {
+  if (escaped || (!covered && fill < 0.2f) || thin_age > sc.t_thin) {
     if (d.spray) {
       // Too thin for the grid: on the ground it soaks in, elsewhere it breaks up into spray.
       if (on_ground) {
@@ -4234,13 +4303,14 @@ __device__ __forceinline__ float g2p_one(const Dev& d, const float* tg, const ui
     vv[1] = fmax_(vv[1], 0.0f);
   }
   if (d.spray && xx[1] < 0.7f * spacing) ground_touch(d, xx[0], xx[2]);
-  const float cs = 4.0f / (hh * hh);
+  const float cs = sc.cs;
   P[0] = make_float4(xx[0], xx[1], xx[2], pos.w);
   P[1] = make_float4(vv[0], vv[1], vv[2], 1.0f);
   P[2] = make_float4(gu.g0 * cs, gu.g1 * cs, gu.g2 * cs, gp.w > 1e-6f ? gp.s / gp.w : 0.0f);
   P[3] = make_float4(gv.g0 * cs, gv.g1 * cs, gv.g2 * cs, thin_age);
   P[4] = make_float4(gw.g0 * cs, gw.g1 * cs, gw.g2 * cs, 0.0f);
-  d.key[i] = pack_key(d, xx[0], xx[1], xx[2], true);
+  cells_of(sc.f, xx[0], xx[1], xx[2], X);
+  d.key[i] = key_of(d.U, X);
   return __builtin_sqrtf((vv[0] * vv[0] + vv[1] * vv[1]) + vv[2] * vv[2]);
 }
 
@@ -4249,10 +4319,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
   const View v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
-  __shared__ float tg[8 * TILE];
+  // Per lattice (u, v, w, pressure) the nodes' values and weights.
+  __shared__ float2 tg[4 * TILE];
   __shared__ uint32_t links[27];
   const uint32_t n = n_blocks(d), tid = threadIdx.x;
   float fastest = 0.0f;
+  const G2pScene sc = g2p_scene(d);
   Dealer deal_s;
   __shared__ uint32_t deal_w[2];
   for (uint32_t b = deal_first(d, DEAL_G2P, n, v.wg, v.wgs, deal_s, deal_w); b < n; b = deal_next(deal_w)) {
@@ -4271,17 +4343,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
           u = cfr(d, NATRAY_F_U + k, cell);
           w = from_fp(accr(d, NATRAY_A_WT(k), cell), NATRAY_FP_W);
         }
-        tg[NATRAY_A_MOM(k) * TILE + t] = u;
-        tg[NATRAY_A_WT(k) * TILE + t] = w;
+        tg[k * TILE + t] = make_float2(u, w);
       }
-      tg[NATRAY_A_PC * TILE + t] = water ? pressure_of(d, cell) : 0.0f;
-      tg[NATRAY_A_WC * TILE + t] = water ? 1.0f : 0.0f;
+      tg[3u * TILE + t] = water ? make_float2(pressure_of(d, cell), 1.0f) : make_float2(0.0f, 0.0f);
     }
     __syncthreads();
     int bx, by, bz;
     slot_coord(d.U, d.block_list[b], bx, by, bz);
     const int corner[3] = {bx * 4 - 1, by * 4 - 1, bz * 4 - 1};
-    for (uint32_t k = tid; k < count; k += 256) fastest = fmax_(fastest, g2p_one<CAV>(d, tg, links, d.sorted[first + k], corner));
+    for (uint32_t k = tid; k < count; k += 256) fastest = fmax_(fastest, g2p_one<CAV>(d, sc, tg, links, d.sorted[first + k], corner));
   }
   // The workgroup's fastest particle goes to its own slot; k_vmax takes the maximum. One
   // atomic per wave on State.max_speed would serialise thousands of device-scope atomics on
