@@ -727,9 +727,12 @@ __device__ __forceinline__ uint32_t tile_cell(const uint32_t* links, uint32_t t)
 }
 
 // P2G's LDS tile: the 7^3 nodes a block's particles reach, x-major with padded strides, so
-// that the atomics of a half-wave's stencils spread over more LDS banks. Each lattice's node
+// that the atomics of a wave's stencils spread over more LDS banks. Each lattice's node
 // holds a pair of 32-bit sums, the weight's first and then the momentum's (or the pressure's).
-constexpr uint32_t P2G_SX = 60, P2G_SY = 8;
+// With one particle per cell of the block, a 64-bit atomic takes 6.2 cycles of the LDS at these
+// strides, the least of all strides below 13 and 113 (two 32-bit atomics take 8.3); at (60, 8) it
+// took 8.2, and the P2G phase 140 us on the 2M impact and 797 on the 15.2M one, now 123 and 663.
+constexpr uint32_t P2G_SX = 79, P2G_SY = 12;
 constexpr uint32_t P2G_TILE = 6u * P2G_SX + 6u * P2G_SY + 7u;
 // The largest weight one particle adds to a node is rint(0.75^3 * FP_W) = 7077888, so the
 // weight sums of a block of at most 606 particles stay below 2^32. Such a block adds each
@@ -866,7 +869,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
   const View v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
-  __shared__ __align__(8) int tile[8 * P2G_TILE];
+  __shared__ __align__(16) int tile[(8 * P2G_TILE + 3) / 4 * 4];
   __shared__ uint32_t cnt[64], drop[64];
   __shared__ uint32_t order[P2G_MAXP];
   __shared__ uint8_t ocell[P2G_MAXP];
@@ -885,7 +888,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
       cnt[tid] = 0;
       drop[tid] = 0;
     }
-    for (uint32_t t = tid; t < 8 * P2G_TILE; t += 256) tile[t] = 0;
+    for (uint32_t t = tid; t < (8 * P2G_TILE + 3) / 4; t += 256) reinterpret_cast<int4*>(tile)[t] = make_int4(0, 0, 0, 0);
     const uint32_t first = d.block_start[b], count = d.block_start[b + 1] - first;
     __syncthreads();
     deal_ahead(d, DEAL_P2G, n, v.wgs, deal_s, deal_w);
