@@ -130,6 +130,15 @@ struct Dev {
   // workgroup stays out (the test of a workgroup that is not resident).
   uint32_t solve_plain;
 };
+// Every pointer of Dev (kernels that read a Dev from memory declare these as global memory).
+#define NATRAY_DEV_POINTERS(X) \
+  X(U) X(sc) X(st) X(P) X(key) X(rank) X(block_ptr) X(slot_count) X(block_list) X(block_nb) \
+  X(block_start) X(sorted) X(acc) X(cf) X(bvec) X(nbm) X(part) X(tile_sum) X(tile_off) X(bar) \
+  X(rwords) X(hz) X(pcg) X(vmax_part) X(solver) X(stats) X(guess) X(ws_r0) X(ws_pcar) \
+  X(tile_map) X(tile_list) X(tile_scale) X(ws_in) X(ws_tgt) X(ws_mask) X(ws_diag) X(ws_nbm) \
+  X(ws_part) X(ws_stat) X(air_x) X(air_tmp) X(prev_ptr) X(block_list_prev) X(block_active) \
+  X(spray) X(landed) X(breakups) X(touch) X(mem_x) X(mem_v) X(mem_mass) X(mem_push) \
+  X(mem_water) X(bullets) X(patches) X(sections) X(bullet_rec) X(pose_log) X(self)
 
 // How a kernel finds its scene. One: a single scene, its Dev passed by value. Many: a batch of
 // scenes in one launch; workgroup w works for scene map[w].scene as its map[w].wg-th of

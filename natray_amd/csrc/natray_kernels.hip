@@ -45,14 +45,43 @@ constexpr float GAS = NATRAY_GAS, WATER = NATRAY_WATER, SOLID = NATRAY_SOLID, CO
 
 // A kernel's scene and its workgroup among the scene's: with One (a single scene, Dev by value)
 // the launch's own; with Many (a batch of scenes in one launch) from the workgroup map.
+template <class D>
 struct View {
-  const Dev& d;
+  D d;
   uint32_t wg, wgs;
 };
-__device__ __forceinline__ View view(const One& l) { return {l.d, blockIdx.x, gridDim.x}; }
-__device__ __forceinline__ View view(const Many& l) {
-  const WgMap m = l.map[blockIdx.x];
-  return {l.scenes[m.scene], m.wg, m.wgs};
+__device__ __forceinline__ View<const Dev&> view(const One& l) { return {l.d, blockIdx.x, gridDim.x}; }
+
+// Words of a struct in memory that no kernel writes, read as a kernel's arguments are.
+using DevWords = const __attribute__((address_space(4))) char*;
+// The pointer at `w`, read as one to global memory, which its loads and stores then say.
+template <class T>
+__device__ __forceinline__ void read_field(T*& f, DevWords w) {
+  using Global = __attribute__((address_space(1))) T*;
+  f = (T*)*(const __attribute__((address_space(4))) Global*)w;
+}
+// A Dev in device memory that no kernel writes, the same in every lane, as a kernel's own argument
+// would be: its words read by scalar loads as they are needed, its pointers known to be global.
+// Read through a plain pointer, every field was a vector load again after each store, and every
+// access behind its pointers a flat one, which waits on the LDS as well as on memory. A step of a
+// batch of 64 scenes (10.8M particles), us before and now: P2G 1134, 765; G2P 1031, 832; the solve
+// 1696, 1508; the rest 670, 570.
+__device__ __forceinline__ Dev load_dev(const Dev* p) {
+  DevWords const w = (DevWords)p;
+  Dev d;
+#pragma unroll
+  for (uint32_t k = 0; k < sizeof(Dev) / 8; ++k)
+    reinterpret_cast<uint64_t*>(&d)[k] = *(const __attribute__((address_space(4))) uint64_t*)(w + 8 * k);
+  static_assert(sizeof(Dev) % 8 == 0, "Dev is read in 8-byte words");
+#define NATRAY_READ(f) read_field(d.f, w + offsetof(Dev, f));
+  NATRAY_DEV_POINTERS(NATRAY_READ)
+#undef NATRAY_READ
+  return d;
+}
+__device__ __forceinline__ View<const Dev> view(const Many& l) {
+  using Words = const __attribute__((address_space(4))) uint32_t;
+  Words* const m = (Words*)(l.map + blockIdx.x);
+  return {load_dev(l.scenes + m[0]), m[1], m[2]};
 }
 
 // ---- small helpers ---------------------------------------------------------------------------
@@ -367,7 +396,7 @@ __device__ __forceinline__ uint32_t deal_next(const uint32_t* s_next) {
 
 template <class L>
 __global__ void k_begin(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (threadIdx.x != 0) return;
   natray_state* st = d.st;
@@ -433,7 +462,7 @@ __global__ void k_begin(L l) {
 // Keys of particles written from the host.
 template <class L>
 __global__ void k_keys(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   uint32_t i = v.wg * blockDim.x + threadIdx.x;
   if (i >= d.N) return;
@@ -450,7 +479,7 @@ __global__ void k_keys(L l) {
 // block pointers and counts are reset by the scan itself.
 template <class L>
 __global__ void k_clear(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   uint32_t n4 = d.st->n_blocks_prev * 16u;  // int4 per field
@@ -481,7 +510,7 @@ __global__ void k_clear(L l) {
 // is used.
 template <class L, uint32_t PER>
 __global__ __launch_bounds__(256) void k_mark(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   const natray_params* U = d.U;
@@ -553,7 +582,7 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
 // scan_blocks, first pass: claimed slots and their particles per tile of SCAN_TILE slots.
 template <class L>
 __global__ __launch_bounds__(256) void k_scan_reduce(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   __shared__ uint32_t ws[2][4];
@@ -591,7 +620,7 @@ __device__ __forceinline__ void wave_scan2(uint32_t& a, uint32_t& b) {
 // count and the overflow flag (claim, fluid.wgsl:117-121).
 template <class L>
 __global__ __launch_bounds__(1024) void k_scan_tiles(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   __shared__ uint32_t wsum[2][16];
@@ -639,7 +668,7 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(L l) {
 // (NONE where unclaimed); resets the counts for the next step.
 template <class L>
 __global__ __launch_bounds__(256) void k_scan_scatter(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   __shared__ uint32_t ws[2][4];
@@ -688,7 +717,7 @@ __global__ __launch_bounds__(256) void k_scan_scatter(L l) {
 // sort_particles (fluid.wgsl:189-196)
 template <class L, uint32_t PER>
 __global__ __launch_bounds__(256) void k_sort(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   // PER particles per thread, 256 apart, each step's loads in flight together (as k_mark).
@@ -866,7 +895,7 @@ constexpr uint32_t P2G_MAXR = 64;
 // lane idles while a crowded cell still has particles. The per-cell counts are A_N.
 template <class L>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_p2g(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   __shared__ __align__(16) int tile[(8 * P2G_TILE + 3) / 4 * 4];
@@ -1018,7 +1047,7 @@ __device__ __forceinline__ void for_blocks(const Dev& d, uint32_t b_lo, uint32_t
 // grid_prep (fluid.wgsl:319-356)
 template <class L>
 __global__ __launch_bounds__(256) void k_grid_prep(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   const float dt = dt_of(d);
@@ -1600,7 +1629,7 @@ __device__ __forceinline__ const float* start_pressure(const Dev& d) {
 // had four, in lock step: 190 us of the 15.2M impact's solve, 25 us here.
 template <class L>
 __global__ __launch_bounds__(256) void k_solve_rows(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   const float* const p0 = start_pressure(d);
@@ -2077,7 +2106,8 @@ __device__ __noinline__ void solve_memory(const Dev* dp, SolveSpan sp, uint32_t 
 
 // This workgroup's chunks and blocks in its scene's solve, and whether every workgroup keeps
 // its blocks on the chip (at most `regs` of them).
-__device__ __forceinline__ SolveSpan solve_span(const View& v, uint32_t regs, bool streams) {
+template <class V>
+__device__ __forceinline__ SolveSpan solve_span(const V& v, uint32_t regs, bool streams) {
   SolveSpan sp;
   sp.n = n_blocks(v.d);
   sp.K = sp.n ? (sp.n + MAX_CHUNKS - 1u) / MAX_CHUNKS : 1u;
@@ -2960,7 +2990,7 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
 
 template <bool MIXED, class L>
 __global__ __launch_bounds__(SOLVE_THREADS) void k_solve(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   using R = typename std::conditional<MIXED, double, float>::type;
   if (d.st->dt_ns == 0u) return;
@@ -3240,7 +3270,7 @@ __device__ __noinline__ void solve_pipe_memory(const Dev* dp, SolveSpan sp, uint
 
 template <class L>
 __global__ __launch_bounds__(SOLVE_THREADS) void k_solve_pipe(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   constexpr uint32_t RM = SOLVE_RMAX;
   if (d.st->dt_ns == 0u) return;
@@ -3533,7 +3563,7 @@ __device__ __forceinline__ uint32_t tile_voxel_cell(const Dev& d, uint32_t t, ui
 // tiles with water marked with their largest |r0|.
 template <class L>
 __global__ __launch_bounds__(256) void k_ws_prepare(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   const float* cP = d.cf + (size_t)NATRAY_F_P * d.capc;
@@ -3558,7 +3588,7 @@ __global__ __launch_bounds__(256) void k_ws_prepare(L l) {
 // clears the marks, and stores the listed count in bar[10].
 template <class L>
 __global__ __launch_bounds__(1024) void k_ws_tiles(L l, uint32_t cap) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   __shared__ uint32_t wsum[16];
   __shared__ uint32_t base;
@@ -3599,7 +3629,7 @@ __global__ __launch_bounds__(1024) void k_ws_tiles(L l, uint32_t cap) {
 // the network's input buffer ([slot][voxel][8], channels 2..7 zero).
 template <class L>
 __global__ __launch_bounds__(256) void k_ws_gather(L l, bf16x8* __restrict__ net_in) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   const uint32_t nb = n_blocks(d);
   const size_t total = (size_t)d.bar[10] * 4096u;
@@ -3634,7 +3664,7 @@ __global__ __launch_bounds__(256) void k_ws_gather(L l, bf16x8* __restrict__ net
 // FP32).
 template <class L>
 __global__ __launch_bounds__(256) void k_ws_scatter(L l, const float* __restrict__ pred) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   const uint32_t nb = n_blocks(d);
   const size_t total = (size_t)d.bar[10] * 4096u;
@@ -3649,7 +3679,7 @@ __global__ __launch_bounds__(256) void k_ws_scatter(L l, const float* __restrict
 // Per block: the squared residuals of the guess and of the carried pressure (lane tree, FP64).
 template <class L>
 __global__ __launch_bounds__(256) void k_ws_check(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   for_blocks(d, v.wg * 4u, n_blocks(d), v.wgs * 4u, [&](uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk) {
@@ -3668,7 +3698,7 @@ __global__ __launch_bounds__(256) void k_ws_check(L l) {
 // when its residual is the smaller; keeps the sums and counts in ws_stat.
 template <class L>
 __global__ __launch_bounds__(1024) void k_ws_decide(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   __shared__ double sh[2][1024];
   if (d.st->dt_ns == 0u) return;
@@ -3704,13 +3734,13 @@ __global__ __launch_bounds__(1024) void k_ws_decide(L l) {
 // host holds at zero.
 template <class L>
 __global__ __launch_bounds__(64) void k_ws_zero_start(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   if (v.wg == 0u && threadIdx.x == 0u) v.d.bar[11] = 1u;
 }
 
 template <class L>
 __global__ __launch_bounds__(256) void k_ws_samples(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   const uint32_t nb = n_blocks(d);
   const float* cP = d.cf + (size_t)NATRAY_F_P * d.capc;
@@ -3731,7 +3761,7 @@ __global__ __launch_bounds__(256) void k_ws_samples(L l) {
 
 template <class L>
 __global__ __launch_bounds__(256) void k_project(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   const float k = dt_of(d) / (d.U->fluid[0] * d.U->origin[3]);
@@ -3777,7 +3807,7 @@ __device__ __forceinline__ void face_offsets(int k, int& ox, int& oy, int& oz) {
 // trip per test; the faces and sums are those of the reference, in its order.
 template <class L>
 __global__ __launch_bounds__(256) void k_extend1(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   for_blocks(d, v.wg * 4u, n_blocks(d), v.wgs * 4u,
@@ -3845,7 +3875,7 @@ __global__ __launch_bounds__(256) void k_extend1(L l) {
 // skips the neighbours, and any other loads every neighbour's mark and value up front.
 template <class L>
 __global__ __launch_bounds__(256) void k_extend2(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   for_blocks(d, v.wg * 4u, n_blocks(d), v.wgs * 4u,
@@ -4116,7 +4146,7 @@ __device__ __forceinline__ void break_up(const Dev& d, float x0, float x1, float
 
 template <class L>
 __global__ __launch_bounds__(256) void k_break_up(L l) {
-  const View vw = view(l);
+  const auto vw = view(l);
   const Dev& d = vw.d;
   if (d.st->dt_ns == 0u || !d.spray) return;
   const uint32_t n = d.bar[12];
@@ -4136,7 +4166,7 @@ __device__ __forceinline__ float drag_cd(float re) {
 // spray_update (fluid.wgsl:686-711), grid-stride over the records made so far.
 template <class L>
 __global__ __launch_bounds__(256) void k_spray_update(L l) {
-  const View vw = view(l);
+  const auto vw = view(l);
   const Dev& d = vw.d;
   if (d.st->dt_ns == 0u || !d.spray) return;
   const uint32_t n = min(d.st->spray_count, d.spray_cap);
@@ -4319,7 +4349,7 @@ __device__ __forceinline__ float g2p_one(const Dev& d, const G2pScene& sc, const
 
 template <class L, bool CAV = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_g2p(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   // Per lattice (u, v, w, pressure) the nodes' values and weights.
@@ -4370,7 +4400,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
 // fluid.wgsl:898-900 as a reduction).
 template <class L>
 __global__ __launch_bounds__(256) void k_vmax(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   const uint32_t parts = d.g2p_wgs;
@@ -4422,7 +4452,7 @@ __device__ __forceinline__ uint32_t cell_at(const Dev& d, int cx, int cy, int cz
 // water are claimed, so the air there is simulated too.
 template <class L>
 __global__ __launch_bounds__(256) void k_mark_rubber(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   const uint32_t i = v.wg * blockDim.x + threadIdx.x;
@@ -4450,7 +4480,7 @@ __global__ __launch_bounds__(256) void k_mark_rubber(L l) {
 // atomics take most. The sums are integers, so their order is free.
 template <class L>
 __global__ __launch_bounds__(256) void k_mem_splat(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   const natray_params* U = d.U;
@@ -4504,7 +4534,7 @@ __global__ __launch_bounds__(256) void k_mem_splat(L l) {
 constexpr uint32_t MEM_VERTS = 8;  // vertices per workgroup
 template <class L>
 __global__ __launch_bounds__(256) void k_mem_sample(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
   __shared__ float2 term[MEM_VERTS][4][28];
@@ -4719,7 +4749,7 @@ constexpr uint32_t PATCH_REC = 12;
 // 144 workgroups of 4 waves.
 template <class L>
 __global__ __launch_bounds__(256) void k_bullet_patches(L l) {
-  const View vw = view(l);
+  const auto vw = view(l);
   const Dev& d = vw.d;
   if (d.st->dt_ns == 0u) return;
   const natray_params* U = d.U;
@@ -4866,7 +4896,7 @@ __global__ __launch_bounds__(256) void k_bullet_patches(L l) {
 // sections' volume source splatted. One workgroup of 256 per bullet.
 template <class L>
 __global__ __launch_bounds__(256) void k_bullet_body(L l) {
-  const View vw = view(l);
+  const auto vw = view(l);
   const Dev& d = vw.d;
   if (d.st->dt_ns == 0u) return;
   const natray_params* U = d.U;
@@ -5028,7 +5058,7 @@ __global__ __launch_bounds__(256) void k_bullet_body(L l) {
 // bullet_apply (bullet.wgsl:379-386): the bullets' pushes onto the water's faces.
 template <class L>
 __global__ __launch_bounds__(256) void k_bullet_apply(L l) {
-  const View vw = view(l);
+  const auto vw = view(l);
   const Dev& d = vw.d;
   if (d.st->dt_ns == 0u) return;
   const uint32_t cells = n_blocks(d) * 64u;
@@ -5072,7 +5102,7 @@ __device__ __forceinline__ void write_gas(float* air, uint32_t capc, uint32_t ce
 // claimed again.
 template <class L>
 __global__ __launch_bounds__(256) void k_keep_blocks(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u || !d.air_x) return;
   for (uint32_t i = v.wg * blockDim.x + threadIdx.x; i < d.st->n_blocks_prev; i += v.wgs * blockDim.x)
@@ -5083,7 +5113,7 @@ __global__ __launch_bounds__(256) void k_keep_blocks(L l) {
 // the ambient air where its block was not allocated then.
 template <class L>
 __global__ __launch_bounds__(256) void k_air_carry(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u || !d.air_x) return;
   const uint32_t n_prev = d.st->n_blocks_prev;
@@ -5101,7 +5131,7 @@ __global__ __launch_bounds__(256) void k_air_carry(L l) {
 // its gas's, a RUBBER cell's the lowest of its GAS neighbours' (gauge).
 template <class L>
 __global__ __launch_bounds__(256) void k_air_fill(L l) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u || !d.air_x) return;
   const uint32_t capc = d.capc;
@@ -5165,7 +5195,7 @@ __device__ __forceinline__ uint2 pack_pos(float px, float py, float pz, bool fla
 // pack_water (pack.wgsl:33-39): two words per particle, the flag for a live particle.
 template <class L>
 __global__ __launch_bounds__(256) void k_pack_water(L l, uint2* __restrict__ out) {
-  const View v = view(l);
+  const auto v = view(l);
   const Dev& d = v.d;
   const uint32_t i = v.wg * blockDim.x + threadIdx.x;
   if (i >= d.N) return;
