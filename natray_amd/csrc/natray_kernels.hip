@@ -2632,6 +2632,7 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
   uint32_t rM[RM], hw[RM];
   QuadHalo hD{};                            // one set: the far halo's directions
   QuadLinks lk = {NONE, NONE, NONE, NONE};  // one set: the links
+  float dOld[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // one set: the direction before the last
   auto first_block = [&](uint32_t r) -> uint32_t { return b0 + 4u * (wv + SOLVE_WAVES * r); };
   // The block of this lane in set r, among the workgroup's.
   uint32_t at = 4u * wv + l.q;
@@ -2858,7 +2859,10 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
       const float dn[4] = {(m & 1u) ? rZ[r][0] + fb * o.x : 0.0f, (m & 2u) ? rZ[r][1] + fb * o.y : 0.0f,
                            (m & 4u) ? rZ[r][2] + fb * o.z : 0.0f, (m & 8u) ? rZ[r][3] + fb * o.w : 0.0f};
       lds.d[pl][l.col] = make_float4(dn[0], dn[1], dn[2], dn[3]);
-      quad_store(cDn, (b0 + pl) * 64u + l.col * 4u, l.odd, dn, m);
+      if (WIDE)
+        quad_store(cDn, (b0 + pl) * 64u + l.col * 4u, l.odd, dn, m);
+      else
+        dOld[0] = o.x, dOld[1] = o.y, dOld[2] = o.z, dOld[3] = o.w;
     }
     wg_sync(false);
     new_pass();
@@ -2964,8 +2968,11 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
     if (!quad_reduce<R, 2>(d, sp, tag, qw, lp, tt, publish_z, halo_z)) break;
     go = solve_beta<R>(d, tt, s);
   }
-  // The fields the other kernels and the host read: p, r, z and q of the water cells (solve_q
-  // stored the directions). q is formed again from the last direction: the same bits.
+  // The fields the other kernels and the host read: p, r, z and q of the water cells, and with one
+  // set the last two directions. Stored in every iteration, as more sets still do for want of
+  // registers, they took 0.2 us of it: 5.6 us at 176 blocks and 6.0 at 961 are now 5.4 and 5.75,
+  // and in mixed precision 8.6 at 2946 are 7.7. q is formed again from the last direction: the
+  // same bits.
   new_pass();
 #pragma unroll
   for (uint32_t r = 0; r < RM; ++r) {
@@ -2984,6 +2991,10 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
     const float dn[4] = {o.x, o.y, o.z, o.w};
     quad_row<float>(dn, g, h, l, q);
     quad_store(cQ, cell0, l.odd, q, m);
+    if (!WIDE) {
+      quad_store(cD + (size_t)(s.iters % 2u) * capc, cell0, l.odd, dn, m);
+      quad_store(cD + (size_t)(1u - s.iters % 2u) * capc, cell0, l.odd, dOld, m);
+    }
   }
   solve_finish<R>(d, sp, tag, s);
 }

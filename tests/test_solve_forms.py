@@ -87,3 +87,12 @@ def test_divisions_outside_the_fast_range(what, precision):
         s.params.fluid[3] = 0.5
         s.scene.fixed_dt = 2e-8
     solve_and_compare(s, 3)
+
+
+@pytest.mark.parametrize("iters", [1, 2, 3])
+@pytest.mark.parametrize("groups", [1, 3])
+def test_few_iterations(iters, groups):
+    """Solves that end at their first iterations: the last two directions, one of them the solve's
+    own start after a single iteration, are among the fields compared."""
+    s = scenes.balloon_impact(side=64, n=32768, seed=2, iters=iters, capacity=4096)
+    solve_and_compare(s, groups)
