@@ -47,7 +47,6 @@ struct Dev {
   uint32_t* nbm;           // capc: bit k = face neighbour k is water, bit 6 = the cell is water
   double* part;            // cap x 4: per-block partial sums of the solver (memory form)
   uint32_t* tile_sum;      // 2 x ntiles: scan tile totals (slots claimed, particles)
-  uint32_t* tile_off;      // 2 x ntiles: their exclusive prefix
   uint32_t* bar;           // control words: [2] the solve's abort flag a stuck wait raises,
                            // [4] its last reduction tag, [10] warm-start tiles this step, [11] 1
                            // when the solve starts from the warm start's guess, [12] particles
@@ -133,7 +132,7 @@ struct Dev {
 // Every pointer of Dev (kernels that read a Dev from memory declare these as global memory).
 #define NATRAY_DEV_POINTERS(X) \
   X(U) X(sc) X(st) X(P) X(key) X(rank) X(block_ptr) X(slot_count) X(block_list) X(block_nb) \
-  X(block_start) X(sorted) X(acc) X(cf) X(bvec) X(nbm) X(part) X(tile_sum) X(tile_off) X(bar) \
+  X(block_start) X(sorted) X(acc) X(cf) X(bvec) X(nbm) X(part) X(tile_sum) X(bar) \
   X(rwords) X(hz) X(pcg) X(vmax_part) X(solver) X(stats) X(guess) X(ws_r0) X(ws_pcar) \
   X(tile_map) X(tile_list) X(tile_scale) X(ws_in) X(ws_tgt) X(ws_mask) X(ws_diag) X(ws_nbm) \
   X(ws_part) X(ws_stat) X(air_x) X(air_tmp) X(prev_ptr) X(block_list_prev) X(block_active) \
@@ -177,7 +176,7 @@ struct Target {
 namespace natray {
 int launch_keys(const Target& t, void* stream);
 int launch_begin(const Target& t, void* stream);
-int launch_bin(const Target& t, void* stream, bool rubber = false, bool air = false);
+int launch_bin(const Target& t, void* stream, bool rubber = false);
 int launch_p2g(const Target& t, void* stream);
 int launch_grid_prep(const Target& t, void* stream);
 // The solve of precision `kind` (NATRAY_CG_FP32, _MIXED or _PIPELINED).

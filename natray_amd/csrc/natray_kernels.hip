@@ -2,10 +2,10 @@
 //
 // One step runs, in the reference's plan order (src/sim.rs:390-426):
 //   k_begin                       begin_step                 shaders/fluid.wgsl:31-89
-//   k_clear k_mark k_scan_* k_sort clear/mark/scan/sort      shaders/fluid.wgsl:91-196
+//   k_mark k_scan_* k_sort        clear/mark/scan/sort       shaders/fluid.wgsl:91-196
 //   k_p2g                         p2g                        shaders/fluid.wgsl:198-303
 //   k_grid_prep                   grid_prep                  shaders/fluid.wgsl:305-356
-//   k_solve (cooperative)         solve_init..solve_beta     shaders/fluid.wgsl:381-578
+//   k_solve_rows k_solve          solve_init..solve_beta     shaders/fluid.wgsl:381-578
 //   k_project                     project                    shaders/fluid.wgsl:580-598
 //   k_extend1 k_extend2           extend_1, extend_2         shaders/fluid.wgsl:600-674
 //   k_g2p                         g2p                        shaders/fluid.wgsl:767-901
@@ -18,10 +18,10 @@
 //     P2G accumulates there with LDS integer atomics and flushes each non-zero tile sum with one
 //     global integer atomic, so grid sums are exact and order-independent;
 //   - block allocation is a deterministic compaction of claimed domain slots in slot order (a
-//     three-kernel scan), replacing the reference's CAS claims; particle ranks use wave-
+//     two-kernel scan), replacing the reference's CAS claims; particle ranks use wave-
 //     aggregated atomics;
-//   - the whole pressure solve is one persistent cooperative launch with a grid barrier, so the
-//     GPU decides when to stop iterating without host round trips.
+//   - the CG iterations are one persistent launch of co-resident workgroups, so the GPU decides
+//     when to stop iterating without host round trips.
 // Every float expression is written in the reference's order and compiled without
 // contraction, so the kernels reproduce the CPU oracle bit for bit given the same inputs.
 #include <hip/hip_runtime.h>
@@ -476,20 +476,17 @@ __global__ void k_keys(L l) {
 // ---- binning (shaders/fluid.wgsl:91-196) ---------------------------------------------------------
 
 // clear_blocks (fluid.wgsl:91-107): zero the transfer sums of last step's cells. The slots'
-// block pointers and counts are reset by the scan itself.
-template <class L>
-__global__ void k_clear(L l) {
-  const auto v = view(l);
-  const Dev& d = v.d;
-  if (d.st->dt_ns == 0u) return;
-  uint32_t n4 = d.st->n_blocks_prev * 16u;  // int4 per field
-  // With the air boundary, the last step's block list and each slot's place in it (read by
-  // air_carry and keep_blocks; this step's list is built after this kernel).
+// block pointers and counts are reset by the scan itself. With the air boundary, also keep the
+// last step's block list and each slot's place in it (read by air_carry), and claim the blocks
+// whose air was active, as keep_blocks does; this step's list is built after this kernel.
+__device__ __forceinline__ void clear_blocks(const Dev& d, uint32_t wg, uint32_t wgs) {
+  const uint32_t n_prev = d.st->n_blocks_prev, n4 = n_prev * 16u;  // int4 per field
   if (d.air_x)
-    for (uint32_t b = v.wg * blockDim.x + threadIdx.x; b < d.st->n_blocks_prev; b += v.wgs * blockDim.x) {
+    for (uint32_t b = wg * blockDim.x + threadIdx.x; b < n_prev; b += wgs * blockDim.x) {
       const uint32_t s = d.block_list[b];
       d.block_list_prev[b] = s;
       d.prev_ptr[s] = b;
+      if (d.block_active[b] != 0u) d.block_ptr[s] = PENDING;
     }
   // The transfer fields, with a membrane its coupling fields (A_MF, A_MA, A_MW, A_MV) and with
   // bullets theirs (A_BU, A_SRC).
@@ -498,8 +495,13 @@ __global__ void k_clear(L l) {
     const bool bullet_f = f >= NATRAY_A_BU && f <= NATRAY_A_SRC;
     if ((mem_f && !d.mem_cap) || (bullet_f && !d.n_bullets)) continue;
     int4* a = reinterpret_cast<int4*>(d.acc + (size_t)f * d.capc);
-    for (uint32_t i = v.wg * blockDim.x + threadIdx.x; i < n4; i += v.wgs * blockDim.x) a[i] = make_int4(0, 0, 0, 0);
+    for (uint32_t i = wg * blockDim.x + threadIdx.x; i < n4; i += wgs * blockDim.x) a[i] = make_int4(0, 0, 0, 0);
   }
+}
+template <class L>
+__global__ void k_clear(L l) {
+  const auto v = view(l);
+  if (v.d.st->dt_ns != 0u) clear_blocks(v.d, v.wg, v.wgs);
 }
 
 // mark_blocks + claim (fluid.wgsl:109-150): mark the blocks of cells c-1..c+2 as claimed and
@@ -507,15 +509,17 @@ __global__ void k_clear(L l) {
 // and atomics are in flight together: the kernel is a chain of dependent round trips (key,
 // block slots, the claim), and fewer, fuller waves wait through fewer of them. Lanes of a wave
 // with the same own block share one atomic; every group's atomic is issued before any result
-// is used.
+// is used. The first `clears` workgroups clear instead: neither needs the other, both are short
+// of work for the chip in a small scene, and a launch of its own cost the clearing 5 us.
 template <class L, uint32_t PER>
-__global__ __launch_bounds__(256) void k_mark(L l) {
+__global__ __launch_bounds__(256) void k_mark(L l, uint32_t clears) {
   const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
+  if (v.wg < clears) return clear_blocks(d, v.wg, clears);
   const natray_params* U = d.U;
   const uint32_t lane = lane_id();
-  const uint32_t i0 = v.wg * 256u * PER + threadIdx.x;
+  const uint32_t i0 = (v.wg - clears) * 256u * PER + threadIdx.x;
   uint32_t key[PER], own[PER];
 #pragma unroll
   for (uint32_t k = 0; k < PER; ++k) {
@@ -616,63 +620,24 @@ __device__ __forceinline__ void wave_scan2(uint32_t& a, uint32_t& b) {
   }
 }
 
-// scan_blocks, second pass: exclusive prefix of the tile totals (one workgroup), the block
-// count and the overflow flag (claim, fluid.wgsl:117-121).
-template <class L>
-__global__ __launch_bounds__(1024) void k_scan_tiles(L l) {
-  const auto v = view(l);
-  const Dev& d = v.d;
-  if (d.st->dt_ns == 0u) return;
-  __shared__ uint32_t wsum[2][16];
-  const uint32_t nt = d.ntiles, t = threadIdx.x;
-  const uint32_t per = (nt + 1023u) / 1024u;
-  const uint32_t lo = min(t * per, nt), hi = min(lo + per, nt);
-  uint32_t fa = 0, ca = 0;
-  for (uint32_t j = lo; j < hi; ++j) {
-    fa += d.tile_sum[j];
-    ca += d.tile_sum[nt + j];
-  }
-  uint32_t fi = fa, ci = ca;
-  wave_scan2(fi, ci);
-  const uint32_t w = t >> 6;
-  if (lane_id() == 63) {
-    wsum[0][w] = fi;
-    wsum[1][w] = ci;
-  }
-  __syncthreads();
-  uint32_t fo = 0, co = 0;
-  for (uint32_t k = 0; k < w; ++k) {
-    fo += wsum[0][k];
-    co += wsum[1][k];
-  }
-  uint32_t frun = fo + fi - fa, crun = co + ci - ca;
-  for (uint32_t j = lo; j < hi; ++j) {
-    d.tile_off[j] = frun;
-    d.tile_off[nt + j] = crun;
-    frun += d.tile_sum[j];
-    crun += d.tile_sum[nt + j];
-  }
-  if (t == 1023) {
-    uint32_t total_f = fo + fi, total_c = co + ci;
-    uint32_t cap = d.U->bdims[3];
-    d.st->n_blocks = total_f;
-    if (total_f > cap) {
-      d.st->overflow = 1u;
-    } else {
-      d.block_start[total_f] = total_c;
-    }
-  }
-}
-
-// scan_blocks, third pass: block indices in slot order, block starts, and every slot's pointer
-// (NONE where unclaimed); resets the counts for the next step.
+// scan_blocks, second pass: block indices in slot order, block starts, and every slot's pointer
+// (NONE where unclaimed); resets the counts for the next step. Each workgroup adds up the totals of
+// the tiles before its own, and the last one's sum gives the block count and the overflow flag
+// (claim, fluid.wgsl:117-121). A pass of one workgroup that formed every tile's prefix first was a
+// launch more: binning took 26.2 us, now 23.1, in a domain of 32 tiles, 28.6, now 25.6, in one of
+// 977, and still 123.1, now 118.7, in the largest (16,193).
 template <class L>
 __global__ __launch_bounds__(256) void k_scan_scatter(L l) {
   const auto v = view(l);
   const Dev& d = v.d;
   if (d.st->dt_ns == 0u) return;
-  __shared__ uint32_t ws[2][4];
+  __shared__ uint32_t ws[2][4], before[2][4];
   const uint32_t j = v.wg, base = j * SCAN_TILE + threadIdx.x * 4u;
+  uint32_t pf = 0, pc = 0;
+  for (uint32_t k = threadIdx.x; k < j; k += 256u) {
+    pf += d.tile_sum[k];
+    pc += d.tile_sum[d.ntiles + k];
+  }
   uint4 bp = *reinterpret_cast<const uint4*>(d.block_ptr + base);
   uint4 sc = *reinterpret_cast<const uint4*>(d.slot_count + base);
   uint32_t fl[4] = {bp.x == PENDING, bp.y == PENDING, bp.z == PENDING, bp.w == PENDING};
@@ -681,19 +646,32 @@ __global__ __launch_bounds__(256) void k_scan_scatter(L l) {
   uint32_t fi = fa, ci = ca;
   wave_scan2(fi, ci);
   const uint32_t w = threadIdx.x >> 6;
+  pf = wave_sum(pf);
+  pc = wave_sum(pc);
   if (lane_id() == 63) {
     ws[0][w] = fi;
     ws[1][w] = ci;
+    before[0][w] = pf;
+    before[1][w] = pc;
   }
   __syncthreads();
-  uint32_t fo = d.tile_off[j], co = d.tile_off[d.ntiles + j];
+  uint32_t fo = before[0][0] + before[0][1] + before[0][2] + before[0][3];
+  uint32_t co = before[1][0] + before[1][1] + before[1][2] + before[1][3];
+  const uint32_t cap = d.U->bdims[3];
+  if (threadIdx.x == 0 && j + 1u == d.ntiles) {
+    const uint32_t total = fo + ws[0][0] + ws[0][1] + ws[0][2] + ws[0][3];
+    d.st->n_blocks = total;
+    if (total > cap)
+      d.st->overflow = 1u;
+    else
+      d.block_start[total] = co + ws[1][0] + ws[1][1] + ws[1][2] + ws[1][3];
+  }
   for (uint32_t k = 0; k < w; ++k) {
     fo += ws[0][k];
     co += ws[1][k];
   }
   fo += fi - fa;
   co += ci - ca;
-  const uint32_t cap = d.U->bdims[3];
   uint32_t out[4];
   for (int q = 0; q < 4; ++q) {
     uint32_t s = base + (uint32_t)q;
@@ -4398,8 +4376,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
     for (uint32_t k = tid; k < count; k += 256) fastest = fmax_(fastest, g2p_one<CAV>(d, sc, tg, links, d.sorted[first + k], corner));
   }
   // The workgroup's fastest particle goes to its own slot; k_vmax takes the maximum. One
-  // atomic per wave on State.max_speed would serialise thousands of device-scope atomics on
-  // one word.
+  // atomic per workgroup on State.max_speed instead of k_vmax's launch took 0.1 us each: 120 us
+  // of a step of the 2M impact.
   __shared__ float s_fast[4];
   for (int off = 32; off > 0; off >>= 1) fastest = fmax_(fastest, __shfl_xor(fastest, off));
   if (lane_id() == 0) s_fast[tid >> 6] = fastest;
@@ -5109,17 +5087,6 @@ __device__ __forceinline__ void write_gas(float* air, uint32_t capc, uint32_t ce
   air[4 * (size_t)capc + cell] = g.e;
 }
 
-// keep_blocks (air.wgsl:271-277): the blocks whose air was doing anything last step are
-// claimed again.
-template <class L>
-__global__ __launch_bounds__(256) void k_keep_blocks(L l) {
-  const auto v = view(l);
-  const Dev& d = v.d;
-  if (d.st->dt_ns == 0u || !d.air_x) return;
-  for (uint32_t i = v.wg * blockDim.x + threadIdx.x; i < d.st->n_blocks_prev; i += v.wgs * blockDim.x)
-    if (d.block_active[i] != 0u) d.block_ptr[d.block_list_prev[i]] = PENDING;
-}
-
 // air_carry (air.wgsl:85-98): each cell of this step's blocks gets the gas it had last step, or
 // the ambient air where its block was not allocated then.
 template <class L>
@@ -5528,19 +5495,19 @@ int launch_begin(const Target& t, void* stream) {
   NATRAY_LAUNCH(k_begin, LK_ONE, 64, t, S(stream));
   return (int)hipGetLastError();
 }
-int launch_bin(const Target& t, void* stream, bool rubber, bool air) {
-  NATRAY_LAUNCH(k_clear, LK_CELLS, 256, t, S(stream));
-  if (air) NATRAY_LAUNCH(k_keep_blocks, LK_ONE, 256, t, S(stream));
-  // A single scene's marks take four particles per thread; a batch's scenes share the particle
-  // workgroup map, one particle per thread.
-  if (t.d)
-    hipLaunchKernelGGL((k_mark<One, 4>), dim3((t.grid[LK_PARTS] + 3u) / 4u), dim3(256), 0, S(stream), One{*t.d});
-  else
+int launch_bin(const Target& t, void* stream, bool rubber) {
+  // A single scene's marks take four particles per thread, and the clearing is in their launch; a
+  // batch's scenes share the particle workgroup map, one particle per thread.
+  if (t.d) {
+    const uint32_t clears = t.grid[LK_CELLS];
+    hipLaunchKernelGGL((k_mark<One, 4>), dim3(clears + (t.grid[LK_PARTS] + 3u) / 4u), dim3(256), 0, S(stream), One{*t.d}, clears);
+  } else {
+    NATRAY_LAUNCH(k_clear, LK_CELLS, 256, t, S(stream));
     hipLaunchKernelGGL((k_mark<Many, 1>), dim3(t.grid[LK_PARTS]), dim3(256), 0, S(stream),
-                       Many{t.scenes, t.map[LK_PARTS]});
+                       Many{t.scenes, t.map[LK_PARTS]}, 0u);
+  }
   if (rubber) NATRAY_LAUNCH(k_mark_rubber, LK_VERTS, 256, t, S(stream));
   NATRAY_LAUNCH(k_scan_reduce, LK_TILES, 256, t, S(stream));
-  NATRAY_LAUNCH(k_scan_tiles, LK_ONE, 1024, t, S(stream));
   NATRAY_LAUNCH(k_scan_scatter, LK_TILES, 256, t, S(stream));
   if (t.d)
     hipLaunchKernelGGL((k_sort<One, 4>), dim3((t.grid[LK_PARTS] + 3u) / 4u), dim3(256), 0, S(stream), One{*t.d});

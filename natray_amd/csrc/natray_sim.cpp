@@ -245,7 +245,7 @@ int enqueue_phase(natray_sim* s, int phase) {
   }
   switch (phase) {
     case NATRAY_PHASE_BEGIN: LAUNCHCHK(natray::launch_begin(s->tgt, st)); break;
-    case NATRAY_PHASE_BIN: LAUNCHCHK(natray::launch_bin(s->tgt, st, s->D.mem_cap > 0, s->D.air_x != nullptr)); break;
+    case NATRAY_PHASE_BIN: LAUNCHCHK(natray::launch_bin(s->tgt, st, s->D.mem_cap > 0)); break;
     case NATRAY_PHASE_P2G:
       LAUNCHCHK(natray::launch_p2g(s->tgt, st));
       if (s->D.air_x) LAUNCHCHK(natray::launch_air_carry(s->tgt, st));
@@ -528,7 +528,6 @@ int natray_sim_create(const natray_params* params, const float* particles, uint3
   TRY(dalloc(s, &D.hz, 3 * capc));
   if (s->sc.precision == NATRAY_CG_PIPELINED) TRY(dalloc(s, &D.pcg, 4 * capc));
   TRY(dalloc(s, &D.tile_sum, (size_t)D.ntiles * 2));
-  TRY(dalloc(s, &D.tile_off, (size_t)D.ntiles * 2));
   TRY(dalloc(s, &D.bar, 1024));
   TRY(dalloc(s, &D.vmax_part, (size_t)D.cap));
   TRY(dalloc(s, &D.solver, 8));
@@ -1542,7 +1541,7 @@ int batch_phase_launch(natray_batch* b, int phase) {
   void* st = b->stream;
   switch (phase) {
     case NATRAY_PHASE_BEGIN: LAUNCHCHK(natray::launch_begin(t, st)); break;
-    case NATRAY_PHASE_BIN: LAUNCHCHK(natray::launch_bin(t, st, false, b->air)); break;
+    case NATRAY_PHASE_BIN: LAUNCHCHK(natray::launch_bin(t, st, false)); break;
     case NATRAY_PHASE_P2G:
       LAUNCHCHK(natray::launch_p2g(t, st));
       if (b->air) LAUNCHCHK(natray::launch_air_carry(t, st));
