@@ -55,9 +55,10 @@ struct Dev {
   unsigned long long* rwords;  // RED_WORDS: tagged chunk sums of the solve's reductions
   unsigned long long* hz;      // 3 x capc: tagged halo words. By cell, for the memory form's
                                // streaming passes (z in the first third, the directions
-                               // alternating between the other two) and the pipelined form
-                               // (alternating between the first two); by face, for the solve's
-                               // on-chip forms (z in the first half, p in the second)
+                               // alternating between the other two) and the pipelined form of
+                               // one block a wave (alternating between the first two); by face,
+                               // for the forms on quads (two halves: z and p, or the pipelined
+                               // form's alternating buffers)
   float* pcg;                  // 4 x capc: z, q and two m buffers of the pipelined solve's memory
                                // form (NATRAY_CG_PIPELINED only; else null)
   float* vmax_part;        // fastest particle of each g2p workgroup (<= cap workgroups)

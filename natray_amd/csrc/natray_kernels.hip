@@ -1115,8 +1115,6 @@ constexpr uint32_t SOLVE_ITER_CAP = 1u << 24;
 
 constexpr uint32_t SOLVE_THREADS = 1024;
 constexpr uint32_t SOLVE_WAVES = SOLVE_THREADS / 64;
-// Blocks a wave of the pipelined solve keeps in registers.
-constexpr uint32_t SOLVE_RMAX = 2;
 // Sets of four blocks a wave of the solve keeps on the chip: one with every field in registers
 // (workgroups of at most 64 blocks), or QUAD_WIDE (at most 256 blocks).
 constexpr uint32_t QUAD_WIDE = 4;
@@ -1587,13 +1585,6 @@ __device__ __forceinline__ void start_cell(const Dev& d, uint32_t cell, uint32_t
     prow[2] = v2;
     prow[3] = (R)nw;
   }
-}
-template <class R>
-__device__ __forceinline__ void init_cell(const Dev& d, uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk,
-                                          unsigned long long* zw, uint32_t ztag, R* prow, const float* p0) {
-  const Row w = row_cell(d, b, lane, lx, ly, lz, lk, p0);
-  start_cell<R>(d, b * 64u + lane, lane, lx, ly, lz, w.water, w.diag, w.water ? w.r : 0.0f, w.water ? w.bv : 0.0f, zw, ztag,
-                prow);
 }
 
 // The starting pressure of this solve: the warm start's guess when it was accepted this step
@@ -3027,14 +3018,15 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_solve(L l) {
 // (the tolerance test's right-hand side times PIPE_REPLACE), where the gap is still small
 // against r; the gap that builds up afterwards starts from residuals that small.
 //
-// Register form: m of the water cells on block faces is published as tagged words and read by
-// the neighbours while the iteration's reduction completes, so the halo exchange costs no wait
-// of its own. A replacement exchanges x, u, p and q in turn. Halo words are numbered 8 t + k
-// (t the iteration's reduction tag; k = 0 for m, 1..4 for x, u, p, q of a replacement; u0 at
-// the start has 8 t + 5 with t the start's reduction) and alternate between two word buffers:
-// m of reduction t and u and q of its replacement in buffer t & 1, x and p in the other, u0
-// in the start's. A wave rewrites a buffer only after a reduction or an exchange that every
-// neighbour joins after it has read the buffer's last words.
+// On the chip, m of the water cells on block faces (on quads, on the faces between workgroups;
+// inside one m goes through LDS) is published as tagged words and read by the neighbours while the
+// iteration's reduction completes, so the halo exchange costs no wait of its own. A replacement
+// exchanges x, u, p and q in turn, all faces by words. Halo words are numbered
+// 8 t + k (t the iteration's reduction tag; k = 0 for m, 1..4 for x, u, p, q of a replacement; u0
+// at the start has 8 t + 5 with t the start's reduction) and alternate between two word buffers:
+// m of reduction t and u and q of its replacement in buffer t & 1, x and p in the
+// other, u0 in the start's. A wave rewrites a buffer only after a reduction or an exchange that
+// every neighbour joins after it has read the buffer's last words.
 
 // The pipelined iteration's scalars from the reduction's (r, u), (w, u), (r, r); returns
 // whether to update (false once (r, r) meets the tolerance or limits.z updates ran).
@@ -3137,7 +3129,10 @@ __device__ __noinline__ void solve_pipe_memory(const Dev* dp, SolveSpan sp, uint
   float* const cM[2] = {d.pcg + 2u * capc, d.pcg + 3u * capc};
   const float* const p0 = start_pressure(d);
   for_blocks<SOLVE_WAVES>(d, b0, b1, SOLVE_WAVES, [&](uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk) {
-    init_cell<double>(d, b, lane, lx, ly, lz, lk, nullptr, 0u, d.part + b * 4u, p0);
+    const uint32_t cell = b * 64u + lane;
+    const bool water = (d.nbm[cell] & 64u) != 0u;
+    start_cell<double>(d, cell, lane, lx, ly, lz, water, water ? cDiag[cell] : 1.0f, water ? cR[cell] : 0.0f,
+                       water ? d.bvec[cell] : 0.0f, nullptr, 0u, d.part + b * 4u);
   });
   double tt[4];
   SolveScalars<double> s;
@@ -3257,157 +3252,110 @@ __device__ __noinline__ void solve_pipe_memory(const Dev* dp, SolveSpan sp, uint
   solve_finish<double>(d, sp, tag, s);
 }
 
-template <class L>
-__global__ __launch_bounds__(SOLVE_THREADS) void k_solve_pipe(L l) {
-  const auto v = view(l);
-  const Dev& d = v.d;
-  constexpr uint32_t RM = SOLVE_RMAX;
-  if (d.st->dt_ns == 0u) return;
-  // A test of the plain launch's failure path: the last workgroup stays out, as one that is not
-  // resident would, and the others' bounded waits abort the solve.
-  if constexpr (std::is_same<L, One>::value) {
-    if (d.solve_plain == 2u && v.wg + 1u == v.wgs) return;
-  }
-  if (__hip_atomic_load(d.bar + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
-  const SolveSpan sp = solve_span(v, SOLVE_WAVES * SOLVE_RMAX, false);
-  uint32_t tag = __hip_atomic_load(d.bar + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (!sp.in_regs) {
-    solve_pipe_memory(d.self, sp, tag);
-    return;
-  }
-
-  // Register form. Wave wv holds blocks b0 + wv + SOLVE_WAVES r (r < RM). Per block and lane:
-  // x, r, u, w, z, q, s, p, m, diag and the neighbour mask; per axis the tagged word of the
-  // halo cell across the block face (when it is water) as last loaded.
+// One block a wave, one cell a lane (workgroups of at most 16 blocks): x, r, u, w, z, q, s, p, m,
+// diag and the neighbour mask; per axis the tagged word of the halo cell across the block face
+// (when it is water) as last loaded.
+__device__ __forceinline__ void solve_pipe_blocks(const Dev& d, const SolveSpan& sp, uint32_t tag) {
   const uint32_t mode = d.sc->precond;
-  const uint32_t b0 = sp.b0, b1 = sp.b1;
   const uint32_t capc = d.capc;
   const float* const p0 = start_pressure(d);
   unsigned long long* const hz = d.hz;
-  __shared__ LPart<double> lp;
+  LPart<double>& lp = part_lds<double>();
+  __shared__ uint32_t lkr[SOLVE_WAVES][27];
+  const uint32_t wv = threadIdx.x >> 6, ln = lane_id();
+  const int lx = (int)(ln >> 4), ly = (int)((ln >> 2) & 3u), lz = (int)(ln & 3u);
+  const uint32_t b = sp.b0 + wv, cell = b * 64u + ln;
+  const bool holds = b < sp.b1;
   const uint32_t t0 = tag + 1u;  // the start's reduction
   unsigned long long* const hz0 = hz + (size_t)(t0 & 1u) * capc;
-  for_blocks<SOLVE_WAVES>(d, b0, b1, SOLVE_WAVES, [&](uint32_t b, uint32_t lane, int lx, int ly, int lz, const uint32_t* lk) {
+  // The rows are in memory (k_solve_rows).
+  float rX = 0.0f, rR = 0.0f, rU = 0.0f, rW = 0.0f, rZ = 0.0f, rQ = 0.0f, rS = 0.0f, rP = 0.0f, rMv = 0.0f, dg = 1.0f;
+  uint32_t mask = 0;
+  if (holds) {
+    if (ln < 27u) lkr[wv][ln] = d.block_nb[b * 27u + ln];
+    mask = d.nbm[cell];
+  }
+  const bool water = (mask & 64u) != 0u;
+  if (holds) {
+    float bv = 0.0f;
+    if (water) {
+      rX = p0[cell];
+      rR = d.cf[(size_t)NATRAY_F_R * capc + cell];
+      dg = d.cf[(size_t)NATRAY_F_DIAG * capc + cell];
+      bv = d.bvec[cell];
+    }
     double v[4];
-    init_cell<double>(d, b, lane, lx, ly, lz, lk, hz0, 8u * t0 + 5u, v, p0);
-    if (lane == 0)
-      for (uint32_t k = 0; k < 4u; ++k) lp.v[k][b - b0] = v[k];
-  });
+    start_cell<double>(d, cell, ln, lx, ly, lz, water, dg, rR, bv, hz0, 8u * t0 + 5u, v);
+    if (water) rU = d.cf[(size_t)NATRAY_F_Z * capc + cell];
+    if (ln == 0u)
+      for (uint32_t k = 0; k < 4u; ++k) lp.v[k][wv] = v[k];
+  }
   double tt[4];
   SolveScalars<double> s;
   bool go = solve_start<double>(d, tt, reduce<double>(d, sp, ++tag, 4, &lp, tt), s);
   const bool refresh_on = d.sc->refresh_every > 0u;
   const double replace_above = PIPE_REPLACE * (double)d.U->solve[0] * (s.b_norm < 1.0 ? 1.0 : s.b_norm);
 
-  __shared__ uint32_t lkr[SOLVE_WAVES][SOLVE_RMAX][27];
-  const uint32_t wv = threadIdx.x >> 6, ln = lane_id();
-  const int lx = (int)(ln >> 4), ly = (int)((ln >> 2) & 3u), lz = (int)(ln & 3u);
   const uint32_t face_bit[3] = {lx == 0 ? 1u : (lx == 3 ? 2u : 0u), ly == 0 ? 4u : (ly == 3 ? 8u : 0u),
                                 lz == 0 ? 16u : (lz == 3 ? 32u : 0u)};
-  float rX[RM], rR[RM], rU[RM], rW[RM], rZ[RM], rQ[RM], rS[RM], rP[RM], rMv[RM], rDg[RM];
-  uint32_t rM[RM];
-  unsigned long long hW[RM][3];
-  auto halo_cell = [&](uint32_t r, int a) -> uint32_t {
+  unsigned long long hW[3] = {0ull, 0ull, 0ull};
+  auto halo_cell = [&](int a) -> uint32_t {
     const int sg = (face_bit[a] & 0x2Au) ? 1 : -1;
-    return nbr(lkr[wv][r], lx, ly, lz, a == 0 ? sg : 0, a == 1 ? sg : 0, a == 2 ? sg : 0);
+    return nbr(lkr[wv], lx, ly, lz, a == 0 ? sg : 0, a == 1 ? sg : 0, a == 2 ? sg : 0);
   };
-  auto has_halo = [&](uint32_t r, int a) -> bool { return (rM[r] & face_bit[a]) != 0u; };
-#pragma unroll
-  for (uint32_t r = 0; r < RM; ++r) {
-    const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-    if (b < b1 && ln < 27) lkr[wv][r][ln] = d.block_nb[b * 27u + ln];
-  }
-  __syncthreads();
-#pragma unroll
-  for (uint32_t r = 0; r < RM; ++r) {
-    rX[r] = rR[r] = rU[r] = rW[r] = rZ[r] = rQ[r] = rS[r] = rP[r] = rMv[r] = 0.0f;
-    rDg[r] = 1.0f;
-    rM[r] = 0;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) hW[r][a] = 0ull;
-    const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-    if (b >= b1) continue;
-    const uint32_t cell = b * 64u + ln;
-    rM[r] = d.nbm[cell];
-    if (rM[r] & 64u) {
-      rX[r] = p0[cell];
-      rR[r] = d.cf[(size_t)NATRAY_F_R * capc + cell];
-      rU[r] = d.cf[(size_t)NATRAY_F_Z * capc + cell];
-      rDg[r] = d.cf[(size_t)NATRAY_F_DIAG * capc + cell];
-    }
-  }
+  auto has_halo = [&](int a) -> bool { return (mask & face_bit[a]) != 0u; };
   bool ok = true;
-  // The halo of word buffer `buf` with tag `want` for block r: waits for each halo word and
-  // returns the payloads (0 where there is no halo cell).
-  auto halo = [&](uint32_t r, const unsigned long long* buf, uint32_t want, float h[3]) {
+  // The halo of word buffer `buf` with tag `want`: waits for each halo word and returns the
+  // payloads (0 where there is no halo cell).
+  auto halo = [&](const unsigned long long* buf, uint32_t want, float h[3]) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       h[a] = 0.0f;
-      if (!has_halo(r, a)) continue;
-      ok = wait_word(d, hW[r][a], &buf[halo_cell(r, a)], want) && ok;
-      h[a] = __uint_as_float((uint32_t)hW[r][a]);
+      if (!has_halo(a)) continue;
+      ok = wait_word(d, hW[a], &buf[halo_cell(a)], want) && ok;
+      h[a] = __uint_as_float((uint32_t)hW[a]);
     }
   };
-  // Publishes vals of this wave's water cells into buffer `buf` with tag `tg`.
-  auto publish = [&](const float* vals, unsigned long long* buf, uint32_t tg) {
-#pragma unroll
-    for (uint32_t r = 0; r < RM; ++r) {
-      const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-      if (b < b1 && (rM[r] & 64u)) store_word(&buf[b * 64u + ln], tag_word(tg, __float_as_uint(vals[r])));
-    }
+  // Publishes the water cells' values into buffer `buf` with tag `tg`.
+  auto publish = [&](float val, unsigned long long* buf, uint32_t tg) {
+    if (water) store_word(&buf[cell], tag_word(tg, __float_as_uint(val)));
   };
-  if (go) {
-    // w = A u from u0 and its halo (published by init_cell with the start's reduction).
-#pragma unroll
-    for (uint32_t r = 0; r < RM; ++r) {
-      const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-      if (b >= b1) continue;
-      float h[3];
-      halo(r, hz0, 8u * t0 + 5u, h);
-      const float w = apply_row(rU[r], rDg[r], rM[r], h, lx, ly, lz);
-      if (rM[r] & 64u) rW[r] = w;
-    }
+  if (go && holds) {
+    // w = A u from u0 and its halo (published with the start's reduction).
+    float h[3];
+    halo(hz0, 8u * t0 + 5u, h);
+    const float w = apply_row(rU, dg, mask, h, lx, ly, lz);
+    if (water) rW = w;
   }
-  __shared__ RedLds<double> rl;
+  RedLds<double>& rl = red_lds<double>();
   while (go) {
     const uint32_t T = tag + 1u;  // this iteration's reduction
     unsigned long long* const hzT = hz + (size_t)(T & 1u) * capc;
     // The block partials of (r, u), (w, u) and (r, r), published at once.
-#pragma unroll
-    for (uint32_t r = 0; r < RM; ++r) {
-      const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-      if (b >= b1) continue;
-      const double v0 = wave_tree<double>(prod<double>(rR[r], rU[r])), v1 = wave_tree<double>(prod<double>(rW[r], rU[r])),
-                   v2 = wave_tree<double>(prod<double>(rR[r], rR[r]));
-      if (ln == 0) {
-        lp.v[0][b - b0] = v0;
-        lp.v[1][b - b0] = v1;
-        lp.v[2][b - b0] = v2;
+    if (holds) {
+      const double v0 = wave_tree<double>(prod<double>(rR, rU)), v1 = wave_tree<double>(prod<double>(rW, rU)),
+                   v2 = wave_tree<double>(prod<double>(rR, rR));
+      if (ln == 0u) {
+        lp.v[0][wv] = v0;
+        lp.v[1][wv] = v1;
+        lp.v[2][wv] = v2;
       }
     }
     reduce_publish<double>(d, sp, ++tag, 3, &lp, rl);
     // While the other workgroups' chunks arrive: m = M^-1 w, published for the neighbours.
-#pragma unroll
-    for (uint32_t r = 0; r < RM; ++r) {
-      const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-      if (b >= b1) continue;
-      const bool water = (rM[r] & 64u) != 0u;
-      const float m = precondition(rW[r], rDg[r], water, lx, ly, lz, mode);
-      rMv[r] = water ? m : 0.0f;
+    if (holds) {
+      const float m = precondition(rW, dg, water, lx, ly, lz, mode);
+      rMv = water ? m : 0.0f;
+      publish(rMv, hzT, 8u * T);
     }
-    publish(rMv, hzT, 8u * T);
     // The halo m words, polled while the reduction completes.
     auto halo_poll = [&](uint32_t) -> bool {
       bool fresh = true;
 #pragma unroll
-      for (uint32_t r = 0; r < RM; ++r) {
-        if (b0 + wv + SOLVE_WAVES * r >= b1) continue;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          if (!has_halo(r, a) || (uint32_t)(hW[r][a] >> 32) == 8u * T) continue;
-          hW[r][a] = load_word(&hzT[halo_cell(r, a)]);
-          fresh = fresh && (uint32_t)(hW[r][a] >> 32) == 8u * T;
-        }
+      for (int a = 0; a < 3; ++a) {
+        if (!has_halo(a) || (uint32_t)(hW[a] >> 32) == 8u * T) continue;
+        hW[a] = load_word(&hzT[halo_cell(a)]);
+        fresh = fresh && (uint32_t)(hW[a] >> 32) == 8u * T;
       }
       return fresh;
     };
@@ -3415,103 +3363,358 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_solve_pipe(L l) {
     if (!pipe_scalars(d, tt, s)) break;
     const float fa = (float)s.alpha, fb = (float)s.beta;
     const bool refresh = refresh_on && (s.iters + 1u) % d.sc->refresh_every == 0u && s.r_norm > replace_above;
-#pragma unroll
-    for (uint32_t r = 0; r < RM; ++r) {
-      const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-      if (b >= b1) continue;
+    if (holds) {
       float hm[3];
 #pragma unroll
-      for (int a = 0; a < 3; ++a) hm[a] = has_halo(r, a) ? __uint_as_float((uint32_t)hW[r][a]) : 0.0f;
-      const float n = apply_row(rMv[r], rDg[r], rM[r], hm, lx, ly, lz);
-      if (rM[r] & 64u) {
-        rZ[r] = n + fb * rZ[r];
-        rQ[r] = rMv[r] + fb * rQ[r];
-        rS[r] = rW[r] + fb * rS[r];
-        rP[r] = rU[r] + fb * rP[r];
-        rX[r] = rX[r] + fa * rP[r];
-        rR[r] = rR[r] - fa * rS[r];
-        rU[r] = rU[r] - fa * rQ[r];
-        rW[r] = rW[r] - fa * rZ[r];
+      for (int a = 0; a < 3; ++a) hm[a] = has_halo(a) ? __uint_as_float((uint32_t)hW[a]) : 0.0f;
+      const float n = apply_row(rMv, dg, mask, hm, lx, ly, lz);
+      if (water) {
+        rZ = n + fb * rZ;
+        rQ = rMv + fb * rQ;
+        rS = rW + fb * rS;
+        rP = rU + fb * rP;
+        rX = rX + fa * rP;
+        rR = rR - fa * rS;
+        rU = rU - fa * rQ;
+        rW = rW - fa * rZ;
       }
     }
     s.iters += 1u;
-    if (refresh) {
+    if (refresh && holds) {
       // Residual replacement through four halo exchanges: x (r = b - A x in double, u = M^-1 r),
       // u (w = A u), p (s = A p, q = M^-1 s), q (z = A q); x and p in the buffer m of this
       // iteration is not in, u and q in the other.
       unsigned long long* const hzA = hz + (size_t)((T + 1u) & 1u) * capc;
+      float h[3];
       publish(rX, hzA, 8u * T + 1u);
-#pragma unroll
-      for (uint32_t r = 0; r < RM; ++r) {
-        const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-        if (b >= b1) continue;
-        const uint32_t cell = b * 64u + ln, mask = rM[r];
-        const bool water = (mask & 64u) != 0u;
-        float h[3];
-        halo(r, hzA, 8u * T + 1u, h);
-        const Faces f = block_faces(rX[r]);
-        if (water) {
-          double ap = (double)rDg[r] * (double)rX[r];
-          if (mask & 1u) ap -= (double)(lx > 0 ? f.xm : h[0]);
-          if (mask & 2u) ap -= (double)(lx < 3 ? f.xp : h[0]);
-          if (mask & 4u) ap -= (double)(ly > 0 ? f.ym : h[1]);
-          if (mask & 8u) ap -= (double)(ly < 3 ? f.yp : h[1]);
-          if (mask & 16u) ap -= (double)(lz > 0 ? f.zm : h[2]);
-          if (mask & 32u) ap -= (double)(lz < 3 ? f.zp : h[2]);
-          rR[r] = (float)((double)d.bvec[cell] - ap);
-        }
-        const float u = precondition(rR[r], rDg[r], water, lx, ly, lz, mode);
-        if (water) rU[r] = u;
+      halo(hzA, 8u * T + 1u, h);
+      const Faces f = block_faces(rX);
+      if (water) {
+        double ap = (double)dg * (double)rX;
+        if (mask & 1u) ap -= (double)(lx > 0 ? f.xm : h[0]);
+        if (mask & 2u) ap -= (double)(lx < 3 ? f.xp : h[0]);
+        if (mask & 4u) ap -= (double)(ly > 0 ? f.ym : h[1]);
+        if (mask & 8u) ap -= (double)(ly < 3 ? f.yp : h[1]);
+        if (mask & 16u) ap -= (double)(lz > 0 ? f.zm : h[2]);
+        if (mask & 32u) ap -= (double)(lz < 3 ? f.zp : h[2]);
+        rR = (float)((double)d.bvec[cell] - ap);
       }
+      const float u = precondition(rR, dg, water, lx, ly, lz, mode);
+      if (water) rU = u;
       publish(rU, hzT, 8u * T + 2u);
-#pragma unroll
-      for (uint32_t r = 0; r < RM; ++r) {
-        if (b0 + wv + SOLVE_WAVES * r >= b1) continue;
-        float h[3];
-        halo(r, hzT, 8u * T + 2u, h);
-        const float w = apply_row(rU[r], rDg[r], rM[r], h, lx, ly, lz);
-        if (rM[r] & 64u) rW[r] = w;
-      }
+      halo(hzT, 8u * T + 2u, h);
+      const float w = apply_row(rU, dg, mask, h, lx, ly, lz);
+      if (water) rW = w;
       publish(rP, hzA, 8u * T + 3u);
-#pragma unroll
-      for (uint32_t r = 0; r < RM; ++r) {
-        if (b0 + wv + SOLVE_WAVES * r >= b1) continue;
-        const bool water = (rM[r] & 64u) != 0u;
-        float h[3];
-        halo(r, hzA, 8u * T + 3u, h);
-        const float sv = apply_row(rP[r], rDg[r], rM[r], h, lx, ly, lz);
-        if (water) rS[r] = sv;
-        const float q = precondition(rS[r], rDg[r], water, lx, ly, lz, mode);
-        if (water) rQ[r] = q;
-      }
+      halo(hzA, 8u * T + 3u, h);
+      const float sv = apply_row(rP, dg, mask, h, lx, ly, lz);
+      if (water) rS = sv;
+      const float q = precondition(rS, dg, water, lx, ly, lz, mode);
+      if (water) rQ = q;
       publish(rQ, hzT, 8u * T + 4u);
-#pragma unroll
-      for (uint32_t r = 0; r < RM; ++r) {
-        if (b0 + wv + SOLVE_WAVES * r >= b1) continue;
-        float h[3];
-        halo(r, hzT, 8u * T + 4u, h);
-        const float z = apply_row(rQ[r], rDg[r], rM[r], h, lx, ly, lz);
-        if (rM[r] & 64u) rZ[r] = z;
-      }
+      halo(hzT, 8u * T + 4u, h);
+      const float z = apply_row(rQ, dg, mask, h, lx, ly, lz);
+      if (water) rZ = z;
     }
   }
   // The fields the other kernels and the host read.
-#pragma unroll
-  for (uint32_t r = 0; r < RM; ++r) {
-    const uint32_t b = b0 + wv + SOLVE_WAVES * r;
-    if (b < b1 && (rM[r] & 64u)) {
-      const uint32_t cell = b * 64u + ln;
-      d.cf[(size_t)NATRAY_F_P * capc + cell] = rX[r];
-      d.cf[(size_t)NATRAY_F_R * capc + cell] = rR[r];
-      d.cf[(size_t)NATRAY_F_Z * capc + cell] = rU[r];
-      if (s.iters > 0u) {
-        d.cf[(size_t)NATRAY_F_Q * capc + cell] = rS[r];
-        d.cf[(size_t)NATRAY_F_D * capc + cell] = rP[r];
-        d.cf[(size_t)(NATRAY_F_D + 1u) * capc + cell] = rW[r];
-      }
+  if (water) {
+    d.cf[(size_t)NATRAY_F_P * capc + cell] = rX;
+    d.cf[(size_t)NATRAY_F_R * capc + cell] = rR;
+    d.cf[(size_t)NATRAY_F_Z * capc + cell] = rU;
+    if (s.iters > 0u) {
+      d.cf[(size_t)NATRAY_F_Q * capc + cell] = rS;
+      d.cf[(size_t)NATRAY_F_D * capc + cell] = rP;
+      d.cf[(size_t)(NATRAY_F_D + 1u) * capc + cell] = rW;
     }
   }
   solve_finish<double>(d, sp, tag, s);
+}
+
+// One set of quads a wave, as solve_quads with one set: r, u, w and m in registers, the vectors an
+// iteration touches once (x, z, s, p and q) in LDS, since all of them in registers spilled (12 us
+// an iteration at 1,594 blocks, 9.4 so).
+__device__ __forceinline__ void solve_pipe_quads(const Dev& d, const SolveSpan& sp, uint32_t tag) {
+  struct Lds {
+    float4 d[SOLVE_WAVES * 4u][16];  // m (u at the start) of the workgroup's cells
+    float4 f[5][SOLVE_WAVES * 4u][16];  // x, z, s, p and q
+    float2 diag[8];
+  };
+  __shared__ Lds lds;
+  LPart<double>& lp = part_lds<double>();
+  const uint32_t mode = d.sc->precond, b0 = sp.b0, b1 = sp.b1, capc = d.capc;
+  const uint32_t wv = threadIdx.x >> 6;
+  const QuadLane l = quad_lane();
+  const float* const p0 = start_pressure(d);
+  const __amdgpu_buffer_rsrc_t w0 = face_rsrc(d, 0u, sp.n), w1 = face_rsrc(d, 1u, sp.n);
+  auto words = [&](uint32_t t) { return (t & 1u) ? w1 : w0; };
+  // The diagonal, as in solve_quads.
+  float kc;
+  {
+    const float h = d.U->origin[3], cs = d.U->gravity[3] * dt_of(d);
+    kc = h * h / (cs * cs);
+  }
+  const bool fast = DivGuard::divisor(kc) && DivGuard::divisor(kc + 6.0f);
+  if (threadIdx.x < 8u) {
+    float dg = kc;
+    for (uint32_t k = 0; k < threadIdx.x; ++k) dg += 1.0f;
+    lds.diag[threadIdx.x] = make_float2(dg, 1.0f / dg);
+  }
+  __syncthreads();
+
+  const uint32_t pl = 4u * wv + l.q, b = b0 + pl, cell0 = b * 64u + l.col * 4u;
+  const bool sets = b0 + 4u * wv < b1, valid = b < b1;
+  float rR[4] = {}, rU[4] = {}, rW[4] = {}, rMv[4] = {};
+  uint32_t m = 0, w = 0;
+  QuadLinks lk = {NONE, NONE, NONE, NONE};
+  auto is = [&](int k) -> bool { return (m >> k & 1u) != 0u; };
+  auto keep = [&](float4& at, const float* v) { at = make_float4(v[0], v[1], v[2], v[3]); };
+  enum { FX, FZ, FS, FP, FQ };
+  auto get = [&](int f, float* v) {
+    const float4 o = lds.f[f][pl][l.col];
+    v[0] = o.x, v[1] = o.y, v[2] = o.z, v[3] = o.w;
+  };
+  auto put = [&](int f, const float* v) { keep(lds.f[f][pl][l.col], v); };
+  auto precondition4 = [&](const float* r, float* z) {
+    float g[4], y[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float2 e = lds.diag[m >> (8 + 3 * k) & 7u];
+      g[k] = e.x, y[k] = e.y;
+    }
+    precondition_quad(r, g, y, fast, m, l, mode, z);
+  };
+  auto diagonal = [&](float* g) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) g[k] = lds.diag[m >> (8 + 3 * k) & 7u].x;
+  };
+  auto part = [&](int k, double v) {
+    if (l.col == 0u && valid) lp.v[k][pl] = v;
+  };
+  auto dot = [&](const float* a, const float* c) -> double {
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = prod<double>(a[k], c[k]);
+    return quad_tree<double>(v);
+  };
+  // The halo inside the workgroup, from LDS, as solve_quads takes its directions.
+  auto near = [&](QuadHalo& h) {
+    auto get4 = [&](uint32_t at, float* hv) {
+      const float4 o = lds.d[at][l.col];
+      hv[0] = o.x, hv[1] = o.y, hv[2] = o.z, hv[3] = o.w;
+    };
+    if ((w & 15u) && !(w >> 10 & 1u)) get4(lk.x, h.x);
+    if ((w & 240u) && !(w >> 11 & 1u)) get4(lk.y, h.y);
+    if ((w & 256u) && !(w >> 12 & 1u)) h.zm = reinterpret_cast<const float*>(&lds.d[lk.m][l.col])[l.odd ? 1 : 3];
+    if ((w & 512u) && !(w >> 13 & 1u)) h.zp = reinterpret_cast<const float*>(&lds.d[lk.p][l.col])[l.odd ? 2 : 0];
+  };
+  // o = A v on the water cells, 0 elsewhere.
+  auto row = [&](const float* v, const QuadHalo& h, float* o) {
+    float g[4], n[4];
+    diagonal(g);
+    quad_row<float>(v, g, h, l, n);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = is(k) ? n[k] : 0.0f;
+  };
+  const uint32_t t0 = tag + 1u;  // the start's reduction
+  if (sets) {
+    uint32_t nb[6] = {NONE, NONE, NONE, NONE, NONE, NONE};
+    if (valid) {
+#pragma unroll
+      for (uint32_t f = 0; f < 6u; ++f) {
+        const uint32_t step = f < 2u ? 9u : (f < 4u ? 3u : 1u);
+        const uint32_t n = d.block_nb[(size_t)b * 27u + ((f & 1u) ? 13u + step : 13u - step)];
+        nb[f] = n == NONE ? NONE : (n >= b0 && n < b1 ? n - b0 : n | QUAD_FAR);
+      }
+    }
+    lk = {l.x3 ? nb[0] : (l.x0 ? nb[1] : NONE), l.y3 ? nb[2] : (l.y0 ? nb[3] : NONE), nb[4], nb[5]};
+    m = quad_mask(d, cell0, valid, l);
+    w = quad_flags(d, nb, lk, l, b0, b1);
+    float bv[4] = {}, x[4] = {};
+    if (valid) {
+      quad_load(d.cf + (size_t)NATRAY_F_R * capc, cell0, l.odd, rR);
+      quad_load(d.bvec, cell0, l.odd, bv);
+      quad_load(p0, cell0, l.odd, x);
+    }
+    uint32_t nw = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (!is(k)) x[k] = rR[k] = bv[k] = 0.0f;
+      nw += (uint32_t)__popcll(__ballot(is(k)) >> (16u * l.q) & 0xffffull);
+    }
+    const float zero[4] = {};
+    put(FX, x);
+    put(FZ, zero);
+    put(FS, zero);
+    put(FP, zero);
+    put(FQ, zero);
+    precondition4(rR, rU);
+    quad_publish(words(t0), b, rU, w >> 14 & 15u, l, 8u * t0 + 5u);
+    keep(lds.d[pl][l.col], rU);
+    part(0, dot(rR, rU));
+    part(1, dot(rR, rR));
+    part(2, dot(bv, bv));
+    part(3, (double)nw);
+  }
+  double tt[4];
+  SolveScalars<double> s;
+  bool go = solve_start<double>(d, tt, reduce<double>(d, sp, ++tag, 4, &lp, tt), s);
+  const bool refresh_on = d.sc->refresh_every > 0u;
+  const double replace_above = PIPE_REPLACE * (double)d.U->solve[0] * (s.b_norm < 1.0 ? 1.0 : s.b_norm);
+
+  auto id = [&](uint32_t link) -> uint32_t { return (link & QUAD_FAR) ? link & ~QUAD_FAR : b0 + link; };
+  const QuadLinks far = {lk.x & ~QUAD_FAR, lk.y & ~QUAD_FAR, lk.m & ~QUAD_FAR, lk.p & ~QUAD_FAR};
+  bool ok = true;
+  // Waits for the halo of buffer t with tag tg from the blocks k.
+  auto await = [&](uint32_t t, const QuadLinks& k, uint32_t want, uint32_t tg, QuadHalo& h) {
+    QuadWords q{};
+    ok = quad_wait(d, words(t), k, want, l, tg, q, quad_had(want)) && ok;
+    quad_payload(q, want, l.odd, h);
+  };
+  if (go && sets) {
+    // w = A u from u0 and its halo.
+    QuadHalo h;
+    await(t0, far, quad_want(w, true), 8u * t0 + 5u, h);
+    near(h);
+    row(rU, h, rW);
+  }
+  RedLds<double>& rl = red_lds<double>();
+  while (go) {
+    const uint32_t T = tag + 1u;  // this iteration's reduction
+    if (sets) {
+      part(0, dot(rR, rU));
+      part(1, dot(rW, rU));
+      part(2, dot(rR, rR));
+    }
+    reduce_publish<double>(d, sp, ++tag, 3, &lp, rl);
+    // While the other workgroups' chunks arrive: m = M^-1 w, published for the neighbours, and
+    // their m's words.
+    if (sets) {
+      precondition4(rW, rMv);
+      quad_publish(words(T), b, rMv, w >> 14 & 15u, l, 8u * T);
+      keep(lds.d[pl][l.col], rMv);
+    }
+    QuadWords q{};
+    QuadHalo h{};
+    const uint32_t want = quad_want(w, true);
+    uint32_t have = quad_had(want);
+    auto halo_m = [&](uint32_t) -> bool { return quad_words(words(T), far, want, l, 8u * T, q, have); };
+    if (!reduce_wait<double>(d, sp, tag, 3, tt, rl, halo_m) || !ok) break;
+    quad_payload(q, want, l.odd, h);
+    if (!pipe_scalars(d, tt, s)) break;
+    const float fa = (float)s.alpha, fb = (float)s.beta;
+    const bool refresh = refresh_on && (s.iters + 1u) % d.sc->refresh_every == 0u && s.r_norm > replace_above;
+    if (sets) {
+      near(h);
+      float n[4], v[4], x[4];
+      row(rMv, h, n);
+      // z = n + beta z, w -= alpha z, and so on; 0 stays 0 off water.
+      auto step = [&](int f, const float* a, float* r) {
+        get(f, v);
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (is(k)) {
+            v[k] = a[k] + fb * v[k];
+            r[k] = r[k] - fa * v[k];
+          }
+        put(f, v);
+      };
+      get(FP, v);
+      get(FX, x);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (is(k)) {
+          v[k] = rU[k] + fb * v[k];
+          x[k] = x[k] + fa * v[k];
+        }
+      put(FP, v);
+      put(FX, x);
+      step(FS, rW, rR);
+      step(FQ, rMv, rU);
+      step(FZ, n, rW);
+    }
+    s.iters += 1u;
+    if (refresh && sets) {
+      // Residual replacement through four halo exchanges: x (r = b - A x in double, u = M^-1 r),
+      // u (w = A u), p (s = A p, q = M^-1 s), q (z = A q); x and p in the buffer m of this
+      // iteration is not in, u and q in the other.
+      const QuadLinks ids = {id(lk.x), id(lk.y), id(lk.m), id(lk.p)};
+      auto exchange = [&](const float* v, uint32_t t, uint32_t tg) {
+        quad_publish(words(t), b, v, w >> 18 & 15u, l, tg);
+        await(t, ids, quad_want(w, false), tg, h);
+      };
+      float v[4], o[4], g[4], bv[4] = {};
+      double ap[4];
+      get(FX, v);
+      exchange(v, T + 1u, 8u * T + 1u);
+      if (m & 15u) quad_load(d.bvec, cell0, l.odd, bv);
+      diagonal(g);
+      quad_row<double>(v, g, h, l, ap);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) rR[k] = is(k) ? (float)((double)bv[k] - ap[k]) : 0.0f;
+      precondition4(rR, rU);
+      exchange(rU, T, 8u * T + 2u);
+      row(rU, h, rW);
+      get(FP, v);
+      exchange(v, T + 1u, 8u * T + 3u);
+      row(v, h, o);
+      put(FS, o);
+      precondition4(o, v);
+      put(FQ, v);
+      exchange(v, T, 8u * T + 4u);
+      row(v, h, o);
+      put(FZ, o);
+    }
+  }
+  // The fields the other kernels and the host read.
+  if (sets) {
+    auto field = [&](uint32_t f) -> float* { return d.cf + (size_t)f * capc; };
+    float v[4];
+    get(FX, v);
+    quad_store(field(NATRAY_F_P), cell0, l.odd, v, m);
+    quad_store(field(NATRAY_F_R), cell0, l.odd, rR, m);
+    quad_store(field(NATRAY_F_Z), cell0, l.odd, rU, m);
+    if (s.iters > 0u) {
+      get(FS, v);
+      quad_store(field(NATRAY_F_Q), cell0, l.odd, v, m);
+      get(FP, v);
+      quad_store(field(NATRAY_F_D), cell0, l.odd, v, m);
+      quad_store(field(NATRAY_F_D + 1u), cell0, l.odd, rW, m);
+    }
+  }
+  solve_finish<double>(d, sp, tag, s);
+}
+
+template <class L>
+__global__ __launch_bounds__(SOLVE_THREADS) void k_solve_pipe(L l) {
+  const auto v = view(l);
+  const Dev& d = v.d;
+  if (d.st->dt_ns == 0u) return;
+  // A test of the plain launch's failure path: the last workgroup stays out, as one that is not
+  // resident would, and the others' bounded waits abort the solve.
+  if constexpr (std::is_same<L, One>::value) {
+    if (d.solve_plain == 2u && v.wg + 1u == v.wgs) return;
+  }
+  if (__hip_atomic_load(d.bar + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
+  SolveSpan sp = solve_span(v, SOLVE_WAVES * 4u, false);
+  const uint32_t tag = (uint32_t)__builtin_amdgcn_readfirstlane(
+      (int)__hip_atomic_load(d.bar + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  if (!sp.in_regs) {
+    solve_pipe_memory(d.self, sp, tag);
+    return;
+  }
+  // A workgroup without a chunk has nothing to do; the one with the first chunk leads.
+  if (sp.c0 == sp.c1 && (sp.m != 0u || v.wg != 0u)) return;
+  sp.lead = sp.c0 == 0u;
+  // A wave of its own for each block while there are enough waves: the iteration is then a chain of
+  // one cell's work a lane, of which quads have four (in double, the dots and the scalars, most of
+  // all). us an iteration, one block a wave and quads: 1,594 blocks in 256 workgroups 6.9 and 9.4,
+  // 2,946 8.1 and 9.4. Two blocks a wave took 11.5 at 5,657 blocks, where quads take 9.7, and from
+  // memory 12,482 blocks took 54, on quads 12.6.
+  if ((sp.m + sp.G - 1u) / sp.G * sp.K <= SOLVE_WAVES)
+    solve_pipe_blocks(d, sp, tag);
+  else
+    solve_pipe_quads(d, sp, tag);
 }
 
 // ---- learned warm start of the solve ---------------------------------------------------------------
@@ -5547,7 +5750,7 @@ int launch_solve(const Target& t, void* stream, int kind) {
   void* args_one[] = {&one};
   void* args_many[] = {&many};
   const void* fn;
-  if (kind != (int)NATRAY_CG_PIPELINED) NATRAY_LAUNCH(k_solve_rows, LK_WAVES, 256, t, S(stream));
+  NATRAY_LAUNCH(k_solve_rows, LK_WAVES, 256, t, S(stream));
   if (kind == (int)NATRAY_CG_PIPELINED)
     fn = t.d ? (const void*)k_solve_pipe<One> : (const void*)k_solve_pipe<Many>;
   else if (kind == (int)NATRAY_CG_MIXED)

@@ -96,3 +96,31 @@ def test_few_iterations(iters, groups):
     own start after a single iteration, are among the fields compared."""
     s = scenes.balloon_impact(side=64, n=32768, seed=2, iters=iters, capacity=4096)
     solve_and_compare(s, groups)
+
+
+@pytest.mark.parametrize("refresh", [0, 3])
+@pytest.mark.parametrize("n,side,groups,per_group", [
+    (32768, 64, 1, (65, 256)),
+    (32768, 64, 3, (1, 64)),
+    (32768, 64, 59, (1, 64)),
+    (262144, 128, 8, (65, 256)),
+    (262144, 128, 16, (60, 64)),
+    (262144, 128, 200, (1, 64)),
+])
+def test_pipelined_forms(n, side, groups, per_group, refresh):
+    """The pipelined solve holds at most 64 blocks a workgroup on the chip and walks larger counts
+    from memory; with replacements of the residual and without."""
+    s = scenes.balloon_impact(side=side, n=n, seed=groups + 1, iters=400, capacity=4096, precision=abi.CG_PIPELINED,
+                              refresh_every=refresh)
+    blocks = solve_and_compare(s, groups)
+    assert per_group[0] <= -(-blocks // groups) <= per_group[1]
+
+
+def test_pipelined_ragged_blocks_and_few():
+    rng = np.random.default_rng(3)
+    for count in (1, 9, 120):
+        P = helpers.records(rng.uniform(0.2, 0.8, (count, 3)), vel=rng.uniform(-2, 2, (count, 3)))
+        for precond in (abi.PRECOND_BLOCK_SGS, abi.PRECOND_JACOBI):
+            for iters in (1, 40):
+                solve_and_compare(helpers.box_scene(P, side=32, precond=precond, gravity=9.81, precision=abi.CG_PIPELINED,
+                                                    iters=iters), 7)
