@@ -1081,10 +1081,10 @@ __global__ __launch_bounds__(256) void k_grid_prep(L l) {
 
 // ---- pressure solve (fluid.wgsl:381-578) ------------------------------------------------------------
 //
-// One cooperative launch runs the whole CG: solve_init, then solve_q .. solve_beta for every
+// k_solve_rows forms the rows; one launch runs the whole CG, solve_q .. solve_beta for every
 // iteration. The n blocks form m = ceil(n / K) chunks of K = ceil(n / MAX_CHUNKS) consecutive
 // blocks (both fixed by n alone, so the sums do not depend on the launch); workgroup g owns
-// the chunks [g m / G, (g + 1) m / G) and their blocks, wave w the blocks b0 + w + 16 r.
+// the chunks [g m / G, (g + 1) m / G) and their blocks.
 //
 // Workgroups talk through 64-bit words that hold a 32-bit tag above a 32-bit payload, stored
 // and loaded with agent-scope relaxed atomics: a reader waits until a word carries the tag
@@ -1096,14 +1096,13 @@ __global__ __launch_bounds__(256) void k_grid_prep(L l) {
 //    order itself, so no workgroup relays for the others. Consecutive reductions alternate
 //    between two word buffers: a workgroup can only publish reduction t + 2 after it has seen
 //    every chunk of t + 1, which every workgroup publishes after it has read all of t.
-//  - Halo z: a wave that keeps its blocks in registers publishes z of its water cells with
-//    the tag of the reduction that follows; neighbours read it in the next solve_q. The other
-//    halo values a block needs (the old direction; p for the residual refresh) are rebuilt by
-//    the reader from values it already holds, with the owner's arithmetic, so they are equal.
-// When the blocks of a workgroup do not fit in registers (a launch with too few workgroups
-// for the block count) every workgroup runs the same iteration on the cf fields in memory,
-// with agent-scope release and acquire fences around each reduction. Both forms evaluate the
-// same expressions in the same order and give the same bits.
+//  - Halo z: a wave publishes z on the faces towards other workgroups with the tag of the
+//    reduction that follows; neighbours read it in the next solve_q. The old direction a halo
+//    cell needs is rebuilt by the reader from values it already holds, with the owner's
+//    arithmetic, so it is equal.
+// Workgroups of at most 256 blocks keep them on the chip (quads, below). Larger ones (a launch
+// with too few workgroups for the block count) run the same iteration on the cf fields in memory.
+// All forms evaluate the same expressions in the same order and give the same bits.
 
 // The pipelined solve replaces its residual only while |r| is above this many times the
 // tolerance test's bound.
@@ -1153,7 +1152,7 @@ __device__ __forceinline__ void store_word(unsigned long long* p, unsigned long 
   __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Workgroup barrier of the register form: orders LDS only, so global stores to other
+// Workgroup barrier of the forms on the chip: orders LDS only, so global stores to other
 // workgroups' words and loads whose results are used later stay in flight across it.
 // `all` makes it a full barrier (global memory too), as the memory form needs.
 __device__ __forceinline__ void wg_sync(bool all) {
@@ -1259,7 +1258,7 @@ struct NoWait {
   __device__ __forceinline__ bool operator()(uint32_t) const { return true; }
 };
 
-// The register form's block partials of one workgroup in LDS, in the reduction's precision and
+// The block partials (forms on the chip) of one workgroup in LDS, in the reduction's precision and
 // component-major: v[k][b - b0]. A block's four components: the reduction's values, or (at the
 // start) r.z, r.r, b.b and its water cells (a count, exact in either precision).
 template <class R>
@@ -1324,7 +1323,7 @@ __device__ __forceinline__ R lane_tree_from(R v, uint32_t off0) {
 
 // Component k of chunk [lo, hi)'s tree sum (the chunk fold: a binary tree over W slots, slot i
 // = block lo + i's partial, zero past the chunk's last block), in lane 0 of the calling wave (all
-// lanes active). The partials come from `lp` (register form) or Dev::part (memory form). Lane l
+// lanes active). The partials come from `lp` (forms on the chip) or Dev::part (memory form). Lane l
 // holds slots l, l + 64, .. and combines them in the tree's order first.
 template <class R>
 __device__ __forceinline__ R chunk_tree(const Dev& d, const SolveSpan& sp, const LPart<R>* lp, uint32_t lo, uint32_t hi,
@@ -1692,7 +1691,7 @@ __device__ __forceinline__ void st_cell(float* f, uint32_t i, float v) {
 // wave wv walks its own blocks b0 + wv + SOLVE_WAVES j with no workgroup barrier, the same
 // blocks in every pass, so a cell's own fields are only ever read back by the wave that wrote
 // them. Values a cell's neighbours in other workgroups need travel as tagged words (tag above
-// the float), as in the register form: z in Dev::hz[cell] with the tag of the reduction after
+// the float), as on quads: z in Dev::hz[cell] with the tag of the reduction after
 // the pass that made it, the new direction in hz[capc (1 + k % 2) + cell] with the tag of
 // iteration k's first reduction, and before a residual refresh p in the other direction buffer
 // (whose last words every neighbour has read) with the tag of the refresh's reduction. A reader
@@ -3050,7 +3049,7 @@ __device__ __forceinline__ bool pipe_scalars(const Dev& d, const double* tt, Sol
   return true;
 }
 
-// (A v) at this lane's cell in register form: diag v minus the water neighbours' v in the order
+// (A v) at this lane's cell of one block a wave: diag v minus the water neighbours' v in the order
 // -x, +x, -y, +y, -z, +z, those across a block face from h (one per axis). Every lane of the
 // wave calls it (block_faces is a wave operation); the result is meaningful on water cells.
 __device__ __forceinline__ float apply_row(float v, float diag, uint32_t mask, const float h[3], int lx, int ly, int lz) {
