@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "natray_dev.h"
+#include "natray_faces.h"
 #include "natray_lanes.h"
 #include "natray_math.h"
 
@@ -2110,14 +2111,8 @@ __device__ __forceinline__ SolveSpan solve_span(const V& v, uint32_t regs, bool 
 // A lane keeps its column in colour order (quad_swap): slots 0, 1 are its red cells ((x + y + z)
 // even) from the bottom up, slots 2, 3 its black ones. A cell's x and y neighbours are then the
 // other colour's slot of the same height in the next lane, and the half sweeps need no selects.
-struct QuadLane {
-  uint32_t ln, q, col;      // lane, block of the set, column 4 x + y
-  bool x0, x3, y0, y3, odd; // odd: the column's red cells are z = 1 and 3
-};
-__device__ __forceinline__ QuadLane quad_lane() {
-  const uint32_t ln = lane_id(), col = ln & 15u, x = col >> 2, y = col & 3u;
-  return {ln, ln >> 4, col, x == 0u, x == 3u, y == 0u, y == 3u, ((x + y) & 1u) != 0u};
-}
+// (QuadLane, and which words a lane exchanges: natray_faces.h.)
+
 // Between z order and colour order (its own inverse).
 template <class T>
 __device__ __forceinline__ void quad_swap(const T* v, T* o, bool odd) {
@@ -2272,48 +2267,12 @@ __device__ __forceinline__ void quad_row(const float* v, const float* dg, const 
 // every neighbour's z read from words by cell, whose z faces are spread over all of a block's
 // lines, the 15.2M impact took 31.9 us per iteration, 9.8 without the halo.)
 constexpr uint32_t FACE_BYTES = 128, FACES_BYTES = 6u * FACE_BYTES;
+static_assert(QUAD_NONE == NONE, "a link without a block");
 // One buffer of face words: z in the first half of Dev::hz, p before a residual refresh in the
 // second.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t face_rsrc(const Dev& d, uint32_t half, uint32_t n) {
   return __builtin_amdgcn_make_buffer_rsrc(d.hz + (size_t)half * (d.capc / 64u) * 96u, 0, (int)(n * FACES_BYTES), 0x00020000);
 }
-// A lane's four halo links: across its x and y faces (lanes at 3 the neighbour below, at 0 the
-// one above, as QuadHalo has them), below and above. Each is a block's place in this workgroup,
-// or QUAD_FAR | a block of another workgroup, or NONE.
-constexpr uint32_t QUAD_FAR = 0x80000000u;
-struct QuadLinks {
-  uint32_t x, y, m, p;
-};
-__device__ __forceinline__ bool quad_far(uint32_t k) { return k != NONE && (k & QUAD_FAR); }
-// A set's face flags, per lane: bits 0..3 and 4..7 the water cells (z order) of the x and y halo
-// columns, 8 and 9 the cells below and above; 10..13 whether x, y, below and above lie in another
-// workgroup; 14..17 whether this lane's own faces (its x face, y face, bottom, top) do, and
-// 18..21 whether they face a block at all.
-__device__ __forceinline__ uint32_t quad_flags(const Dev& d, const uint32_t* nb, const QuadLinks& k, const QuadLane& l,
-                                               uint32_t b0, uint32_t b1) {
-  uint32_t w = 0;
-  auto cells = [](uint4 v) -> uint32_t { return (v.x >> 6 & 1u) | (v.y >> 5 & 2u) | (v.z >> 4 & 4u) | (v.w >> 3 & 8u); };
-  auto id = [&](uint32_t link) -> uint32_t { return (link & QUAD_FAR) ? link & ~QUAD_FAR : b0 + link; };
-  if (k.x != NONE) w |= cells(*reinterpret_cast<const uint4*>(d.nbm + (size_t)id(k.x) * 64u + l.col * 4u));
-  if (k.y != NONE) w |= cells(*reinterpret_cast<const uint4*>(d.nbm + (size_t)id(k.y) * 64u + l.col * 4u)) << 4;
-  if (k.m != NONE) w |= (d.nbm[(size_t)id(k.m) * 64u + l.col * 4u + 3u] >> 6 & 1u) << 8;
-  if (k.p != NONE) w |= (d.nbm[(size_t)id(k.p) * 64u + l.col * 4u] >> 6 & 1u) << 9;
-  w |= (quad_far(k.x) ? 1u << 10 : 0u) | (quad_far(k.y) ? 1u << 11 : 0u) | (quad_far(k.m) ? 1u << 12 : 0u) |
-       (quad_far(k.p) ? 1u << 13 : 0u);
-  const uint32_t own[4] = {l.x0 ? nb[0] : (l.x3 ? nb[1] : NONE), l.y0 ? nb[2] : (l.y3 ? nb[3] : NONE), nb[4], nb[5]};
-#pragma unroll
-  for (uint32_t f = 0; f < 4u; ++f) {
-    if (own[f] != NONE) w |= 1u << (18u + f);
-    if (quad_far(own[f])) w |= 1u << (14u + f);
-  }
-  return w;
-}
-// The halo words to wait for: all, or (far) those of other workgroups.
-__device__ __forceinline__ uint32_t quad_want(uint32_t w, bool far) {
-  if (!far) return w & 0x3ffu;
-  return w & (((w >> 10 & 1u) ? 15u : 0u) | ((w >> 11 & 1u) ? 240u : 0u) | ((w >> 12 & 3u) << 8));
-}
-
 // Tagged halo words of a column as loaded, two per 16-byte record.
 struct QuadWords {
   u32x4 x0, x1, y0, y1;
@@ -2577,7 +2536,7 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
   LPart<R>& lp = part_lds<R>();
   const uint32_t mode = d.sc->precond, b0 = sp.b0, b1 = sp.b1, capc = d.capc;
   const uint32_t wv = threadIdx.x >> 6;
-  QuadLane l = quad_lane();
+  QuadLane l = quad_lane(lane_id());
   float* const cP = d.cf + (size_t)NATRAY_F_P * capc;
   float* const cR = d.cf + (size_t)NATRAY_F_R * capc;
   float* const cZ = d.cf + (size_t)NATRAY_F_Z * capc;
@@ -2725,7 +2684,7 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
     }
     const QuadLinks q = {l.x3 ? nb[0] : (l.x0 ? nb[1] : NONE), l.y3 ? nb[2] : (l.y0 ? nb[3] : NONE), nb[4], nb[5]};
     rM[r] = quad_mask(d, cell0, valid, l);
-    hw[r] = quad_flags(d, nb, q, l, b0, b1);
+    hw[r] = quad_flags(d.nbm, nb, q, l, b0);
     float bv[4] = {0.0f, 0.0f, 0.0f, 0.0f}, d0[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (valid) {
       quad_load(cR, cell0, l.odd, rR[r]);
@@ -2783,7 +2742,7 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
     for (int k = 0; k < 4; ++k)
       if (!(rM[r] >> k & 1u)) rR[r][k] = bv[k] = 0.0f;
     precondition_quad(rR[r], g, y, fast, rM[r], l, mode, rZ[r]);
-    quad_publish(wz, b, rZ[r], hw[r] >> 14 & 15u, l, tag + 1u);
+    quad_publish(wz, b, rZ[r], quad_faces(hw[r], true), l, tag + 1u);
     R v0[4], v1[4], v2[4];
     uint32_t nw = 0;
 #pragma unroll
@@ -2887,7 +2846,7 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
         if (m >> k & 1u) rP[r][k] += fa * dn[k];
         rR[r][k] = (m >> k & 1u) ? rR[r][k] - fa * rZ[r][k] : 0.0f;
       }
-      if (refresh) quad_publish(wp, b0 + pl, rP[r], hw[r] >> 18 & 15u, l, tag + 1u);
+      if (refresh) quad_publish(wp, b0 + pl, rP[r], quad_faces(hw[r], false), l, tag + 1u);
     }
     new_pass();
 #pragma unroll
@@ -2928,7 +2887,7 @@ __device__ __forceinline__ void solve_quads(const Dev& d, const SolveSpan& sp, u
       new_pass();
 #pragma unroll
       for (uint32_t r = 0; r < RM; ++r)
-        if (first_block(r) < b1) quad_publish(wz, b0 + place(r), rZ[r], fresh(hw[r]) >> 14 & 15u, l, tag);
+        if (first_block(r) < b1) quad_publish(wz, b0 + place(r), rZ[r], quad_faces(fresh(hw[r]), true), l, tag);
     };
     auto halo_z = [&]() -> bool {
       if (WIDE) return true;
@@ -3024,7 +2983,8 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_solve(L l) {
 // On the chip, m of the water cells on block faces (on quads, on the faces between workgroups;
 // inside one m goes through LDS) is published as tagged words and read by the neighbours while the
 // iteration's reduction completes, so the halo exchange costs no wait of its own. A replacement
-// exchanges x, u, p and q in turn, all faces by words. Halo words are numbered
+// exchanges x, u, p and q in turn, all faces by words, with no reduction between: there quads wait
+// for the words of dry cells too (quad_exchange). Halo words are numbered
 // 8 t + k (t the iteration's reduction tag; k = 0 for m, 1..4 for x, u, p, q of a replacement; u0
 // at the start has 8 t + 5 with t the start's reduction) and alternate between two word buffers:
 // m of reduction t and u and q of its replacement in buffer t & 1, x and p in the
@@ -3447,7 +3407,7 @@ __device__ __forceinline__ void solve_pipe_quads(const Dev& d, const SolveSpan& 
   LPart<double>& lp = part_lds<double>();
   const uint32_t mode = d.sc->precond, b0 = sp.b0, b1 = sp.b1, capc = d.capc;
   const uint32_t wv = threadIdx.x >> 6;
-  const QuadLane l = quad_lane();
+  const QuadLane l = quad_lane(lane_id());
   const float* const p0 = start_pressure(d);
   const __amdgpu_buffer_rsrc_t w0 = face_rsrc(d, 0u, sp.n), w1 = face_rsrc(d, 1u, sp.n);
   auto words = [&](uint32_t t) { return (t & 1u) ? w1 : w0; };
@@ -3532,7 +3492,7 @@ __device__ __forceinline__ void solve_pipe_quads(const Dev& d, const SolveSpan& 
     }
     lk = {l.x3 ? nb[0] : (l.x0 ? nb[1] : NONE), l.y3 ? nb[2] : (l.y0 ? nb[3] : NONE), nb[4], nb[5]};
     m = quad_mask(d, cell0, valid, l);
-    w = quad_flags(d, nb, lk, l, b0, b1);
+    w = quad_flags(d.nbm, nb, lk, l, b0);
     float bv[4] = {}, x[4] = {};
     if (valid) {
       quad_load(d.cf + (size_t)NATRAY_F_R * capc, cell0, l.odd, rR);
@@ -3552,7 +3512,7 @@ __device__ __forceinline__ void solve_pipe_quads(const Dev& d, const SolveSpan& 
     put(FP, zero);
     put(FQ, zero);
     precondition4(rR, rU);
-    quad_publish(words(t0), b, rU, w >> 14 & 15u, l, 8u * t0 + 5u);
+    quad_publish(words(t0), b, rU, quad_faces(w, true), l, 8u * t0 + 5u);
     keep(lds.d[pl][l.col], rU);
     part(0, dot(rR, rU));
     part(1, dot(rR, rR));
@@ -3568,16 +3528,16 @@ __device__ __forceinline__ void solve_pipe_quads(const Dev& d, const SolveSpan& 
   auto id = [&](uint32_t link) -> uint32_t { return (link & QUAD_FAR) ? link & ~QUAD_FAR : b0 + link; };
   const QuadLinks far = {lk.x & ~QUAD_FAR, lk.y & ~QUAD_FAR, lk.m & ~QUAD_FAR, lk.p & ~QUAD_FAR};
   bool ok = true;
-  // Waits for the halo of buffer t with tag tg from the blocks k.
-  auto await = [&](uint32_t t, const QuadLinks& k, uint32_t want, uint32_t tg, QuadHalo& h) {
+  // Waits for the words `want` of buffer t with tag tg from the blocks k; h takes those of `use`.
+  auto await = [&](uint32_t t, const QuadLinks& k, uint32_t want, uint32_t use, uint32_t tg, QuadHalo& h) {
     QuadWords q{};
     ok = quad_wait(d, words(t), k, want, l, tg, q, quad_had<1>(want)) && ok;
-    quad_payload(q, want, l.odd, h);
+    quad_payload(q, use, l.odd, h);
   };
   if (go && sets) {
     // w = A u from u0 and its halo.
     QuadHalo h;
-    await(t0, far, quad_want(w, true), 8u * t0 + 5u, h);
+    await(t0, far, quad_want(w, true), quad_want(w, true), 8u * t0 + 5u, h);
     near(h);
     row(rU, h, rW);
   }
@@ -3594,7 +3554,7 @@ __device__ __forceinline__ void solve_pipe_quads(const Dev& d, const SolveSpan& 
     // their m's words.
     if (sets) {
       precondition4(rW, rMv);
-      quad_publish(words(T), b, rMv, w >> 14 & 15u, l, 8u * T);
+      quad_publish(words(T), b, rMv, quad_faces(w, true), l, 8u * T);
       keep(lds.d[pl][l.col], rMv);
     }
     QuadWords q{};
@@ -3643,8 +3603,8 @@ __device__ __forceinline__ void solve_pipe_quads(const Dev& d, const SolveSpan& 
       // iteration is not in, u and q in the other.
       const QuadLinks ids = {id(lk.x), id(lk.y), id(lk.m), id(lk.p)};
       auto exchange = [&](const float* v, uint32_t t, uint32_t tg) {
-        quad_publish(words(t), b, v, w >> 18 & 15u, l, tg);
-        await(t, ids, quad_want(w, false), tg, h);
+        quad_publish(words(t), b, v, quad_faces(w, false), l, tg);
+        await(t, ids, quad_exchange(lk), quad_want(w, false), tg, h);
       };
       float v[4], o[4], g[4], bv[4] = {};
       double ap[4];
