@@ -1702,10 +1702,11 @@ int natray_batch_create(natray_sim* const* sims, uint32_t n, natray_batch** out)
   b->solve_budget = sims[0]->solve_grid;
   b->tgt.plain_solve = true;  // natray_batch_set_solve_launch
   // More workgroups than a CU holds at once: each belongs to one scene, and small ones even out the
-  // scenes' ends. Batch steps, ms, at (8, 8) workgroups a CU and now: 64 scenes of 16k to 524k
-  // particles 3.29, 3.06; 24 of 66k to 262k 1.28, 1.25; 16 of 16k to 131k 0.61, 0.60. At (32, 32)
-  // the 64 scenes gain 1% more and the 24 lose 3%.
-  b->shape = {20u, 16u, 4u, 0u};
+  // scenes' ends. Batch steps, ms, at (8, 8) workgroups a CU, (16, 16) and (20, 16): 64 scenes of 16k
+  // to 524k particles 3.78, 3.58, 3.53; 24 of 66k to 262k 1.25, 1.23, 1.24; 16 of 16k to 131k 0.56,
+  // 0.57, 0.56; 4 of 16k to 66k 0.35 each. One of natray_batch_tune's candidates, so that tuning
+  // can keep it.
+  b->shape = {16u, 16u, 4u, 0u};
   auto bail = [&](int code) {
     batch_free(b);
     delete b;
