@@ -71,8 +71,10 @@ __device__ __forceinline__ Dev load_dev(const Dev* p) {
   DevWords const w = (DevWords)p;
   Dev d;
 #pragma unroll
-  for (uint32_t k = 0; k < sizeof(Dev) / 8; ++k)
-    reinterpret_cast<uint64_t*>(&d)[k] = *(const __attribute__((address_space(4))) uint64_t*)(w + 8 * k);
+  for (uint32_t k = 0; k < sizeof(Dev) / 8; ++k) {
+    const uint64_t word = *(const __attribute__((address_space(4))) uint64_t*)(w + 8 * k);
+    __builtin_memcpy(reinterpret_cast<char*>(&d) + 8 * k, &word, 8);
+  }
   static_assert(sizeof(Dev) % 8 == 0, "Dev is read in 8-byte words");
 #define NATRAY_READ(f) read_field(d.f, w + offsetof(Dev, f));
   NATRAY_DEV_POINTERS(NATRAY_READ)
