@@ -175,6 +175,10 @@ struct Target {
 // Launch wrappers (natray_kernels.hip), on one scene or a batch (Target). Each returns the
 // hipError_t of its launches as int.
 namespace natray {
+// Workgroups of the membrane's kernels, which take 32 lanes a vertex, from those at a thread a vertex.
+// A launch holds fewer than 2^32 threads, which 32 lanes a vertex reach at 2^27 vertices: from 2^25 on
+// the kernels walk them with a stride.
+inline uint32_t mem_groups(uint32_t groups) { return groups < (1u << 17) ? groups * 32u : 1u << 22; }
 int launch_keys(const Target& t, void* stream);
 int launch_begin(const Target& t, void* stream);
 int launch_bin(const Target& t, void* stream, bool rubber = false);

@@ -5782,17 +5782,15 @@ int launch_g2p(const Target& t, void* stream) {
 }
 
 int launch_mem_splat(const Target& t, void* stream) {
-  // 32 lanes a vertex.
   if (t.d)
-    hipLaunchKernelGGL(k_mem_splat<One>, dim3(t.grid[LK_VERTS] * 32u), dim3(256), 0, S(stream), One{*t.d});
+    hipLaunchKernelGGL(k_mem_splat<One>, dim3(mem_groups(t.grid[LK_VERTS])), dim3(256), 0, S(stream), One{*t.d});
   else
     hipLaunchKernelGGL(k_mem_splat<Many>, dim3(t.grid[LK_VERTS]), dim3(256), 0, S(stream), Many{t.scenes, t.map[LK_VERTS]});
   return (int)hipGetLastError();
 }
 int launch_mem_sample(const Target& t, void* stream) {
-  // 32 lanes a vertex.
   if (t.d)
-    hipLaunchKernelGGL(k_mem_sample<One>, dim3(t.grid[LK_VERTS] * 32u), dim3(256), 0, S(stream), One{*t.d});
+    hipLaunchKernelGGL(k_mem_sample<One>, dim3(mem_groups(t.grid[LK_VERTS])), dim3(256), 0, S(stream), One{*t.d});
   else
     hipLaunchKernelGGL(k_mem_sample<Many>, dim3(t.grid[LK_VERTS]), dim3(256), 0, S(stream), Many{t.scenes, t.map[LK_VERTS]});
   return (int)hipGetLastError();
