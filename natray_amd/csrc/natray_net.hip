@@ -198,7 +198,8 @@ __global__ void k_pack(PackJobs jobs) {
   wb[i] = out;
 }
 
-// dZ = dY where the layer's ReLU output was positive (all of dY without ReLU), as BF16.
+// dZ = dY where the layer's ReLU output was positive (all of dY without ReLU), as BF16. For the check
+// of one layer, whose dY is given; in training k_conv's gate does this where dY is made.
 __global__ void k_relu_back(const float* __restrict__ dY, const __bf16* __restrict__ Y, int relu, __bf16* __restrict__ dZ,
                             size_t n) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
@@ -864,7 +865,11 @@ int natray_net_layer_check(uint32_t cin_real, uint32_t cout_real, int relu, cons
   pj.job[1] = PackJob{dWd, (int)cin_real, (int)cout_real, 16, 1, wt};
   hipLaunchKernelGGL(k_pack, dim3(PACK_MAX, 2), dim3(256), 0, 0, pj);
   launch_conv(cin, tiles, 0, xb, wb, bd, relu, nullptr, yb, yf, nullptr, nullptr);
-  hipLaunchKernelGGL(k_take, dim3(grid), dim3(256), 0, 0, yf, (int)cout_real, stage, vox);
+  // The one-channel output as the network's last layer writes it, or the first channels of 16.
+  if (cout_real == 1)
+    launch_conv(cin, tiles, 0, xb, wb, bd, relu, nullptr, nullptr, nullptr, stage, nullptr);
+  else
+    hipLaunchKernelGGL(k_take, dim3(grid), dim3(256), 0, 0, yf, (int)cout_real, stage, vox);
   if (hipMemcpy(Y, stage, vox * cout_real * 4, hipMemcpyDeviceToHost)) return done(nfail(NATRAY_E_HIP, "download Y"));
   // Backward from dY.
   if (hipMemcpy(stage, dY, vox * cout_real * 4, hipMemcpyHostToDevice)) return done(nfail(NATRAY_E_HIP, "upload dY"));
