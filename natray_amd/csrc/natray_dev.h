@@ -44,7 +44,8 @@ struct Dev {
   int32_t* acc;            // 19 x capc fixed-point transfer sums
   float* cf;               // 11 x capc solver fields
   float* bvec;             // capc: CG right-hand side (true-residual refresh)
-  uint32_t* nbm;           // capc: bit k = face neighbour k is water, bit 6 = the cell is water
+  uint32_t* nbm;           // capc: bit k = face neighbour k is water, bit 6 = the cell is water, bits
+                           // 8..10 = its face neighbours that are not solid (0..6); 0 off water
   double* part;            // cap x 4: per-block partial sums of the solver (memory form)
   uint32_t* tile_sum;      // 2 x ntiles: scan tile totals (slots claimed, particles)
   uint32_t* bar;           // control words: [2] the solve's abort flag a stuck wait raises,

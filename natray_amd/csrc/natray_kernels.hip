@@ -1595,9 +1595,9 @@ __device__ __forceinline__ const float* start_pressure(const Dev& d) {
   return d.bar[11] ? d.guess : d.cf + (size_t)NATRAY_F_P * d.capc;
 }
 
-// The rows of every cell, before the solve. On its own the pass has eight waves a SIMD to hide
-// its chain of loads (block links, types, pressures and velocities) behind; inside the solve it
-// had four, in lock step: 190 us of the 15.2M impact's solve, 25 us here.
+// The rows of every cell, before the solve. On its own the pass has five waves a SIMD (85 VGPRs),
+// each on its way, to hide its chain of loads (block links, types, pressures and velocities)
+// behind; inside the solve it had four, in lock step: 190 us of the 15.2M impact's solve, 37 us here.
 template <class L>
 __global__ __launch_bounds__(256) void k_solve_rows(L l) {
   const auto v = view(l);
@@ -3674,8 +3674,8 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_solve_pipe(L l) {
   // A wave of its own for each block while there are enough waves: the iteration is then a chain of
   // one cell's work a lane, of which quads have four (in double, the dots and the scalars, most of
   // all). us an iteration, one block a wave and quads: 1,594 blocks in 256 workgroups 6.9 and 9.4,
-  // 2,946 8.1 and 9.4. Two blocks a wave took 11.5 at 5,657 blocks, where quads take 9.7, and from
-  // memory 12,482 blocks took 54, on quads 12.6.
+  // 2,946 8.1 and 9.4. Two blocks a wave took 11.5 at 5,657 blocks, where quads take 9.95, and from
+  // memory 12,482 blocks took 54, on quads 12.8.
   if ((sp.m + sp.G - 1u) / sp.G * sp.K <= SOLVE_WAVES)
     solve_pipe_blocks(d, sp, tag);
   else
